@@ -32,6 +32,7 @@
 #include "launch.hpp"
 #include "profile.hpp"
 #include "softmax.hpp"
+#include "tile_groups.hpp"
 
 namespace cuflash {
 namespace dev {
@@ -48,12 +49,11 @@ namespace dev {
 //  * K and V blocks of 64 keys go global -> LDS with global_load_lds_dwordx4 (no staging
 //    registers, no VALU or ds_write for the copy) into double buffers, so one barrier per block
 //    suffices and the next blocks load while the current one is consumed;
-//  * LDS layout of a 64 x 128 tile: 16 groups of 4 rows, 1088 bytes each (1 KB + 64 bytes of
-//    padding); inside a group the 16-byte chunk c of row r sits at (4 c + r % 4) * 16. One load
-//    instruction fills one group (lane i: row r0 + i % 4, chunk i / 4, i.e. 1 KB of contiguous
-//    global memory), and both consumers read conflict-free with immediate offsets: the K row
-//    reads of S^T (16 rows, one chunk: 4 groups x 4 rows -> 16 distinct 16-byte bank slots) and
-//    the V transpose reads of P V (4 rows x 4 chunks of one group: 256 contiguous bytes);
+//  * LDS layout of a 64 x 128 tile: 16 groups of 4 rows (TileGroups). One load instruction fills
+//    one group from 1 KB of contiguous global memory, and both consumers read conflict-free
+//    with immediate offsets: the K row reads of S^T (16 rows, one chunk: 4 groups x 4 rows -> 16
+//    distinct 16-byte bank slots) and the V transpose reads of P V (4 rows x 4 chunks of one
+//    group: 256 contiguous bytes);
 //  * the scores of block j+1 are formed by MFMA while the softmax of block j runs on the VALU
 //    (two score register sets), and P V of block j follows;
 //  * the lane-pair row max / sum use v_permlane32_swap instead of an LDS permute.
@@ -69,7 +69,8 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
     constexpr int BM = 32 * NW;  // query rows per workgroup (NW waves of 32 rows)
     constexpr int BN = 64;
     constexpr int kParts = 16 / NW;  // load instructions per wave per 64-row tile
-    constexpr int GRP = 1088;              // bytes per 4-row group
+    using Lay = TileGroups<D>;
+    constexpr int GRP = Lay::kBytes;       // bytes per 4-row group
     constexpr int TILE = (BN / 4) * GRP;   // bytes per 64-row tile
     using frag = typename Elem<T>::frag;
     __shared__ __attribute__((aligned(1024))) unsigned char Kb0[TILE];
@@ -110,10 +111,10 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
     // the operand reads; the loop orders every LDS access itself (s_waitcnt(0) and a barrier
     // before a tile is read and before a buffer is refilled).
     // A tile that lies inside [0, Nk) is addressed as a scalar base plus a fixed per-lane offset.
-    const int ld_row = lane & 3;
+    const int ld_row = Lay::ld_row(lane);
     // At head_dim 96 a row fills chunks 0-11 of its 256-byte slot; lanes 48-63 load chunks 0-3
     // again into the unused slots 12-15.
-    const int ld_col = ((lane >> 2) % (D / 8)) * 8;
+    const int ld_col = Lay::ld_col(lane);
     const unsigned ld_voff = static_cast<unsigned>(((4 * wave + ld_row) * D + ld_col) * 2);
     // Part i (0..kParts-1) of a tile load: this wave's group wave + NW i.
     auto load_part = [&](const uint16_t* src, int key0, unsigned char* dst, int i) {
@@ -131,10 +132,8 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
         for (int i = 0; i < kParts; ++i) load_part(src, key0, dst, i);
     };
     // Per-lane byte offsets of the operand reads (see the layout above).
-    const int k_off = (l32 >> 2) * GRP + g2 * 64 + (l32 & 3) * 16;
-    const int kq = lane & 15;
-    const int v_off = g2 * GRP + (2 * ((lane >> 4) & 1) + ((kq & 3) >> 1)) * 64 + (kq >> 2) * 16 +
-                      (kq & 1) * 8;
+    const int k_off = Lay::row_base(lane, 0);
+    const int v_off = Lay::tr_off(lane);
 
     auto scores = [&](const unsigned char* kt, f32x16 (&s)[2]) {
 #pragma unroll
@@ -142,7 +141,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
             s[t] = f32x16{};
 #pragma unroll
             for (int ks = 0; ks < D / 16; ++ks)
-                s[t] = Elem<T>::mma(as_frag<T>(ld16(kt + k_off + 8 * t * GRP + ks * 128)), qf[ks],
+                s[t] = Elem<T>::mma(as_frag<T>(ld16(kt + k_off + 8 * t * GRP + Lay::k_off(ks))), qf[ks],
                                     s[t]);
         }
     };
@@ -187,10 +186,10 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
     // Operand fragment i of the score MFMAs (K rows of tile half i / 8, k-step i % 8) and of
     // the P V MFMAs (V^T for key group i / 4 and d tile i % 4).
     auto k_frag = [&](const unsigned char* kt, int i) {
-        return as_frag<T>(ld16(kt + k_off + 8 * (i / KS) * GRP + (i % KS) * 128));
+        return as_frag<T>(ld16(kt + k_off + 8 * (i / KS) * GRP + Lay::k_off(i % KS)));
     };
     auto v_frag = [&](const unsigned char* vt, int i) {
-        const unsigned char* a0 = vt + v_off + 4 * (i / NDT) * GRP + (i % NDT) * 256;
+        const unsigned char* a0 = vt + v_off + 4 * (i / NDT) * GRP + Lay::dtile_off(i % NDT);
         return tr_frag_at<T>(a0, a0 + 2 * GRP);
     };
 
@@ -392,8 +391,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
 // ------------------------------------------------------------------------------------------
 // fwd16_d128_kernel's data path and pipeline at head_dim 256: a 4-row group holds the two
 // 128-column halves of its rows one after the other, each in the 1 KB layout of the head_dim-128
-// groups, plus 64 bytes of padding (so row reads and transpose reads stay conflict-free as
-// there). O (8 accumulator tiles) and Q^T (16 fragments) need one workgroup of NW waves per
+// groups, plus padding (so row reads and transpose reads stay conflict-free as there). O (8 accumulator tiles) and Q^T (16 fragments) need one workgroup of NW waves per
 // CU, i.e. one wave per SIMD for NW = 4.
 template <typename T, int NW>
 __global__ void __launch_bounds__(64 * NW, 1)
@@ -406,7 +404,8 @@ __global__ void __launch_bounds__(64 * NW, 1)
     constexpr int BN = 64;
     constexpr int kParts = 32 / NW;  // load instructions per wave per 64-row tile
     constexpr int HALF = 1024;             // bytes of one 128-column half of a 4-row group
-    constexpr int GRP = 2 * HALF + 64;     // bytes per 4-row group
+    using Lay = TileGroups<D>;
+    constexpr int GRP = Lay::kBytes;       // bytes per 4-row group
     constexpr int TILE = (BN / 4) * GRP;   // bytes per 64-row tile
     using frag = typename Elem<T>::frag;
     __shared__ __attribute__((aligned(1024))) unsigned char Kb0[TILE];
@@ -444,8 +443,8 @@ __global__ void __launch_bounds__(64 * NW, 1)
     // Loads of one 64-row tile: 16 groups of 4 rows, two load instructions per group (columns
     // 0-127 and 128-255, 1 KB each, in the layout of fwd16_d128_kernel's groups). Part i of a
     // wave loads half i % 2 of group wave + NW (i / 2). Rows past Nk are clamped to row Nk - 1.
-    const int ld_row = lane & 3;
-    const int ld_col = (lane >> 2) * 8;
+    const int ld_row = Lay::ld_row(lane);
+    const int ld_col = Lay::ld_col(lane);
     const unsigned ld_voff = static_cast<unsigned>(((4 * wave + ld_row) * D + ld_col) * 2);
     auto load_part = [&](const uint16_t* src, int key0, unsigned char* dst, int i) {
         const int grp = wave + NW * (i >> 1);
@@ -464,14 +463,12 @@ __global__ void __launch_bounds__(64 * NW, 1)
         for (int i = 0; i < kParts; ++i) load_part(src, key0, dst, i);
     };
     // Per-lane byte offsets of the operand reads (see the layout above).
-    const int k_off = (l32 >> 2) * GRP + g2 * 64 + (l32 & 3) * 16;
-    const int kq = lane & 15;
-    const int v_off = g2 * GRP + (2 * ((lane >> 4) & 1) + ((kq & 3) >> 1)) * 64 + (kq >> 2) * 16 +
-                      (kq & 1) * 8;
+    const int k_off = Lay::row_base(lane, 0);
+    const int v_off = Lay::tr_off(lane);
 
     // K row reads, k-step ks (16 columns): half ks / 8, chunk 2 (ks % 8) + lane / 32.
     auto k_addr = [&](const unsigned char* kt, int t, int ks) {
-        return kt + k_off + 8 * t * GRP + (ks >> 3) * HALF + (ks & 7) * 128;
+        return kt + k_off + 8 * t * GRP + Lay::k_off(ks);
     };
     auto scores = [&](const unsigned char* kt, f32x16 (&s)[2]) {
 #pragma unroll
@@ -528,7 +525,7 @@ __global__ void __launch_bounds__(64 * NW, 1)
     auto v_frag = [&](const unsigned char* vt, int i) {
         const int dt = i & 7;
         const unsigned char* a0 =
-            vt + v_off + 4 * (i >> 3) * GRP + (dt >> 2) * HALF + (dt & 3) * 256;
+            vt + v_off + 4 * (i >> 3) * GRP + Lay::dtile_off(dt);
         return tr_frag_at<T>(a0, a0 + 2 * GRP);
     };
 
@@ -714,7 +711,8 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
     constexpr int BM = 32 * NW;  // query rows per workgroup (NW waves of 32 rows)
     constexpr int BN = 64;
     constexpr int kParts = 8 / NW;  // load instructions per wave per 64-row tile
-    constexpr int GRP = 1152;              // bytes per 8-row group
+    using Lay = TileGroups<D>;
+    constexpr int GRP = Lay::kBytes;       // bytes per 8-row group
     constexpr int TILE = (BN / 8) * GRP;   // bytes per 64-row tile
     static_assert(kParts >= 1, "at most eight waves");
     using frag = typename Elem<T>::frag;
@@ -751,14 +749,14 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
     const int nkb = (kv_end + BN - 1) / BN;
 
     // Loads of one 64-row tile: wave w fills groups w, w + NW, ... (kParts of them), one
-    // 8-row group (1 KB) per load instruction: lane i writes slot i, i.e. chunk i / 8 of row
-    // (i % 8) ^ (4 ((i >> 4) & 1)) of the group. Rows past Nk are clamped to row Nk - 1 (finite
-    // values; their scores are masked). Issued from inline assembly as in fwd16_d128_kernel.
+    // 8-row group (1 KB, TileGroups) per load instruction. Rows past Nk are clamped to row Nk - 1
+    // (finite values; their scores are masked). Issued from inline assembly as in
+    // fwd16_d128_kernel.
     // A tile that lies inside [0, Nk) is addressed as a scalar base plus a fixed per-lane offset.
-    const int ld_row = (lane & 7) ^ (4 * ((lane >> 4) & 1));
+    const int ld_row = Lay::ld_row(lane);
     // At head_dim 32 a row fills chunks 0-3 of its 128-byte slot; lanes 32-63 load the same
     // chunks again into the unused slots 4-7.
-    const int ld_col = ((lane >> 3) % (D / 8)) * 8;
+    const int ld_col = Lay::ld_col(lane);
     const unsigned ld_voff = static_cast<unsigned>(((8 * wave + ld_row) * D + ld_col) * 2);
     // Part i (0..kParts-1) of a tile load: this wave's group wave + NW i.
     auto load_part = [&](const uint16_t* src, int key0, unsigned char* dst, int i) {
@@ -775,20 +773,15 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
 #pragma unroll
         for (int i = 0; i < kParts; ++i) load_part(src, key0, dst, i);
     };
-    // Per-lane byte offsets of the operand reads. Chunk c of row r of a group sits at
-    // 16 (8 c + (r ^ 4 ((c >> 1) & 1))): 16 rows of one chunk (K row reads) fall on 16 distinct
-    // 16-byte bank slots (the 128 bytes of padding per group shift the next 8 rows by 8 slots),
-    // and the 32 lanes of a V transpose read (4 rows x 8 chunk halves) on 32 distinct 8-byte
-    // slots (the row swizzle moves the chunks 2-3 of a 64-byte span to the other rows).
-    // K row reads: chunk 2 ks + g2, so the swizzle bit is ks & 1.
-    const int k_off_even = (l32 >> 3) * GRP + g2 * 128 + (l32 & 7) * 16;
-    const int k_off_odd = (l32 >> 3) * GRP + g2 * 128 + ((l32 & 7) ^ 4) * 16;
-    const int kq = lane & 15;
-    const int gl = (lane >> 4) & 1;
-    const int v_off = (2 * gl + ((kq & 3) >> 1)) * 128 + (g2 ^ gl) * 64 + (kq >> 2) * 16 +
-                      (kq & 1) * 8;
+    // Per-lane byte offsets of the operand reads (TileGroups): 16 rows of one chunk (K row
+    // reads) fall on 16 distinct 16-byte bank slots and the 32 lanes of a V transpose read
+    // (4 rows x 8 chunk halves) on 32 distinct 8-byte slots. K row reads: chunk 2 ks + g2, so
+    // the swizzle depends on ks & 1.
+    const int k_off_even = Lay::row_base(lane, 0);
+    const int k_off_odd = Lay::row_base(lane, 1);
+    const int v_off = Lay::tr_off(lane);
     auto k_addr = [&](const unsigned char* kt, int t, int ks) {
-        return kt + ((ks & 1) ? k_off_odd : k_off_even) + 4 * t * GRP + ks * 256;
+        return kt + ((ks & 1) ? k_off_odd : k_off_even) + 4 * t * GRP + Lay::k_off(ks);
     };
 
     auto scores = [&](const unsigned char* kt, f32x16 (&s)[2]) {
@@ -844,7 +837,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
         return as_frag<T>(ld16(k_addr(kt, i / KS, i % KS)));
     };
     auto v_frag = [&](const unsigned char* vt, int i) {
-        const unsigned char* a0 = vt + v_off + 2 * (i / NDT) * GRP + (i % NDT) * 512;
+        const unsigned char* a0 = vt + v_off + 2 * (i / NDT) * GRP + Lay::dtile_off(i % NDT);
         return tr_frag_at<T>(a0, a0 + GRP);
     };
 
@@ -1056,7 +1049,8 @@ __global__ void __launch_bounds__(64 * NW, 16 / NW)
     constexpr int BM = 32 * NW;  // query rows per workgroup
     constexpr int BN = 64;
     constexpr int kParts = 8 / NW;         // load instructions per wave per 64-row tile
-    constexpr int GRP = 1152;              // bytes per 8-row group (fwd16_d64_kernel's layout)
+    using Lay = TileGroups<D>;
+    constexpr int GRP = Lay::kBytes;       // bytes per 8-row group
     constexpr int TILE = (BN / 8) * GRP;   // bytes per 64-row tile
     using frag = typename Elem<T>::frag;
     __shared__ __attribute__((aligned(1024))) unsigned char Kb0[TILE];
@@ -1090,8 +1084,8 @@ __global__ void __launch_bounds__(64 * NW, 16 / NW)
     const int nkb = (kv_end + BN - 1) / BN;
 
     // Tile loads, operand offsets and masking exactly as in fwd16_d64_kernel.
-    const int ld_row = (lane & 7) ^ (4 * ((lane >> 4) & 1));
-    const int ld_col = ((lane >> 3) % (D / 8)) * 8;
+    const int ld_row = Lay::ld_row(lane);
+    const int ld_col = Lay::ld_col(lane);
     const unsigned ld_voff = static_cast<unsigned>(((8 * wave + ld_row) * D + ld_col) * 2);
     auto load_tile = [&](const uint16_t* src, int key0, unsigned char* dst) {
 #pragma unroll
@@ -1106,18 +1100,15 @@ __global__ void __launch_bounds__(64 * NW, 16 / NW)
             }
         }
     };
-    const int k_off_even = (l32 >> 3) * GRP + g2 * 128 + (l32 & 7) * 16;
-    const int k_off_odd = (l32 >> 3) * GRP + g2 * 128 + ((l32 & 7) ^ 4) * 16;
-    const int kq = lane & 15;
-    const int gl = (lane >> 4) & 1;
-    const int v_off = (2 * gl + ((kq & 3) >> 1)) * 128 + (g2 ^ gl) * 64 + (kq >> 2) * 16 +
-                      (kq & 1) * 8;
+    const int k_off_even = Lay::row_base(lane, 0);
+    const int k_off_odd = Lay::row_base(lane, 1);
+    const int v_off = Lay::tr_off(lane);
     auto k_frag = [&](const unsigned char* kt, int i) {  // K rows of tile i / KS, k-step i % KS
         const int t = i / KS, ks = i % KS;
-        return as_frag<T>(ld16(kt + ((ks & 1) ? k_off_odd : k_off_even) + 4 * t * GRP + ks * 256));
+        return as_frag<T>(ld16(kt + ((ks & 1) ? k_off_odd : k_off_even) + 4 * t * GRP + Lay::k_off(ks)));
     };
     auto v_frag = [&](const unsigned char* vt, int i) {  // V^T, key group i / NDT, d tile i % NDT
-        const unsigned char* a0 = vt + v_off + 2 * (i / NDT) * GRP + (i % NDT) * 512;
+        const unsigned char* a0 = vt + v_off + 2 * (i / NDT) * GRP + Lay::dtile_off(i % NDT);
         return tr_frag_at<T>(a0, a0 + GRP);
     };
 
