@@ -338,6 +338,17 @@ __device__ __forceinline__ void lds_dma4_async(const void* src, unsigned char* l
                  : "memory");
 }
 
+// Waits until at most N of this wave's global loads are in flight (vmcnt; they land in order). The
+// memory clobber keeps every LDS read of what they brought behind it.
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
+// Waits for this wave's LDS reads, before loads are issued into the bytes that they read.
+__device__ __forceinline__ void wait_lds() {
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+}
+
 // ---------------------------------------------------------------------------------------------
 // Wave reductions
 // ---------------------------------------------------------------------------------------------

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "common.hpp"
+#include "kv_block.hpp"
 #include "launch.hpp"
 #include "profile.hpp"
 #include "softmax.hpp"
@@ -345,80 +346,6 @@ struct DecRowLayout {
     static constexpr int dtile_off(int dt) { return dt * 64; }
 };
 
-// One 32-key block of the matrix-core decode for this wave's query heads (lane l32 = head): the
-// scores S^T = K Q^T, the mask past kend, the lazily rescaled softmax (m in log2 units, l this
-// lane's share of the row sum), and O^T += V^T P^T. kt / vt are the block's K / V tiles; k_base
-// (for even and odd k-steps) and v_off are this lane's operand offsets in layout Lay.
-template <typename T, int D, class Lay>
-__device__ __forceinline__ void decode_mma_block(const unsigned char* kt, const unsigned char* vt,
-                                                 const int (&k_base)[2], int v_off, int key0,
-                                                 int kend, int g2, float cs,
-                                                 const typename Elem<T>::frag (&qf)[D / 16],
-                                                 f32x16 (&o)[D / 32], float& m, float& l) {
-    using frag = typename Elem<T>::frag;
-    constexpr int KS = D / 16;
-    constexpr int NDT = D / 32;
-    constexpr int BN = 32;
-    constexpr int kAhead = 3;
-    f32x16 s = f32x16{};
-    {
-        frag fk[KS];
-#pragma unroll
-        for (int k = 0; k < kAhead && k < KS; ++k)
-            fk[k] = as_frag<T>(ld16(kt + k_base[k & 1] + Lay::k_off(k)));
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            if (ks + kAhead < KS)
-                fk[ks + kAhead] =
-                    as_frag<T>(ld16(kt + k_base[(ks + kAhead) & 1] + Lay::k_off(ks + kAhead)));
-            s = Elem<T>::mma(fk[ks], qf[ks], s);
-        }
-    }
-    if (key0 + BN > kend) {
-        const int lim = kend - key0 - 4 * g2;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = (8 * (r >> 2) + (r & 3) < lim) ? s[r] : -INFINITY;
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) mx = __builtin_elementwise_maximum(mx, s[r]);
-    const float m_new = fmaxf(m, pair_max(mx) * cs);
-    const bool grow = m_new > m + kLazyRescale;
-    const float alpha = grow ? fast_exp2(m_new == -INFINITY ? 0.0f : m - m_new) : 1.0f;
-    m = grow ? m_new : m;
-    l *= alpha;
-    if (__ballot(grow) != 0) {
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) o[dt] *= alpha;
-    }
-    const float m_use = (m == -INFINITY) ? 0.0f : m;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(fmaf(s[r], cs, -m_use));
-    float sum = 0.0f;
-#pragma unroll
-    for (int r = 0; r < 16; r += 2) sum += s[r] + s[r + 1];
-    l += sum;
-    frag p[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-        p[h] = pack_frag<T>(s[8 * h + 0], s[8 * h + 1], s[8 * h + 2], s[8 * h + 3], s[8 * h + 4],
-                            s[8 * h + 5], s[8 * h + 6], s[8 * h + 7]);
-    constexpr int kMma = 2 * NDT;
-    frag fv[kMma];
-    auto v_frag = [&](int i) {
-        const unsigned char* a0 =
-            vt + v_off + (i / NDT) * Lay::kTrRows16 + Lay::dtile_off(i % NDT);
-        return tr_frag_at<T>(a0, a0 + Lay::kTrHigh);
-    };
-#pragma unroll
-    for (int k = 0; k < kAhead && k < kMma; ++k) fv[k] = v_frag(k);
-#pragma unroll
-    for (int i = 0; i < kMma; ++i) {
-        if (i + kAhead < kMma) fv[i + kAhead] = v_frag(i + kAhead);
-        o[i % NDT] = Elem<T>::mma(fv[i], p[i / NDT], o[i % NDT]);
-    }
-}
-
 // ------------------------------------------------------------------------------------------
 // Grouped-query decode on the matrix cores (fp16 / bf16, head_dim 32, 64, 128)
 // ------------------------------------------------------------------------------------------
@@ -556,7 +483,7 @@ __global__ void __launch_bounds__(64)
     const float cs = fmaxf(a.c, kFltMin);  // scale 0: -inf * 0 would make the masked scores NaN
 
     auto block = [&](const unsigned char* kt, const unsigned char* vt, int key0) {
-        decode_mma_block<T, D, G>(kt, vt, k_base, v_off, key0, kend, g2, cs, qf, o, m, l);
+        kv_block32<T, D, G>(kt, vt, k_base, v_off, key0, kend, kend, g2, cs, qf, o, m, l, [] {});
     };
 
     // Block j in Kb[j & 1] / Vb[j & 1]; block j + 1's loads are issued once block j's have
@@ -619,7 +546,7 @@ __global__ void __launch_bounds__(64)
 // fills one key row of all NW heads (1 KB contiguous in HBM and in LDS), wave w loading rows
 // RPW w .. RPW w + RPW - 1 of each tile (RPW = 32 / NW), and the waves share the tiles through
 // one barrier per block. The tiles use the row layout (DecRowLayout), 133 KB for the two buffers
-// of K and V, one workgroup per CU; each wave runs decode_mma_block on its own head's 2D-byte
+// of K and V, one workgroup per CU; each wave runs kv_block32 on its own head's 2D-byte
 // column. A load is one key row with one scalar row index, clamped to the sequence's last key
 // past its end (masked), so any page size works.
 template <typename T, int D>
@@ -732,8 +659,8 @@ __global__ void __launch_bounds__(64 * (512 / D))
             load_tile(Vq, kbeg + (j + 1) * BN, Vb1, Lay::kRowV, pages);
             pages = fetch_pages(kbeg + (j + 2) * BN);
         }
-        decode_mma_block<T, D, Lay>(Kb0, Vb0, k_base, v_off, kbeg + j * BN, kend, g2, cs, qf, o, m,
-                                    l);
+        kv_block32<T, D, Lay>(Kb0, Vb0, k_base, v_off, kbeg + j * BN, kend, kend, g2, cs, qf, o, m,
+                              l, [] {});
         if (j + 1 >= nblk) break;
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
@@ -742,8 +669,8 @@ __global__ void __launch_bounds__(64 * (512 / D))
             load_tile(Vq, kbeg + (j + 2) * BN, Vb0, Lay::kRowV, pages);
             pages = fetch_pages(kbeg + (j + 3) * BN);
         }
-        decode_mma_block<T, D, Lay>(Kb1, Vb1, k_base, v_off, kbeg + (j + 1) * BN, kend, g2, cs, qf,
-                                    o, m, l);
+        kv_block32<T, D, Lay>(Kb1, Vb1, k_base, v_off, kbeg + (j + 1) * BN, kend, kend, g2, cs, qf,
+                              o, m, l, [] {});
     }
 
     // Partials of this wave's query heads: lane l32 < G holds head h0 + l32, dims 32 dt + 8 q +

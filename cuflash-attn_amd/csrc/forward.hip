@@ -28,7 +28,11 @@
 // j <= i + coff, coff = Nk - Nq >= 0 (the queries are the last Nq positions of the key
 // sequence; Nq == Nk gives the usual j <= i).
 
+#include <algorithm>
+#include <cmath>
+
 #include "common.hpp"
+#include "kv_block.hpp"
 #include "launch.hpp"
 #include "profile.hpp"
 #include "softmax.hpp"
@@ -1235,6 +1239,348 @@ __global__ void __launch_bounds__(64 * NW, 16 / NW)
 }
 
 // ------------------------------------------------------------------------------------------
+// Split keys
+// ------------------------------------------------------------------------------------------
+// A launch with few query rows leaves most CUs without a workgroup, and its time is the longest
+// workgroup's walk over the keys. With kSplit the keys are cut into `nsplit` chunks of `chunk`
+// keys (whole blocks), one workgroup per (row block, chunk), and each stores its rows'
+// unnormalized fp32 (O, m, l) at slot split * rows + row; fwd_combine_kernel merges them by the
+// split-KV decode's rule. The query heads of one key/value head are packed into the row blocks
+// (row r of a key/value head is token r / group of its query head r % group), so a few tokens of
+// grouped heads still fill the 32-row tiles and the K/V chunk is read once for all of them. The
+// sums of a row depend only on the chunk, not on the packing or the block it falls into.
+struct FwdSplit {
+    float* acc;   // [nsplit, rows, D]
+    float2* ml;   // [nsplit, rows]: m in log2 units, l
+    int chunk;    // keys per split, a multiple of the 32-key blocks
+    int nsplit;
+};
+
+// The workgroup's place in a split launch: key/value head, row block, split.
+__device__ __forceinline__ void split_item(int nqb, int nsplit, int& kvh, int& qb, int& split) {
+    int r;
+    item_order(blockIdx.x, gridDim.x / (nqb * nsplit), nqb * nsplit, true, kvh, r);
+    split = r / nqb;  // the row blocks of one chunk run together: they share its K/V rows
+    qb = r % nqb;
+}
+
+// Merges the splits of each query row: O = sum O_s 2^(m_s - M) / l with M = max m_s and
+// l = sum l_s 2^(m_s - M), L = (M + log2 l) ln 2. D / 4 lanes hold a row, four columns each;
+// `ways` groups of D / 4 lanes (a power of two) take every ways-th split of a row, kBatch of them
+// in flight, and are merged through LDS in order, so that a few rows with many splits are not one
+// serial walk. A causal row has only the splits that begin before its last key.
+template <typename T, int D>
+__global__ void __launch_bounds__(256)
+    fwd_combine_kernel(FwdSplit sp, uint16_t* __restrict__ O, float* __restrict__ L,
+                       unsigned rows, int Nq, int Nk, int coff, int causal, int ways) {
+    constexpr int LPR = D / 4;         // lanes per row
+    constexpr int SLOTS = 256 / LPR;   // row slots per workgroup (the last lanes idle at D = 96)
+    constexpr int kBatch = 8;
+    __shared__ float4 s_acc[SLOTS][LPR];
+    __shared__ float2 s_ml[SLOTS];
+    const int slot = threadIdx.x / LPR;
+    const int part = threadIdx.x % LPR;
+    const int way = slot % ways;
+    const unsigned row = blockIdx.x * (SLOTS / ways) + slot / ways;
+    const bool on = slot / ways < SLOTS / ways && row < rows;
+    float M = -INFINITY, l = 0.0f;
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    // A part whose scores were all -inf has m = -inf: weight 0, also where M = -inf.
+    auto weight = [](float m, float to) { return m == -INFINITY ? 0.0f : fast_exp2(m - to); };
+    if (on) {
+        const int keys = causal ? min(Nk, static_cast<int>(row % Nq) + 1 + coff) : Nk;
+        const int ns = (keys + sp.chunk - 1) / sp.chunk;
+        const float2* ml = sp.ml + row;
+        const float4* a = reinterpret_cast<const float4*>(sp.acc) +
+                          static_cast<size_t>(row) * LPR + part;
+        for (int s0 = way; s0 < ns; s0 += kBatch * ways) {
+            float2 v[kBatch];
+            float4 x[kBatch];
+            float M2 = M;
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+                const int s = s0 + i * ways;
+                v[i] = make_float2(-INFINITY, 0.0f);
+                x[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (s < ns) {
+                    v[i] = ml[static_cast<size_t>(s) * rows];
+                    x[i] = a[static_cast<size_t>(s) * rows * LPR];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) M2 = fmaxf(M2, v[i].x);
+            const float f0 = weight(M, M2);
+            l *= f0;
+            acc.x *= f0;
+            acc.y *= f0;
+            acc.z *= f0;
+            acc.w *= f0;
+            M = M2;
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+                const float f = weight(v[i].x, M);
+                l = fmaf(v[i].y, f, l);
+                acc.x = fmaf(x[i].x, f, acc.x);
+                acc.y = fmaf(x[i].y, f, acc.y);
+                acc.z = fmaf(x[i].z, f, acc.z);
+                acc.w = fmaf(x[i].w, f, acc.w);
+            }
+        }
+    }
+    if (ways > 1) {
+        if (on) {
+            s_acc[slot][part] = acc;
+            if (part == 0) s_ml[slot] = make_float2(M, l);
+        }
+        __syncthreads();
+        if (on && way == 0) {
+            for (int w = 1; w < ways; ++w) M = fmaxf(M, s_ml[slot + w].x);
+            acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            l = 0.0f;
+            for (int w = 0; w < ways; ++w) {
+                const float2 v = s_ml[slot + w];
+                const float4 x = s_acc[slot + w][part];
+                const float f = weight(v.x, M);
+                l = fmaf(v.y, f, l);
+                acc.x = fmaf(x.x, f, acc.x);
+                acc.y = fmaf(x.y, f, acc.y);
+                acc.z = fmaf(x.z, f, acc.z);
+                acc.w = fmaf(x.w, f, acc.w);
+            }
+        }
+    }
+    if (on && way == 0) {
+        const float inv = 1.0f / l;
+        u32x2 w;
+        w[0] = Elem<T>::pack2(acc.x * inv, acc.y * inv);
+        w[1] = Elem<T>::pack2(acc.z * inv, acc.w * inv);
+        st8(O + static_cast<size_t>(row) * D + part * 4, w);
+        if (part == 0) L[row] = (M + fast_log2(l)) * kLn2;
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// fp16 / bf16 kernel for few query rows: one 32-row tile per workgroup, its keys over the waves
+// ------------------------------------------------------------------------------------------
+// The kernels above give a wave 32 rows and all their keys, so a launch of a few hundred rows
+// runs a few dozen waves, each a serial chain of blocks. Here the NW waves of a workgroup share
+// one 32-row tile: wave w takes the 32-key blocks w, w + NW, ... through LDS tiles of its own (no
+// barrier in the loop), and the waves' (O, m, l) are merged through LDS at the end. The query
+// heads of a key/value head are packed into the tiles (FwdSplit), and with kSplit the keys are
+// also cut into chunks over workgroups.
+// What bounds it: every wave loads its own tiles, 128 KB for a round of eight blocks at head_dim
+// 128, 1.0 us at the CU's 64 bytes per clock, beside 0.5 us of MFMAs; measured 1.36 us a round.
+// Eight waves with one buffer each for K and V (two waves per SIMD, one computing while the
+// other loads) take 11.7 us where four waves with double buffers in the same LDS take 14.6 (head_dim
+// 128, 4 heads, N = 1024), 20.6 against 35 at head_dim 256 with four waves against two.
+template <int D>
+constexpr int fwd_rows_waves() {
+    return D == 256 ? 4 : 8;  // LDS: 135 KB at head_dim 256, 139 KB at 128 and 96, 74 KB below
+}
+template <typename T, int D, bool kSplit>
+__global__ void __launch_bounds__(64 * fwd_rows_waves<D>(), D <= 64 ? 2 : 1)
+    fwd16_rows_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
+                      const uint16_t* __restrict__ V, uint16_t* __restrict__ O,
+                      float* __restrict__ L, int Nq, int Nk, int coff, int group, int nqb,
+                      float c, int causal, FwdSplit sp) {
+    using Lay = TileGroups<D>;
+    constexpr int NW = fwd_rows_waves<D>();
+    constexpr int KS = D / 16;
+    constexpr int NDT = D / 32;
+    constexpr int BN = 32;            // keys per block
+    constexpr int GR = Lay::kRows;
+    constexpr int NG = BN / GR;       // row groups per tile
+    constexpr int TILE = NG * Lay::kBytes;
+    constexpr int P = D + 4;          // pitch of the merge rows (floats)
+    using frag = typename Elem<T>::frag;
+    constexpr int kTiles = NW * 2 * TILE;
+    static_assert(NW * 32 * P * 4 <= kTiles, "the merge rows fit the tiles");
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[kTiles];
+    __shared__ float s_m[NW][32];
+    __shared__ float s_l[NW][32];
+
+    int bh, rank, split = 0;  // bh: key/value head
+    if constexpr (kSplit)
+        split_item(nqb, sp.nsplit, bh, rank, split);
+    else
+        item_order(blockIdx.x, gridDim.x / nqb, nqb, causal == 0, bh, rank);
+    const int qb = causal ? nqb - 1 - rank : rank;  // causal: longest tiles first
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31;
+    const int g2 = lane >> 5;
+
+    const int nrows = Nq * group;
+    const int r0 = qb * 32;
+    const int row = r0 + l32;
+    const int q = row / group;  // token
+    const uint16_t* Kh = K + static_cast<size_t>(bh) * Nk * D;
+    const uint16_t* Vh = V + static_cast<size_t>(bh) * Nk * D;
+    if constexpr (kSplit) {
+        // Keys are counted from the split's first one below.
+        const int kbeg = split * sp.chunk;
+        Kh += static_cast<size_t>(kbeg) * D;
+        Vh += static_cast<size_t>(kbeg) * D;
+        Nk -= kbeg;
+        coff -= kbeg;
+    }
+    int kv_end = causal ? min(Nk, (r0 + 31) / group + 1 + coff) : Nk;
+    if constexpr (kSplit) {
+        if (kv_end <= 0) return;  // every row of the tile ends before this split
+        kv_end = min(kv_end, sp.chunk);
+    }
+    const int nblk = (kv_end + BN - 1) / BN;
+
+    unsigned char* kt = smem + wave * 2 * TILE;
+    unsigned char* vt = kt + TILE;
+    // One load instruction per kilobyte of a row group (two at head_dim 256); rows past Nk are
+    // clamped to the last one (masked).
+    const int ld_row = Lay::ld_row(lane);
+    const int ld_col = Lay::ld_col(lane);
+    const unsigned ld_voff = static_cast<unsigned>((ld_row * D + ld_col) * 2);
+    auto load_tile = [&](const uint16_t* src, int key0, unsigned char* dst) {
+        if (key0 + BN <= Nk) {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+#pragma unroll
+                for (int h = 0; h < Lay::kHalves; ++h)
+                    lds_dma16_async_s(src + static_cast<size_t>(key0 + GR * g) * D + 128 * h,
+                                      ld_voff, dst + g * Lay::kBytes + h * 1024);
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                const int r = min(key0 + GR * g + ld_row, Nk - 1);
+#pragma unroll
+                for (int h = 0; h < Lay::kHalves; ++h)
+                    lds_dma16_async(src + static_cast<size_t>(r) * D + 128 * h + ld_col,
+                                    dst + g * Lay::kBytes + h * 1024);
+            }
+        }
+    };
+    frag qf[KS];
+    {
+        const size_t q_row = (static_cast<size_t>(bh) * group + row % group) * Nq + q;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (row < nrows) v = ld16(Q + q_row * D + 16 * ks + 8 * g2);
+            qf[ks] = as_frag<T>(v);
+        }
+    }
+    // After the Q loads, so that waiting for those leaves the tile loads in flight.
+    asm volatile("" ::: "memory");
+    if (wave < nblk) {
+        load_tile(Kh, wave * BN, kt);
+        load_tile(Vh, wave * BN, vt);
+    }
+
+    const int k_base[2] = {Lay::row_base(lane, 0), Lay::row_base(lane, 1)};
+    const int v_off = Lay::tr_off(lane);
+    f32x16 o[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16{};
+    float m = -INFINITY;
+    float l = 0.0f;
+    const float cs = fmaxf(c, kFltMin);
+    // This lane's key limit, and the first key that some row of the tile does not see.
+    const int kend = causal ? min(Nk, q + 1 + coff) : Nk;
+    const int mask_from = causal ? min(Nk, r0 / group + 1 + coff) : Nk;
+    // K and V are waited for separately (vmcnt counts a wave's loads in order, kLoads per tile):
+    // the scores start when K has landed, with V still in flight; the next K is issued once the
+    // scores have read this one, the next V once P V has.
+    constexpr int kLoads = NG * Lay::kHalves;
+    for (int b = wave; b < nblk; b += NW) {
+        const bool next = b + NW < nblk;
+        wait_loads<kLoads>();
+        kv_block32<T, D, Lay>(kt, vt, k_base, v_off, b * BN, mask_from, kend, g2, cs, qf, o, m, l,
+                              [&] {
+                                  if (next) {
+                                      wait_lds();
+                                      load_tile(Kh, (b + NW) * BN, kt);
+                                      wait_loads<kLoads>();
+                                  } else {
+                                      wait_loads<0>();
+                                  }
+                              });
+        if (next) {
+            wait_lds();
+            load_tile(Vh, (b + NW) * BN, vt);
+        }
+    }
+
+    // Merge: every wave scales its rows to the common max and leaves them in LDS, then the
+    // workgroup sums them wave after wave and writes whole 16-byte pieces.
+    l = pair_sum(l);
+    if (g2 == 0) {
+        s_m[wave][l32] = m;
+        s_l[wave][l32] = l;
+    }
+    __syncthreads();  // also ends every wave's use of its tiles
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, s_m[w][l32]);
+    const float f = m == -INFINITY ? 0.0f : fast_exp2(m - M);
+    float* mrg = reinterpret_cast<float*>(smem);
+    {
+        float* dst = mrg + (wave * 32 + l32) * P + 4 * g2;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                f32x4 w;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) w[u] = o[dt][4 * a + u] * f;
+                st16(dst + 32 * dt + 8 * a, __builtin_bit_cast(u32x4, w));
+            }
+        }
+    }
+    __syncthreads();
+    constexpr int CPR = D / 8;  // 8-column pieces per row
+#pragma unroll
+    for (int i0 = 0; i0 < 32 * CPR; i0 += 64 * NW) {
+        const int i = i0 + threadIdx.x;
+        const int r = i / CPR;
+        const int cc = (i % CPR) * 8;
+        const int rr = r0 + r;
+        if (r >= 32 || rr >= nrows) break;
+        float ms[NW], MM = -INFINITY, lt = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            ms[w] = s_m[w][r];
+            MM = fmaxf(MM, ms[w]);
+        }
+        f32x4 a0 = {0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            lt = fmaf(s_l[w][r], ms[w] == -INFINITY ? 0.0f : fast_exp2(ms[w] - MM), lt);
+            const float* src = mrg + (w * 32 + r) * P + cc;
+            a0 += __builtin_bit_cast(f32x4, ld16(src));
+            a1 += __builtin_bit_cast(f32x4, ld16(src + 4));
+        }
+        const int tok = rr / group;
+        const size_t orow = (static_cast<size_t>(bh) * group + rr % group) * Nq + tok;
+        if constexpr (kSplit) {
+            if (causal && tok + 1 + coff <= 0) continue;  // the combine does not read this row
+            const size_t heads = gridDim.x / (nqb * sp.nsplit);
+            const size_t slot = split * heads * nrows + orow;
+            st16(sp.acc + slot * D + cc, __builtin_bit_cast(u32x4, a0));
+            st16(sp.acc + slot * D + cc + 4, __builtin_bit_cast(u32x4, a1));
+            if (cc == 0) sp.ml[slot] = make_float2(MM, lt);
+        } else {
+            const float inv = 1.0f / lt;
+            u32x4 w;
+            w[0] = Elem<T>::pack2(a0[0] * inv, a0[1] * inv);
+            w[1] = Elem<T>::pack2(a0[2] * inv, a0[3] * inv);
+            w[2] = Elem<T>::pack2(a1[0] * inv, a1[1] * inv);
+            w[3] = Elem<T>::pack2(a1[2] * inv, a1[3] * inv);
+            st16_nt(O + orow * D + cc, w);
+            if (cc == 0) L[orow] = (MM + fast_log2(lt)) * kLn2;
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
 // fp32 kernel
 // ------------------------------------------------------------------------------------------
 // Two workgroups per CU, except at head_dim 256 (O, Q^T and the scores need more than the
@@ -1608,6 +1954,102 @@ struct FwdShape {
     int group;  // query heads per key/value head
 };
 
+// Chunks over which fwd16_rows_kernel cuts the keys of this launch, or 0 where the general kernels
+// are faster. The times are modelled in microseconds from measurements (causal and not, 4 to 32
+// heads, 64 to 16384 keys; event times of one box):
+//  * fwd16_rows_kernel: a workgroup walks its longest tile in rounds of one block per wave, tb
+//    each, and t0 for its start, merge and store; as many workgroups as the slots run at once.
+//    Several chunks add the merge kernel and the partials, written and read at about 4 TB/s.
+//  * the general kernels, when their 128-row workgroups all run at once: g per 64-key block of the
+//    longest row, up to 1.3 g with two workgroups per CU at head_dim 64 and 32.
+// bf16/fp16, causal, B = 1, before -> after: 8 heads, head_dim 128, N = 129 8.4 -> 6.3, 1024 23.9 ->
+// 11.9, 4096 82 -> 64; head_dim 64, N = 256 6.3 -> 5.0, 1024 16.9 -> 8.5, 4096 55.6 -> 34.5;
+// head_dim 256, N = 1024 40.1 -> 22.0; 32 heads over 8 against 8253 keys, head_dim 128: 61 queries
+// 160 -> 22 (4 chunks), one query 156 -> 11.6 (16 chunks). The other side of the line: 32 heads,
+// head_dim 128, N = 1024 25.7 general, 32.7 here; head_dim 64, N = 1536 25.8 and 26.9.
+template <int D>
+int forward_rows_chunks(const FwdShape& sh, bool causal) {
+    constexpr double tb = D == 32 ? 1.2 : D == 64 ? 1.6 : D == 96 ? 1.1 : D == 128 ? 1.36 : 1.95;
+    constexpr double t0 = D <= 64 ? 3.0 : 4.2;
+    constexpr double g = D == 32 ? 0.75 : D == 64 ? 0.85 : D == 96 ? 1.15 : D == 128 ? 1.27 : 2.25;
+    constexpr int kWaves = dev::fwd_rows_waves<D>();
+    const double cus = compute_units();
+    const double slots = D <= 64 ? 2 * cus : cus;
+    const double rows = static_cast<double>(sh.BH) * sh.Nq;
+    const double units = static_cast<double>(sh.BH) * ((sh.Nq + 127) / 128);
+    if (units > 2 * cus) return 0;
+    const double tiles = static_cast<double>(sh.BH / sh.group) *
+                         ((static_cast<long long>(sh.group) * sh.Nq + 31) / 32);
+    const double longest = (sh.Nk + 31) / 32 / static_cast<double>(kWaves);
+    const double average = causal ? longest * (2.0 * sh.Nk - sh.Nq) / (2.0 * sh.Nk) : longest;
+    double best = 0.0;
+    int chunks = 0;
+    for (int n = 1; n == 1 || (n <= 32 && 2 * n <= longest); ++n) {
+        const double rounds = std::ceil(tiles * n / slots);
+        const double walk = rounds > 1 ? average / n : std::ceil(longest / n);
+        double t = rounds * (walk * tb + t0) - 2.0;
+        if (n > 1) t += 4.0 + 2.0 * n * rows * D * sizeof(float) / 4e6;
+        if (chunks == 0 || t < best) {
+            best = t;
+            chunks = n;
+        }
+    }
+    const double crowd = D <= 64 ? 1.0 + 0.3 * std::min(1.0, std::max(0.0, units / cus - 1.0)) : 1.0;
+    return 1.1 * best < g * crowd * ((sh.Nk + 63) / 64) ? chunks : 0;
+}
+
+// One workgroup per (32 rows of a key/value head's query heads, chunk of keys), and a merge kernel
+// when there are several chunks. The partials need a workspace: a launch that cannot have one,
+// and a captured one (a graph would hold an allocation of tens of MiB where the forward had none),
+// walks all keys in one chunk.
+template <typename T, int D>
+FlashAttentionError run_forward16_rows(const T* Q, const T* K, const T* V, T* O, float* L,
+                                       const FwdShape& sh, int chunks, float scale, bool causal,
+                                       hipStream_t stream) {
+    const long long rows = static_cast<long long>(sh.BH) * sh.Nq;
+    const long long nqb = (static_cast<long long>(sh.group) * sh.Nq + 31) / 32;
+    dev::FwdSplit sp{nullptr, nullptr, sh.Nk, 1};
+    StreamWorkspace ws(stream, true);
+    if (chunks > 1) {
+        const int chunk = ((sh.Nk + chunks - 1) / chunks + 31) / 32 * 32;
+        const int nsplit = (sh.Nk + chunk - 1) / chunk;
+        const size_t slots = static_cast<size_t>(rows) * nsplit;
+        const size_t bytes = slots * (D * sizeof(float) + sizeof(float2));
+        if (nsplit > 1 && bytes <= kStreamCacheBytes && !stream_capturing(stream) &&
+            ws.alloc(bytes) == FlashAttentionError::SUCCESS) {
+            sp.acc = static_cast<float*>(ws.get());
+            sp.ml = reinterpret_cast<float2*>(sp.acc + slots * D);
+            sp.chunk = chunk;
+            sp.nsplit = nsplit;
+        }
+    }
+    const long long blocks = nqb * (sh.BH / sh.group) * sp.nsplit;
+    const int coff = sh.Nk - sh.Nq;
+    ProfileEvents tok = profile_kernel<T, D>("forward");
+    launch_kernel(tok,
+                  sp.nsplit > 1 ? dev::fwd16_rows_kernel<T, D, true>
+                                : dev::fwd16_rows_kernel<T, D, false>,
+                  dim3(static_cast<unsigned>(blocks)), dim3(64 * dev::fwd_rows_waves<D>()), 0,
+                  stream, reinterpret_cast<const uint16_t*>(Q),
+                  reinterpret_cast<const uint16_t*>(K), reinterpret_cast<const uint16_t*>(V),
+                  reinterpret_cast<uint16_t*>(O), L, sh.Nq, sh.Nk, coff, sh.group,
+                  static_cast<int>(nqb), scale * dev::kLog2e, causal ? 1 : 0, sp);
+    const FlashAttentionError err = from_hip(hipGetLastError());
+    if (err != FlashAttentionError::SUCCESS || sp.nsplit == 1) return err;
+    // Row slots per merge workgroup; several share a row while the rows are few.
+    constexpr int kSlots = 256 / (D / 4);
+    int ways = 1;
+    while (2 * ways <= kSlots && 8 * ways < sp.nsplit && rows * ways < 8LL * compute_units())
+        ways *= 2;
+    const long long per_wg = kSlots / ways;
+    tok = profile_kernel<T, D>("forward_combine");
+    launch_kernel(tok, (dev::fwd_combine_kernel<T, D>),
+                  dim3(static_cast<unsigned>((rows + per_wg - 1) / per_wg)), dim3(256), 0, stream,
+                  sp, reinterpret_cast<uint16_t*>(O), L, static_cast<unsigned>(rows), sh.Nq,
+                  sh.Nk, coff, causal ? 1 : 0, ways);
+    return from_hip(hipGetLastError());
+}
+
 template <typename T, int D>
 FlashAttentionError run_forward16(const T* Q, const T* K, const T* V, T* O, float* L,
                                   const FwdShape& sh, float scale, bool causal,
@@ -1624,6 +2066,9 @@ FlashAttentionError run_forward16(const T* Q, const T* K, const T* V, T* O, floa
     long long blocks = static_cast<long long>(nqb) * sh.BH;
     if (blocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;
     const int coff = sh.Nk - sh.Nq;
+    const int chunks = forward_rows_chunks<D>(sh, causal);
+    if (chunks > 0)
+        return run_forward16_rows<T, D>(Q, K, V, O, L, sh, chunks, scale, causal, stream);
     const ProfileEvents tok = profile_kernel<T, D>("forward");
     if constexpr (D == 64) {
         // Launches with at least as many 256-row blocks as CUs: eight-wave workgroups of the
