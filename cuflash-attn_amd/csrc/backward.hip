@@ -578,12 +578,21 @@ __global__ void __launch_bounds__(256)
 // and stores its fp32 share of dK (scaled) and dV at part[bh] and part[BH + bh] ([BH, Nk, D]
 // each), which dkdv_reduce_kernel sums over each group.
 // Whether the items address the tile loads of whole tiles as a scalar base plus a fixed
-// per-lane offset (no per-load VALU address arithmetic). Measured at config 3's shape: head_dim
-// 128 causal 1.5% faster, 96 5%; head_dim 256 and the head_dim-64 layout (also used at 32)
-// 0.5-2% slower, so those keep the per-lane addresses.
+// per-lane offset (no per-load VALU address arithmetic): not at head_dim 256, where it measured 1%
+// slower (993 against 998 us, causal B=2 H=16 N=4096; head_dim 64 270 -> 266, 32 210 -> 207).
 template <int D>
 constexpr bool bwd_scalar_tile_base() {
-    return D == 128 || D == 96;
+    return D != 256;
+}
+// Where the items issue the next block's tile loads. A load waits at issue while the CU's vector
+// memory path drains the other waves' loads: after the S / dP MFMAs that wait overlaps the MFMAs
+// in flight, except at head_dim 256, whose 32 MFMAs leave the loads too little of the block
+// behind them. Measured early -> late, dq items: head_dim 64 non-causal B=4 H=16 N=2048 298 -> 279
+// us, head_dim 128 non-causal B=2 H=16 N=4096 862 -> 850, causal 458 -> 456; dkdv items late -> early:
+// head_dim 256 N=2049 163 -> 159, head_dim 128 non-causal 862 -> 901.
+template <int D>
+constexpr bool bwd_early_loads() {
+    return D == 256;
 }
 // Whether the items store their output rows through LDS (store_rows_staged: whole contiguous
 // rows per store instruction). Not at head_dim 128, where the staging code makes the kernel
@@ -717,6 +726,7 @@ __device__ __forceinline__ void dkdv_lds_tiles(const uint16_t* __restrict__ Q,
         const unsigned char* ot = qt + QT;
         const float2* ldv = reinterpret_cast<const float2*>(qt + 2 * QT);
         const float* ldf = reinterpret_cast<const float*>(ldv);  // neg_d_rows: 32 L, then 32 -D
+        if (bwd_early_loads<D>() && it + 1 < n_it) load_block(it + 1, b ^ 1);
 
         // S = Q K^T and dP = dO V^T: rows = queries, lane = key. Operand i (i even: Q, odd: dO;
         // k-step i / 2) is read kAhead MFMAs before its product; the scheduling fences keep the
@@ -762,11 +772,7 @@ __device__ __forceinline__ void dkdv_lds_tiles(const uint16_t* __restrict__ Q,
             for (int r = 0; r < 16; ++r)
                 s[r] = (8 * (r >> 2) + (r & 3) < lim) ? -INFINITY : s[r];
         }
-        // Next block's tile loads. Issued here, after the S / dP MFMAs: a load waits at issue
-        // while the CU's vector memory path drains the other waves' loads, and here that wait
-        // overlaps the MFMAs in flight; before them it delays the MFMAs, after the P / dS
-        // arithmetic it delays the dV / dK MFMAs (both measured slower).
-        if (it + 1 < n_it) load_block(it + 1, b ^ 1);
+        if (!bwd_early_loads<D>() && it + 1 < n_it) load_block(it + 1, b ^ 1);
         frag bp[2], bs[2];
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
@@ -995,7 +1001,7 @@ __device__ __forceinline__ void dq_lds_tiles(const uint16_t* __restrict__ Q,
         const int key0 = kb * BN;
         __builtin_amdgcn_s_waitcnt(0);  // block kb is in LDS
         __syncthreads();                // ... for every wave; block kb - 1 is no longer read
-        if (kb + 1 < nkb) load_block(kb + 1, b ^ 1);
+        if (bwd_early_loads<D>() && kb + 1 < nkb) load_block(kb + 1, b ^ 1);
         const unsigned char* kt = smem + b * SET;
         const unsigned char* vt = kt + KT;
 
@@ -1030,6 +1036,7 @@ __device__ __forceinline__ void dq_lds_tiles(const uint16_t* __restrict__ Q,
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if (!bwd_early_loads<D>() && kb + 1 < nkb) load_block(kb + 1, b ^ 1);
         if (key0 + BN > Nk || (causal && key0 + BN - 1 > q0 + coff)) {
             const int lim = min(Nk, causal ? q + 1 + coff : Nk) - key0 - 4 * g2;
 #pragma unroll
