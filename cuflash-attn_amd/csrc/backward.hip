@@ -8,7 +8,8 @@
 //                     (reference flash_attention_backward_dq_kernel, :37-143);
 //   3. dkdv_kernel:   KV-stationary. Per query block: P as above, dV += P^T dO,
 //                     dS = P (dP - D), dK += scale * dS^T Q
-//                     (reference flash_attention_backward_dkdv_kernel, :146-288).
+//                     (reference flash_attention_backward_dkdv_kernel, :146-288);
+//      bwd32_kernel:  2 and 3 in one launch of smaller items (fp32, where it is faster).
 // Masked (causal / out-of-range) entries contribute 0, as in the reference (:108-110, :214-220).
 //
 // Every product runs on MFMA (32x32x16 for fp16/bf16, 32x32x2 for fp32) through the Mma<T>
@@ -19,7 +20,7 @@
 // so each lane owns one query row of dQ, or one key row of dK/dV, for the whole kernel. For
 // fp16/bf16 P and dS are rounded to the input type before their products (fp32 accumulate).
 // For fp16/bf16 (every head_dim) the same steps run as delta_ld_kernel, then
-// dq_lds_tiles and dkdv_lds_tiles items in one launch (bwd_fused_kernel, section 4). Every path is
+// dq_lds_tiles and dkdv_lds_tiles items in one launch (bwd_fused_kernel, section 5). Every path is
 // deterministic: no atomics, and each output element is written by exactly one lane.
 //
 // Shapes: Q, O, dO, dQ are [BH, Nq, D], K, V, dK, dV are [BH / group, Nk, D] (query head bh
@@ -33,6 +34,7 @@
 #include "tile_groups.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace cuflash {
@@ -505,7 +507,315 @@ __global__ void __launch_bounds__(256, 1)
 }
 
 // ------------------------------------------------------------------------------------------
-// 4. Backward for head_dim 64, 128 and 256 (fp16 / bf16)
+// 4. fp32 backward up to head_dim 128: one 32-row tile per workgroup, its blocks over the waves
+// ------------------------------------------------------------------------------------------
+// fp32 products run at 64 clocks per v_mfma_f32_32x32x2f32, so an item is bound by its own chain
+// of MFMAs (head_dim 64: 128 per 32 x 32 block for dK and dV, 96 for dQ) and a launch by its
+// longest item. Here the four waves of a workgroup share one tile (32 keys for dK and dV, 32
+// queries for dQ) and take every fourth block of the other side, so the longest chain is a
+// quarter as long, and items of both kinds run in one launch, the longest first. Each wave stages
+// its own blocks (through registers into LDS: no barrier in the loop) and the
+// waves' sums are added through LDS in wave order at the end. One copy of a block in LDS serves
+// both kinds of operand: row operands as 16-byte reads of four k-steps (k = 8 i + 4 (lane / 32) +
+// j on both sides of the product; the 16 bytes of padding per row spread 16 rows over the banks)
+// and column operands as 4-byte reads of 32 consecutive columns. Two workgroups share a CU up to
+// head_dim 64 (70 KB of LDS each), one above.
+// The loads of a block are issued where it is staged, not a block ahead: the 64 registers per lane
+// that prefetching takes made the kernel spill and run 10% slower, and the second wave of the SIMD
+// covers the wait. 101 us against 169 for the 128-row kernels (causal, B=2 H=8 N=1024, head_dim
+// 64: 53 TFLOP/s; bwd32_faster has the other shapes).
+template <int D>
+struct Bwd32Cfg {
+    static constexpr int P = D + 4;          // pitch of a staged row (floats)
+    static constexpr int kTile = 32 * P;     // floats per staged 32-row block
+    static constexpr int kWave = 2 * kTile;  // two blocks per wave
+    static constexpr int kPerCu = D <= 64 ? 2 : 1;
+};
+
+// The wave's copy of 32 rows of a [rows, D] matrix: 16 bytes per lane and load.
+template <int D>
+struct WaveTile {
+    static constexpr int CPR = D / 4;       // 16-byte chunks per row
+    static constexpr int N = 32 * CPR / 64;  // loads per lane
+    u32x4 reg[N];
+    __device__ __forceinline__ void fetch(const float* src, int valid_rows, int lane) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int id = 64 * i + lane;
+            const int row = id / CPR;
+            reg[i] = u32x4{0u, 0u, 0u, 0u};
+            if (row < valid_rows) reg[i] = ld16(src + static_cast<size_t>(row) * D + (id % CPR) * 4);
+        }
+    }
+    __device__ __forceinline__ void stage(float* dst, int lane) const {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int id = 64 * i + lane;
+            st16(dst + (id / CPR) * Bwd32Cfg<D>::P + (id % CPR) * 4, reg[i]);
+        }
+    }
+};
+
+// This lane's operand values of row `row` of a [rows, D] matrix in global memory (k = 8 i +
+// 4 (lane / 32) + j at [4 i + j]); zeros where !ok.
+template <int D>
+__device__ __forceinline__ void row_values(const float* row, bool ok, int g2, float (&out)[D / 2]) {
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) {
+        f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (ok) v = __builtin_bit_cast(f32x4, ld16(row + 8 * i + 4 * g2));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out[4 * i + j] = v[j];
+    }
+}
+
+// Two products of a staged block's rows with this lane's row values: s = A a^T, t = B b^T.
+template <int D>
+__device__ __forceinline__ void row_products(const float* A, const float* B, int l32, int g2,
+                                             const float (&a)[D / 2], const float (&b)[D / 2],
+                                             f32x16& s, f32x16& t) {
+    const int at = l32 * Bwd32Cfg<D>::P + 4 * g2;
+    f32x4 x = __builtin_bit_cast(f32x4, ld16(A + at));
+    f32x4 y = __builtin_bit_cast(f32x4, ld16(B + at));
+    // The fences keep the reads one step ahead of their products and no further (left alone, the
+    // compiler reads the whole block first and spills).
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) {
+        f32x4 xn = x, yn = y;
+        if (i + 1 < D / 8) {
+            xn = __builtin_bit_cast(f32x4, ld16(A + at + 8 * (i + 1)));
+            yn = __builtin_bit_cast(f32x4, ld16(B + at + 8 * (i + 1)));
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s = mma_f32(x[j], a[4 * i + j], s);
+            t = mma_f32(y[j], b[4 * i + j], t);
+        }
+        x = xn;
+        y = yn;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// Adds the four waves' accumulators of one 32-row tile through LDS (`area`: 4 kTile floats, tile
+// w of wave w) and stores the rows below nrows times mul. Every wave passes the same barriers.
+template <int D>
+__device__ __forceinline__ void sum_and_store(const f32x16 (&acc)[D / 32], float mul, float* area,
+                                              int wave, int lane, float* base, int nrows) {
+    constexpr int P = Bwd32Cfg<D>::P;
+    constexpr int CPR = D / 4;
+    __syncthreads();  // the area is free
+    float* dst = area + wave * Bwd32Cfg<D>::kTile + (lane & 31) * P + 4 * (lane >> 5);
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            f32x4 w;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) w[u] = acc[dt][4 * a + u];
+            st16(dst + 32 * dt + 8 * a, __builtin_bit_cast(u32x4, w));
+        }
+    }
+    __syncthreads();
+    for (int id = threadIdx.x; id < 32 * CPR; id += 256) {
+        const int row = id / CPR;
+        const int col = (id % CPR) * 4;
+        f32x4 v = __builtin_bit_cast(f32x4, ld16(area + row * P + col));
+#pragma unroll
+        for (int w = 1; w < 4; ++w)
+            v += __builtin_bit_cast(f32x4, ld16(area + w * Bwd32Cfg<D>::kTile + row * P + col));
+        if (row < nrows)
+            st16(base + static_cast<size_t>(row) * D + col, __builtin_bit_cast(u32x4, v * mul));
+    }
+}
+
+template <int D>
+__global__ void __launch_bounds__(256, (Bwd32Cfg<D>::kPerCu))
+    bwd32_kernel(const float* __restrict__ Q, const float* __restrict__ K,
+                 const float* __restrict__ V, const float* __restrict__ L,
+                 const float* __restrict__ dO, const float* __restrict__ Dl,
+                 float* __restrict__ dQ, float* __restrict__ dK, float* __restrict__ dV, int Nq,
+                 int Nk, int coff, int group, int nqt, int nkt, int BH, float c, float scale,
+                 int causal, int head_major) {
+    using Cfg = Bwd32Cfg<D>;
+    constexpr int P = Cfg::P;
+    constexpr int NDT = D / 32;
+    __shared__ __attribute__((aligned(16))) float smem[4 * Cfg::kWave];
+    __shared__ __attribute__((aligned(16))) float s_ld[4][64];
+
+    // Eight workgroups of one kind (one per XCD), then eight of the other.
+    const int bid = blockIdx.x;
+    const int id = (bid >> 4) * 8 + (bid & 7);
+    const bool is_dq = (bid >> 3) & 1;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31;
+    const int g2 = lane >> 5;
+    float* ta = smem + wave * Cfg::kWave;  // Q or K block
+    float* tb = ta + Cfg::kTile;           // dO or V block
+    WaveTile<D> ca, cb;
+
+    if (is_dq) {
+        if (id >= BH * nqt) return;
+        int bh, rank;
+        item_order(id, BH, nqt, head_major, bh, rank);
+        const int q0 = (causal ? nqt - 1 - rank : rank) * 32;  // causal: longest first
+        const int q = q0 + l32;
+        const bool q_ok = q < Nq;
+        const size_t head = static_cast<size_t>(bh) * Nq * D;             // Q, dO, dQ
+        const size_t kv_head = static_cast<size_t>(bh / group) * Nk * D;  // K, V
+        const int kv_end = causal ? min(Nk, q0 + 32 + coff) : Nk;
+        const int nkb = (kv_end + 31) / 32;
+        auto fetch = [&](int kb) {
+            const size_t off = kv_head + static_cast<size_t>(kb) * 32 * D;
+            ca.fetch(K + off, Nk - kb * 32, lane);
+            cb.fetch(V + off, Nk - kb * 32, lane);
+        };
+        float qf[D / 2], of[D / 2];
+        row_values<D>(Q + head + static_cast<size_t>(q) * D, q_ok, g2, qf);
+        row_values<D>(dO + head + static_cast<size_t>(q) * D, q_ok, g2, of);
+        // Rows past Nq get L = +inf so that P = exp(S - L) is exactly 0 there.
+        const float l2 = q_ok ? L[static_cast<size_t>(bh) * Nq + q] * kLog2e : INFINITY;
+        const float d_row = q_ok ? Dl[static_cast<size_t>(bh) * Nq + q] : 0.0f;
+        f32x16 acc[NDT];
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) acc[dt] = f32x16{};
+        for (int kb = wave; kb < nkb; kb += 4) {
+            fetch(kb);
+            ca.stage(ta, lane);
+            cb.stage(tb, lane);
+            const int key0 = kb * 32;
+            f32x16 s = f32x16{};
+            f32x16 dp = f32x16{};
+            row_products<D>(ta, tb, l32, g2, qf, of, s, dp);
+            const bool masked = key0 + 32 > Nk || (causal && key0 + 31 > q0 + coff);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float p = fast_exp2(fmaf(s[r], c, -l2));
+                if (masked) {
+                    const int key = key0 + 8 * (r >> 2) + 4 * g2 + (r & 3);
+                    if (key >= Nk || (causal && key > q + coff)) p = 0.0f;
+                }
+                s[r] = p * (dp[r] - d_row);
+            }
+            // dQ^T += K^T dS^T: step r contracts the block's row 8 (r / 4) + 4 g2 + r % 4.
+            const float* col = ta + 4 * g2 * P + l32;
+            float x[NDT];
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) x[dt] = col[32 * dt];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float xn[NDT];
+                const int next = r < 15 ? (8 * ((r + 1) >> 2) + ((r + 1) & 3)) * P : 0;
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt) xn[dt] = col[next + 32 * dt];
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt) {
+                    acc[dt] = mma_f32(x[dt], s[r], acc[dt]);
+                    x[dt] = xn[dt];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        sum_and_store<D>(acc, scale, smem, wave, lane, dQ + head + static_cast<size_t>(q0) * D,
+                         Nq - q0);
+        return;
+    }
+
+    const int BHkv = BH / group;
+    if (id >= BHkv * nkt) return;
+    int bkv, kt;  // ascending key tiles: with a causal mask the first carry the most work
+    item_order(id, BHkv, nkt, head_major, bkv, kt);
+    const int k0 = kt * 32;
+    const int key = k0 + l32;
+    const bool key_ok = key < Nk;
+    const size_t kv_head = static_cast<size_t>(bkv) * Nk * D;  // K, V, dK, dV
+    // Query blocks [qb_begin, nqt) of each query head of the group as one sequence; with a causal
+    // mask the blocks before the first query that sees key k0 are skipped.
+    const int qb_begin = causal ? max(0, k0 - coff) / 32 : 0;
+    const int span = nqt - qb_begin;
+    const int n_it = group * span;
+    float lreg = 0.0f;
+    auto fetch = [&](int it) {
+        const int bh = bkv * group + it / span;
+        const int r0 = (qb_begin + it % span) * 32;
+        const size_t off = (static_cast<size_t>(bh) * Nq + r0) * D;
+        ca.fetch(Q + off, Nq - r0, lane);
+        cb.fetch(dO + off, Nq - r0, lane);
+        // Lanes 0-31: L of the block's rows, 32-63: D. Rows past Nq: P = 0.
+        const size_t row = static_cast<size_t>(bh) * Nq + r0 + l32;
+        const bool ok = r0 + l32 < Nq;
+        lreg = g2 ? (ok ? Dl[row] : 0.0f) : (ok ? L[row] * kLog2e : INFINITY);
+    };
+    float kf[D / 2], vf[D / 2];
+    row_values<D>(K + kv_head + static_cast<size_t>(key) * D, key_ok, g2, kf);
+    row_values<D>(V + kv_head + static_cast<size_t>(key) * D, key_ok, g2, vf);
+    f32x16 dk[NDT];
+    f32x16 dv[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) {
+        dk[dt] = f32x16{};
+        dv[dt] = f32x16{};
+    }
+    float* ld = s_ld[wave];
+    for (int it = wave; it < n_it; it += 4) {
+        const int q0 = (qb_begin + it % span) * 32;
+        fetch(it);
+        ca.stage(ta, lane);
+        cb.stage(tb, lane);
+        ld[lane] = lreg;
+        // S = Q K^T and dP = dO V^T: rows = queries, column = this lane's key.
+        f32x16 s = f32x16{};
+        f32x16 dp = f32x16{};
+        row_products<D>(ta, tb, l32, g2, kf, vf, s, dp);
+        const bool masked = causal && k0 + 31 > q0 + coff;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const f32x4 lv = __builtin_bit_cast(f32x4, ld16(ld + 8 * a + 4 * g2));
+            const f32x4 dd = __builtin_bit_cast(f32x4, ld16(ld + 32 + 8 * a + 4 * g2));
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int r = 4 * a + u;
+                float p = fast_exp2(fmaf(s[r], c, -lv[u]));
+                if (masked && key > q0 + 8 * a + 4 * g2 + u + coff) p = 0.0f;
+                s[r] = p;
+                dp[r] = p * (dp[r] - dd[u]);
+            }
+        }
+        // dV^T += dO^T P and dK^T += Q^T dS: step r contracts row 8 (r / 4) + 4 g2 + r % 4.
+        const int col = 4 * g2 * P + l32;
+        float x[NDT], y[NDT];
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) {
+            x[dt] = tb[col + 32 * dt];
+            y[dt] = ta[col + 32 * dt];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float xn[NDT], yn[NDT];
+            const int next = r < 15 ? (8 * ((r + 1) >> 2) + ((r + 1) & 3)) * P : 0;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+                xn[dt] = tb[col + next + 32 * dt];
+                yn[dt] = ta[col + next + 32 * dt];
+            }
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+                dv[dt] = mma_f32(x[dt], s[r], dv[dt]);
+                dk[dt] = mma_f32(y[dt], dp[r], dk[dt]);
+                x[dt] = xn[dt];
+                y[dt] = yn[dt];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    const size_t out = kv_head + static_cast<size_t>(k0) * D;
+    sum_and_store<D>(dk, scale, smem, wave, lane, dK + out, Nk - k0);
+    sum_and_store<D>(dv, 1.0f, smem, wave, lane, dV + out, Nk - k0);
+}
+
+// ------------------------------------------------------------------------------------------
+// 5. Backward for head_dim 64, 128 and 256 (fp16 / bf16)
 // ------------------------------------------------------------------------------------------
 // Row statistics for bwd_fused_kernel: LD[bh * Npad + r] = (L * log2(e), D) for r < N and
 // (+inf, 0) for the padding rows N <= r < Npad (Npad = N rounded up to 32), so that P = 0 there
@@ -1221,7 +1531,35 @@ struct BwdShape {
     int group;  // query heads per key/value head
 };
 
-// Generic path (fp32, and head_dim 32 / 64 / 96 / 256): delta, dq_kernel, dkdv_kernel.
+// Whether bwd32_kernel (32-row items whose blocks are spread over the waves) beats the kernels of
+// 128-row items for an fp32 backward, from a model of both in units of one matrix-core product over
+// a 128-row item (dq 3, dkdv 4 per query head): the 128-row kernels run in whole rounds of
+// workgroups, each as long as its longest item, or, under a causal mask, in their total plus a
+// tail; bwd32_kernel in its total, at a lower rate, since each wave stages blocks of its own.
+// Measured (128-row kernels -> bwd32_kernel, us, whole backward). Taken: causal B=2 H=8 N=1024
+// head_dim 64 169 -> 101, head_dim 32 104 -> 52; B=2 H=16 N=4096 head_dim 64 2930 -> 2330; B=1 H=8
+// N=4096 head_dim 128 2037 -> 1343; 32 heads over 8, N=512, head_dim 128 575 -> 173; non-causal
+// B=2 H=8 N=1024 head_dim 64 170 -> 156. Not taken: causal B=2 H=16 N=4096 head_dim 128 4726, 5314;
+// non-causal B=2 H=16 N=4096 head_dim 64 3853, 4455; B=1 H=8 N=2048 head_dim 128 586, 661;
+// 32 heads over 8, N=2000, head_dim 128 3240, 4030.
+template <int D>
+bool bwd32_faster(const BwdShape& sh, bool causal, double qblocks, double kblocks) {
+    constexpr double kPer = D <= 64 ? 2.0 : 1.0;  // workgroups of the 128-row kernels per CU
+    const double rate = D <= 64 ? 1.13 : sh.group > 1 && !causal ? 1.6 : 1.25;
+    const double cus = compute_units();
+    const double frac = causal ? (2.0 * sh.Nk - sh.Nq + 128.0) / (2.0 * sh.Nk) : 1.0;
+    const double dq = 3.0, dkdv = 4.0 * sh.group;
+    auto rounds = [&](double blocks) {
+        return causal ? std::max(1.0, kPer * (blocks * frac / (cus * kPer) + 0.4))
+                      : std::max(1.0, kPer * std::ceil(blocks / (cus * kPer)));
+    };
+    const double old_time = qblocks + kblocks <= cus
+                                ? std::max(dq, dkdv)
+                                : rounds(qblocks) * dq + rounds(kblocks) * dkdv;
+    return (qblocks * dq + kblocks * dkdv) * frac / cus * rate < old_time;
+}
+
+// Generic path (fp32): delta_kernel, then bwd32_kernel or dq_kernel and dkdv_kernel.
 template <typename T, int D>
 FlashAttentionError run_backward_two_pass(const T* Q, const T* K, const T* V, const T* O,
                                           const float* L, const T* dO, T* dQ, T* dK, T* dV,
@@ -1260,10 +1598,27 @@ FlashAttentionError run_backward_two_pass(const T* Q, const T* K, const T* V, co
     const long long qblocks = static_cast<long long>(nqb) * sh.BH;
     const long long kblocks = static_cast<long long>(nkb) * BHkv;
     if (qblocks + kblocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;
-    // Both grids together fit in one round of workgroups: one launch, so that the dq and dkdv
-    // items run side by side instead of each half-filling the GPU in turn (up to head_dim 128:
-    // the two bodies' LDS arrays add up).
     if constexpr (D <= 128) {
+        if (bwd32_faster<D>(sh, causal, static_cast<double>(qblocks), static_cast<double>(kblocks))) {
+            const int nqt = (sh.Nq + 31) / 32;
+            const int nkt = (sh.Nk + 31) / 32;
+            const long long items =
+                std::max(static_cast<long long>(nqt) * sh.BH, static_cast<long long>(nkt) * BHkv);
+            const long long blocks = (items + 7) / 8 * 16;
+            if (blocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;
+            // Longest items first, unless all are of one length or there are many per slot.
+            const bool head_major =
+                !causal || items >= 8LL * dev::Bwd32Cfg<D>::kPerCu * compute_units();
+            tok = profile_kernel<T, D>("backward_dq_dkdv");
+            launch_kernel(tok, (dev::bwd32_kernel<D>), dim3(static_cast<unsigned>(blocks)),
+                          dim3(256), 0, stream, Q, K, V, L, dO, delta, dQ, dK, dV, sh.Nq, sh.Nk,
+                          coff, sh.group, nqt, nkt, sh.BH, c, scale, causal ? 1 : 0,
+                          head_major ? 1 : 0);
+            return from_hip(hipGetLastError());
+        }
+        // Both grids together fit in one round of workgroups: one launch, so that the dq and
+        // dkdv items run side by side instead of each half-filling the GPU in turn (up to
+        // head_dim 128: the two bodies' LDS arrays add up).
         if (qblocks + kblocks <= compute_units()) {
             tok = profile_kernel<T, D>("backward_dq_dkdv");
             launch_kernel(tok, (dev::dq_dkdv_kernel<T, D>),
@@ -1287,8 +1642,7 @@ FlashAttentionError run_backward_two_pass(const T* Q, const T* K, const T* V, co
                        dim3(KCfg::kThreads), 0, stream, q, k, v, L, go, delta,
                        reinterpret_cast<E*>(dK), reinterpret_cast<E*>(dV), sh.Nq, sh.Nk, coff,
                        sh.group, nkb, c, scale, causal ? 1 : 0);
-    err = from_hip(hipGetLastError());
-    return err;
+    return from_hip(hipGetLastError());
 }
 
 // Path for fp16 / bf16 at head_dim 128 and 64: delta_ld_kernel, then bwd_fused_kernel (dq and
