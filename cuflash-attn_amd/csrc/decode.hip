@@ -776,22 +776,13 @@ namespace detail {
 
 namespace {
 
-int device_cu_count() {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-        return 256;
-    return cus;
-}
-
 // Split count: enough (batch*head, split) workgroups to give every CU per_cu, with chunks of at
 // least min_chunk keys; an explicit request is clamped to [1, min(1024, ceil(kv_len / 16))]
 // (1024 = dev::kMaxSplits, the combine kernel's bound).
 int choose_splits(int requested, int BH, int kv_len, int min_chunk, int per_cu) {
     const int max_useful = std::max(1, std::min(dev::kMaxSplits, (kv_len + 15) / 16));
     if (requested > 0) return std::min(requested, max_useful);
-    const int target_blocks = per_cu * device_cu_count();
+    const int target_blocks = per_cu * compute_units();
     int s = (target_blocks + BH - 1) / BH;
     s = std::min(s, std::max(1, kv_len / min_chunk));
     return std::max(1, std::min(s, max_useful));

@@ -173,10 +173,16 @@ def load_library(path: Optional[str] = None) -> CuFlashLibrary:
 # PyTorch tensor helpers (device memory and streams come from PyTorch-ROCm)
 # ---------------------------------------------------------------------------------------------
 
-def _torch():
-    import torch  # noqa: WPS433 (imported lazily: the ctypes layer itself needs no torch)
+_TORCH = None
 
-    return torch
+
+def _torch():
+    global _TORCH
+    if _TORCH is None:
+        import torch  # noqa: WPS433 (imported lazily: the ctypes layer itself needs no torch)
+
+        _TORCH = torch
+    return _TORCH
 
 
 def _suffix(t) -> str:
@@ -197,9 +203,12 @@ def _check(tensors, dtype):
 
 
 def _stream_ptr(stream=None):
+    if stream is not None:
+        return stream.cuda_stream
+    # The handle of torch.cuda.current_stream() without building a Stream object around it (2.8 us
+    # of a small call's 12.8).
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _raise(lib: CuFlashLibrary, status: int):
@@ -218,7 +227,7 @@ def flash_attention_forward(q, k, v, scale: Optional[float] = None, causal: bool
         raise ValueError("q, k, v must have the same shape")
     scale = float(D ** -0.5) if scale is None else float(scale)
     out = torch.empty_like(q) if out is None else out
-    lse = torch.empty((B, H, N), device=q.device, dtype=torch.float32) if lse is None else lse
+    lse = q.new_empty((B, H, N), dtype=torch.float32) if lse is None else lse
     status = lib.fn("forward", _suffix(q))(q.data_ptr(), k.data_ptr(), v.data_ptr(),
                                            out.data_ptr(), lse.data_ptr(), B, H, N, D, scale,
                                            bool(causal), _stream_ptr(stream))
@@ -266,7 +275,7 @@ def flash_attention_forward_ext(q, k, v, scale: Optional[float] = None, causal: 
     B, H, Hkv, Nq, Nk, D = _ext_shapes(q, k, v)
     scale = float(D ** -0.5) if scale is None else float(scale)
     out = torch.empty_like(q) if out is None else out
-    lse = torch.empty((B, H, Nq), device=q.device, dtype=torch.float32) if lse is None else lse
+    lse = q.new_empty((B, H, Nq), dtype=torch.float32) if lse is None else lse
     status = lib.fn("forward_ext", _suffix(q))(q.data_ptr(), k.data_ptr(), v.data_ptr(),
                                                out.data_ptr(), lse.data_ptr(), B, H, Hkv, Nq,
                                                Nk, D, scale, bool(causal), _stream_ptr(stream))
@@ -309,7 +318,7 @@ def flash_attention_decode(q, k, v, scale: Optional[float] = None, num_splits: i
     Hkv, kv_len = k.shape[1], k.shape[2]
     scale = float(D ** -0.5) if scale is None else float(scale)
     out = torch.empty_like(q) if out is None else out
-    lse = torch.empty((B, H, 1), device=q.device, dtype=torch.float32) if lse is None else lse
+    lse = q.new_empty((B, H, 1), dtype=torch.float32) if lse is None else lse
     if Hkv == H:
         status = lib.fn("decode", _suffix(q))(q.data_ptr(), k.data_ptr(), v.data_ptr(),
                                               out.data_ptr(), lse.data_ptr(), B, H, kv_len, D,
@@ -346,7 +355,7 @@ def flash_attention_decode_paged(q, k_cache, v_cache, block_table, seq_lens,
     page_size, Hkv = k_cache.shape[1], k_cache.shape[2]
     scale = float(D ** -0.5) if scale is None else float(scale)
     out = torch.empty_like(q) if out is None else out
-    lse = torch.empty((B, H, 1), device=q.device, dtype=torch.float32) if lse is None else lse
+    lse = q.new_empty((B, H, 1), dtype=torch.float32) if lse is None else lse
     status = lib.fn("decode_paged", _suffix(q))(q.data_ptr(), k_cache.data_ptr(),
                                                 v_cache.data_ptr(), out.data_ptr(),
                                                 lse.data_ptr(), block_table.data_ptr(),
