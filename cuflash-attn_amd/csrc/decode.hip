@@ -808,6 +808,8 @@ constexpr int kMinChunk = 128;
 // in flight (16 x 8 key/value heads x 32768 keys: 130 -> 89 us; head_dim 64: 156 -> 161 us).
 constexpr int mma_per_cu(int D) { return D == 32 ? 8 : 4; }
 constexpr int kRowsPerCu = 1;
+// Longest cache that an automatic grouped-query decode gives to the forward (run_decode_grouped).
+constexpr int kShortCache = 1024;
 
 // MMA: the matrix-core kernels, splits of whole 32-key blocks: decode_mma_rows_kernel (paged,
 // one workgroup per (batch, 512 / D key/value heads, split)) or decode_mma_kernel (one
@@ -901,7 +903,7 @@ FlashAttentionError run_decode(const T* Q, const T* K, const T* V, T* O, float* 
 // K/V row is then read once for G query heads.
 template <typename T, int D, bool PAGED>
 FlashAttentionError run_decode_grouped(const T* Q, const T* K, const T* V, T* O, float* L, int B,
-                                       const dev::DecodeArgs& a, int num_splits,
+                                       const dev::DecodeArgs& a, float scale, int num_splits,
                                        const FixedScratch& fx, hipStream_t stream) {
     const int hpk = a.H / a.Hkv;
     if constexpr (!std::is_same<T, float>::value) {
@@ -911,6 +913,16 @@ FlashAttentionError run_decode_grouped(const T* Q, const T* K, const T* V, T* O,
         // 64 and 32) whose per-lane byte offset within a group, (rows - 1) Hkv D 2 + 256, fits
         // 32 bits.
         constexpr int kGroupRows = dev::TileGroups<D>::kRows;
+        // Short caches: the forward of one query per head packs the query heads of a key/value
+        // head into one tile and spreads its keys over the waves of one workgroup: one launch and
+        // no partials. Per call, us, 32 heads over 8: head_dim 128, 1000 keys, B = 1
+        // 11.1 -> 8.7, B = 16 17.1 -> 13.2, B = 64 50.0 -> 41.4; 512 keys, B = 1 9.9 -> 7.2;
+        // head_dim 64, 512 keys, B = 64 17.6 -> 12.6. From 2000 keys on the split kernels are
+        // level or faster (B = 64, head_dim 128: 87.2 against 93.4).
+        if (!PAGED && num_splits == 0 && fx.ptr == nullptr && hpk >= 2 && hpk <= 32 && a.kv_len <= kShortCache &&
+            static_cast<long long>(B) * a.Hkv <= 2LL * compute_units())
+            return launch_forward_ext<T>(Q, K, V, O, L, B, a.H, a.Hkv, 1, a.kv_len, D,
+                                         scale, false, stream);
         if (hpk >= 2 && hpk <= 32 &&
             (!PAGED || a.Hkv % (512 / D) == 0 ||
              (a.page_size % kGroupRows == 0 && a.Hkv <= (1 << 20))))
@@ -927,15 +939,18 @@ FlashAttentionError run_decode_grouped(const T* Q, const T* K, const T* V, T* O,
 
 template <typename T, bool PAGED>
 FlashAttentionError run_decode_dims(const T* Q, const T* K, const T* V, T* O, float* L, int B,
-                                    const dev::DecodeArgs& a, int head_dim, int num_splits,
-                                    const FixedScratch& fx, hipStream_t stream) {
+                                    const dev::DecodeArgs& a, float scale, int head_dim,
+                                    int num_splits, const FixedScratch& fx, hipStream_t stream) {
     switch (head_dim) {
         case 32:
-            return run_decode_grouped<T, 32, PAGED>(Q, K, V, O, L, B, a, num_splits, fx, stream);
+            return run_decode_grouped<T, 32, PAGED>(Q, K, V, O, L, B, a, scale, num_splits, fx,
+                                                    stream);
         case 64:
-            return run_decode_grouped<T, 64, PAGED>(Q, K, V, O, L, B, a, num_splits, fx, stream);
+            return run_decode_grouped<T, 64, PAGED>(Q, K, V, O, L, B, a, scale, num_splits, fx,
+                                                    stream);
         case 128:
-            return run_decode_grouped<T, 128, PAGED>(Q, K, V, O, L, B, a, num_splits, fx, stream);
+            return run_decode_grouped<T, 128, PAGED>(Q, K, V, O, L, B, a, scale, num_splits, fx,
+                                                    stream);
     }
     return FlashAttentionError::UNSUPPORTED_HEAD_DIM;
 }
@@ -962,8 +977,8 @@ FlashAttentionError launch_decode_gqa(const T* Q, const T* K, const T* V, T* O, 
                                       int kv_len, int head_dim, float scale, int num_splits,
                                       hipStream_t stream) {
     const dev::DecodeArgs a = decode_args(num_heads, num_kv_heads, kv_len, scale);
-    return run_decode_dims<T, false>(Q, K, V, O, L, batch_size, a, head_dim, num_splits,
-                                     kAllocate, stream);
+    return run_decode_dims<T, false>(Q, K, V, O, L, batch_size, a, scale, head_dim,
+                                     num_splits, kAllocate, stream);
 }
 
 template <typename T>
@@ -988,7 +1003,7 @@ FlashAttentionError launch_decode_paged(const T* Q, const T* K_cache, const T* V
     a.page_size = page_size;
     a.max_pages = max_pages_per_seq;
     a.page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
-    return run_decode_dims<T, true>(Q, K_cache, V_cache, O, L, batch_size, a, head_dim,
+    return run_decode_dims<T, true>(Q, K_cache, V_cache, O, L, batch_size, a, scale, head_dim,
                                     num_splits, kAllocate, stream);
 }
 
@@ -1041,8 +1056,8 @@ FlashAttentionError launch_decode_noalloc(const T* Q, const T* K, const T* V, T*
     if (err != FlashAttentionError::SUCCESS) return err;
     const dev::DecodeArgs a = decode_args(num_heads, num_heads, kv_len, scale);
     const FixedScratch fx{ptr, kDecodeScratchBytes};
-    return run_decode_dims<T, false>(Q, K, V, O, L, batch_size, a, head_dim, num_splits, fx,
-                                     stream);
+    return run_decode_dims<T, false>(Q, K, V, O, L, batch_size, a, scale, head_dim, num_splits,
+                                     fx, stream);
 }
 
 template FlashAttentionError launch_decode_noalloc<__half>(const __half*, const __half*,

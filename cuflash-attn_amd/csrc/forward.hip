@@ -1960,12 +1960,14 @@ struct FwdShape {
 //  * fwd16_rows_kernel: a workgroup walks its longest tile in rounds of one block per wave, tb
 //    each, and t0 for its start, merge and store; as many workgroups as the slots run at once.
 //    Several chunks add the merge kernel and the partials, written and read at about 4 TB/s.
-//  * the general kernels, when their 128-row workgroups all run at once: g per 64-key block of the
-//    longest row, up to 1.3 g with two workgroups per CU at head_dim 64 and 32.
+//  * the general kernels: g per 64-key block of the longest row while their 128-row workgroups all
+//    run at once (more with two workgroups per CU), else 1.5 g per round of them and block of the
+//    average row. They do not pack heads: a few tokens of many heads fill their rows badly.
 // bf16/fp16, causal, B = 1, before -> after: 8 heads, head_dim 128, N = 129 8.4 -> 6.3, 1024 23.9 ->
 // 11.9, 4096 82 -> 64; head_dim 64, N = 256 6.3 -> 5.0, 1024 16.9 -> 8.5, 4096 55.6 -> 34.5;
 // head_dim 256, N = 1024 40.1 -> 22.0; 32 heads over 8 against 8253 keys, head_dim 128: 61 queries
-// 160 -> 22 (4 chunks), one query 156 -> 11.6 (16 chunks). The other side of the line: 32 heads,
+// 160 -> 22 (4 chunks), one query 156 -> 11.6 (16 chunks); one query of 64 x 32 heads over 8,
+// 1000 keys 206 -> 41. The other side of the line: 32 heads,
 // head_dim 128, N = 1024 25.7 general, 32.7 here; head_dim 64, N = 1536 25.8 and 26.9.
 template <int D>
 int forward_rows_chunks(const FwdShape& sh, bool causal) {
@@ -1977,7 +1979,6 @@ int forward_rows_chunks(const FwdShape& sh, bool causal) {
     const double slots = D <= 64 ? 2 * cus : cus;
     const double rows = static_cast<double>(sh.BH) * sh.Nq;
     const double units = static_cast<double>(sh.BH) * ((sh.Nq + 127) / 128);
-    if (units > 2 * cus) return 0;
     const double tiles = static_cast<double>(sh.BH / sh.group) *
                          ((static_cast<long long>(sh.group) * sh.Nq + 31) / 32);
     const double longest = (sh.Nk + 31) / 32 / static_cast<double>(kWaves);
@@ -1994,8 +1995,15 @@ int forward_rows_chunks(const FwdShape& sh, bool causal) {
             chunks = n;
         }
     }
-    const double crowd = D <= 64 ? 1.0 + 0.3 * std::min(1.0, std::max(0.0, units / cus - 1.0)) : 1.0;
-    return 1.1 * best < g * crowd * ((sh.Nk + 63) / 64) ? chunks : 0;
+    const double blocks = (sh.Nk + 63) / 64;
+    double general;
+    if (units > 2 * cus)
+        general = 1.5 * g * blocks * (average / longest) * units / (2 * cus);
+    else if (D <= 64)
+        general = g * blocks * (1.0 + 0.3 * std::min(1.0, std::max(0.0, units / cus - 1.0)));
+    else
+        general = g * blocks + 4.0 * units / cus;
+    return 1.1 * best < general ? chunks : 0;
 }
 
 // One workgroup per (32 rows of a key/value head's query heads, chunk of keys), and a merge kernel

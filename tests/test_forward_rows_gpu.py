@@ -37,7 +37,12 @@ SHAPES = [
     (1, 3, 1, 40, 1300, 256, True),
     (1, 2, 2, 300, 300, 256, False),
     (1, 8, 1, 17, 2048, 128, False),
+    (20, 32, 8, 1, 70, 64, False),
+    (20, 32, 8, 2, 130, 128, True),
 ]
+
+# B, H, Hkv, keys, D: grouped-query decodes of short caches, which run the same kernel.
+DECODES = [(1, 32, 8, 1000, 128), (3, 12, 2, 1, 128), (2, 32, 1, 33, 64), (5, 8, 4, 1024, 32)]
 
 
 @pytest.mark.gpu
@@ -56,3 +61,21 @@ def test_forward_of_few_rows_matches_the_oracle(torch_gpu, dtype, shape):
                                   causal)
     assert max_abs(synth.to_numpy(o), o_ref) <= 2.25 * UNIT[dtype]
     assert max_abs(synth.to_numpy(lse), l_ref) <= 2e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("shape", DECODES, ids=lambda s: "-".join(map(str, s)))
+def test_short_grouped_decode_matches_the_oracle(torch_gpu, dtype, shape):
+    B, H, Hkv, Nk, D = shape
+    q = synth.round_to(synth.uniform(1, (B, H, 1, D)), dtype)
+    k, v = (synth.round_to(synth.uniform(s, (B, Hkv, Nk, D)), dtype) for s in (2, 3))
+    print(f"[short decode] {dtype} {shape}", flush=True)
+    for scale in (2.0 * D ** -0.5, 0.0):
+        o, lse = cuflash_attn.flash_attention_decode(
+            *(synth.to_torch(x, dtype) for x in (q, k, v)), scale=scale)
+        torch_gpu.cuda.synchronize()
+        o_ref, l_ref = oracle.forward(q, *(np.repeat(x, H // Hkv, axis=1) for x in (k, v)), scale,
+                                      False)
+        assert max_abs(synth.to_numpy(o), o_ref) <= 2.25 * UNIT[dtype]
+        assert max_abs(synth.to_numpy(lse), l_ref) <= 2e-5
