@@ -20,7 +20,8 @@
 // so each lane owns one query row of dQ, or one key row of dK/dV, for the whole kernel. For
 // fp16/bf16 P and dS are rounded to the input type before their products (fp32 accumulate).
 // For fp16/bf16 (every head_dim) the same steps run as delta_ld_kernel, then
-// dq_lds_tiles and dkdv_lds_tiles items in one launch (bwd_fused_kernel, section 5). Every path is
+// dq_lds_tiles and dkdv_lds_tiles items in one launch (bwd_fused_kernel, section 5), or in smaller
+// items for launches that would not fill the GPU (bwd16_rows_kernel, section 6). Every path is
 // deterministic: no atomics, and each output element is written by exactly one lane.
 //
 // Shapes: Q, O, dO, dQ are [BH, Nq, D], K, V, dK, dV are [BH / group, Nk, D] (query head bh
@@ -1517,6 +1518,354 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// ------------------------------------------------------------------------------------------
+// 6. Small fp16 / bf16 backward: one 32-row tile per workgroup, its blocks over the waves
+// ------------------------------------------------------------------------------------------
+// bwd_fused_kernel's items are 128 rows whose waves each walk every 32-row block of the other side,
+// so a launch of few items is as long as its longest item's chain of blocks, on few CUs. Here (as in
+// bwd32_kernel) the waves of a workgroup share one 32-row tile and take every NW-th block through
+// LDS-DMA double buffers of their own (no barrier in the loop), and their sums are added through
+// LDS in wave order at the end: chains a fourth or an eighth as long over four times the workgroups.
+// A key tile runs over all query heads of its group, so grouped heads need no shares. Products,
+// roundings and the order inside a block are those of dq_lds_tiles and dkdv_lds_tiles.
+// Backward kernel, causal, us (bwd_fused_kernel -> this): head_dim 64, 8 heads, N=300 13.1 -> 6.8,
+// N=1024 28.5 -> 14.4, 4 heads, N=2048 50.2 -> 18.9; head_dim 128, 4 heads, N=1024 41.5 -> 18.4,
+// 8 heads 42.7 -> 24.2; head_dim 96, 8 heads, N=1024 36.0 -> 21.1. bwd16_rows_faster draws the line:
+// every wave loads its own tiles, four times the bytes per product of the fused items.
+template <int D>
+struct Bwd16RowsCfg {
+    static constexpr int kWaves = D <= 64 ? 8 : 4;  // two waves per SIMD, or one (registers)
+    static constexpr int kTile = (32 / TileGroups<D>::kRows) * TileGroups<D>::kBytes;
+    static constexpr int kSet = 2 * kTile + 256;  // Q and dO (or K and V) block, 32 (L, D)
+    static constexpr int P = D + 4;               // pitch of the merge rows (floats)
+    static constexpr int kTiles = kWaves * 2 * kSet;
+    static constexpr int kMerge = kWaves * 32 * P * 4;
+    static constexpr int kLds = kTiles > kMerge ? kTiles : kMerge;
+};
+
+// Adds the waves' accumulators of one 32-row tile through LDS and stores the rows below nrows
+// times mul, rounded to T. Every wave passes the same barriers.
+template <typename T, int D>
+__device__ __forceinline__ void sum_and_store16(const f32x16 (&acc)[D / 32], float mul,
+                                                unsigned char* area, int wave, int lane,
+                                                uint16_t* base, int nrows) {
+    using Cfg = Bwd16RowsCfg<D>;
+    constexpr int P = Cfg::P;
+    constexpr int CPR = D / 8;
+    float* rows = reinterpret_cast<float*>(area);
+    __syncthreads();  // the area is free
+    float* dst = rows + (wave * 32 + (lane & 31)) * P + 4 * (lane >> 5);
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            f32x4 w;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) w[u] = acc[dt][4 * a + u];
+            st16(dst + 32 * dt + 8 * a, __builtin_bit_cast(u32x4, w));
+        }
+    }
+    __syncthreads();
+    for (int id = threadIdx.x; id < 32 * CPR; id += 64 * Cfg::kWaves) {
+        const int row = id / CPR;
+        const int col = (id % CPR) * 8;
+        f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+#pragma unroll
+        for (int w = 0; w < Cfg::kWaves; ++w) {
+            const float* src = rows + (w * 32 + row) * P + col;
+            a += __builtin_bit_cast(f32x4, ld16(src));
+            b += __builtin_bit_cast(f32x4, ld16(src + 4));
+        }
+        if (row < nrows) {
+            u32x4 v;
+            v[0] = Elem<T>::pack2(a[0] * mul, a[1] * mul);
+            v[1] = Elem<T>::pack2(a[2] * mul, a[3] * mul);
+            v[2] = Elem<T>::pack2(b[0] * mul, b[1] * mul);
+            v[3] = Elem<T>::pack2(b[2] * mul, b[3] * mul);
+            st16(base + static_cast<size_t>(row) * D + col, v);
+        }
+    }
+}
+
+template <typename T, int D>
+__global__ void __launch_bounds__(64 * Bwd16RowsCfg<D>::kWaves, 1)
+    bwd16_rows_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
+                      const uint16_t* __restrict__ V, const float2* __restrict__ LD,
+                      const uint16_t* __restrict__ dO, uint16_t* __restrict__ dQ,
+                      uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int Nq, int Nk,
+                      int coff, int group, int Npad, int nkt, int BH, float c, float scale,
+                      int causal) {
+    using Cfg = Bwd16RowsCfg<D>;
+    using G = TileGroups<D>;
+    constexpr int NW = Cfg::kWaves;
+    constexpr int QT = Cfg::kTile;
+    constexpr int KS = D / 16;
+    constexpr int NDT = D / 32;
+    constexpr int GR = G::kRows;
+    constexpr int kAhead = 3;
+    using frag = typename Elem<T>::frag;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[Cfg::kLds];
+
+    // Eight workgroups of one kind (one per XCD), then eight of the other.
+    const int bid = blockIdx.x;
+    const int id = (bid >> 4) * 8 + (bid & 7);
+    const bool is_dq = (bid >> 3) & 1;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31;
+    const int g2 = lane >> 5;
+    const int nqt = Npad / 32;
+    const float cs = fmaxf(c, kFltMin);
+    unsigned char* sets = smem + wave * 2 * Cfg::kSet;
+
+    const int ld_row = G::ld_row(lane);
+    const int ld_col = G::ld_col(lane);
+    const unsigned ld_voff = static_cast<unsigned>((ld_row * D + ld_col) * 2);
+    // Rows r0 .. r0 + 31 of a [n, D] matrix (rows past n clamped to the last one).
+    auto load_tile = [&](const uint16_t* src, int r0, int n, unsigned char* dst) {
+        if (r0 + 32 <= n) {
+#pragma unroll
+            for (int g = 0; g < 32 / GR; ++g)
+                lds_dma16_async_s(src + static_cast<size_t>(r0 + GR * g) * D, ld_voff,
+                                  dst + g * G::kBytes);
+        } else {
+#pragma unroll
+            for (int g = 0; g < 32 / GR; ++g) {
+                const int row = min(r0 + GR * g + ld_row, n - 1);
+                lds_dma16_async(src + static_cast<size_t>(row) * D + ld_col, dst + g * G::kBytes);
+            }
+        }
+    };
+    const int row_base[2] = {G::row_base(lane, 0), G::row_base(lane, 1)};
+    const int tr_off = G::tr_off(lane);
+    // s += A a^T and t += B b^T over the tiles at ta and tb (operand i: even A, odd B, k-step
+    // i / 2, read kAhead products ahead).
+    auto row_products = [&](const unsigned char* ta, const unsigned char* tb, const frag (&a)[KS],
+                            const frag (&b)[KS], f32x16& s, f32x16& t) {
+        frag f[2 * KS];
+        auto operand = [&](int k) {
+            return as_frag<T>(ld16((k & 1 ? tb : ta) + row_base[(k >> 1) & 1] + G::k_off(k >> 1)));
+        };
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) f[k] = operand(k);
+#pragma unroll
+        for (int i = 0; i < 2 * KS; ++i) {
+            if (i + kAhead < 2 * KS) f[i + kAhead] = operand(i + kAhead);
+            if (i & 1)
+                t = Elem<T>::mma(f[i], b[i >> 1], t);
+            else
+                s = Elem<T>::mma(f[i], a[i >> 1], s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto pack8 = [](const f32x16& x, int j) {
+        return pack_frag<T>(x[8 * j + 0], x[8 * j + 1], x[8 * j + 2], x[8 * j + 3], x[8 * j + 4],
+                            x[8 * j + 5], x[8 * j + 6], x[8 * j + 7]);
+    };
+    auto row_frags = [&](const uint16_t* row, bool ok, frag (&out)[KS]) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (ok) v = ld16(row + 16 * ks + 8 * g2);
+            out[ks] = as_frag<T>(v);
+        }
+    };
+
+    if (is_dq) {
+        if (id >= BH * nqt) return;
+        int bh, rank;
+        item_order(id, BH, nqt, causal == 0, bh, rank);
+        const int q0 = (causal ? nqt - 1 - rank : rank) * 32;  // causal: longest first
+        const int q = q0 + l32;
+        const size_t head = static_cast<size_t>(bh) * Nq * D;             // Q, dO, dQ
+        const size_t kv_head = static_cast<size_t>(bh / group) * Nk * D;  // K, V
+        const int kv_end = causal ? min(Nk, q0 + 32 + coff) : Nk;
+        const int nkb = (kv_end + 31) / 32;
+        auto load = [&](int kb, int b) {
+            unsigned char* set = sets + b * Cfg::kSet;
+            load_tile(K + kv_head, kb * 32, Nk, set);
+            load_tile(V + kv_head, kb * 32, Nk, set + QT);
+        };
+        frag qf[KS], of[KS];
+        row_frags(Q + head + static_cast<size_t>(q) * D, q < Nq, qf);
+        row_frags(dO + head + static_cast<size_t>(q) * D, q < Nq, of);
+        // (L log2 e, D) of this lane's query; padding rows give P = 0.
+        float lq, dq;
+        if constexpr (neg_d_rows<D>()) {
+            const float* blk = reinterpret_cast<const float*>(LD) +
+                               (static_cast<size_t>(bh) * Npad + q0) * 2 + l32;
+            lq = blk[0];
+            dq = -blk[32];
+        } else {
+            const float2 v = LD[static_cast<size_t>(bh) * Npad + q];
+            lq = v.x;
+            dq = v.y;
+        }
+        f32x16 acc[NDT];
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) acc[dt] = f32x16{};
+        if (wave < nkb) load(wave, 0);
+        int b = 0;
+        for (int kb = wave; kb < nkb; kb += NW, b ^= 1) {
+            wait_loads<0>();  // block kb has landed
+            wait_lds();       // and the reads of the block before it are done
+            if (kb + NW < nkb) load(kb + NW, b ^ 1);
+            const unsigned char* kt = sets + b * Cfg::kSet;
+            const int key0 = kb * 32;
+            f32x16 s = f32x16{};
+            f32x16 dp = f32x16{};
+            if constexpr (neg_d_rows<D>()) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dp[r] = -dq;
+            }
+            row_products(kt, kt + QT, qf, of, s, dp);
+            if (key0 + 32 > Nk || (causal && key0 + 31 > q0 + coff)) {
+                const int lim = min(Nk, causal ? q + 1 + coff : Nk) - key0 - 4 * g2;
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    s[r] = (8 * (r >> 2) + (r & 3) < lim) ? s[r] : -INFINITY;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float p = fast_exp2(fmaf(s[r], cs, -lq));
+                if constexpr (neg_d_rows<D>())
+                    s[r] = p * dp[r];
+                else
+                    s[r] = p * (dp[r] - dq);
+            }
+            // dQ^T += K^T dS^T
+            const frag bs[2] = {pack8(s, 0), pack8(s, 1)};
+            constexpr int kMma = 2 * NDT;
+            constexpr int kTrAhead = kMma < kAhead ? kMma : kAhead;
+            frag f[kMma];
+            auto operand = [&](int i) {
+                const unsigned char* a = kt + tr_off + (i / NDT) * G::kTrRows16 + G::dtile_off(i % NDT);
+                return tr_frag_at<T>(a, a + G::kTrHigh);
+            };
+#pragma unroll
+            for (int k = 0; k < kTrAhead; ++k) f[k] = operand(k);
+#pragma unroll
+            for (int i = 0; i < kMma; ++i) {
+                if (i + kTrAhead < kMma) f[i + kTrAhead] = operand(i + kTrAhead);
+                acc[i % NDT] = Elem<T>::mma(f[i], bs[i / NDT], acc[i % NDT]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        sum_and_store16<T, D>(acc, scale, smem, wave, lane, dQ + head + static_cast<size_t>(q0) * D,
+                              Nq - q0);
+        return;
+    }
+
+    const int BHkv = BH / group;
+    if (id >= BHkv * nkt) return;
+    int bkv, kt_i;  // ascending key tiles: with a causal mask the first carry the most work
+    item_order(id, BHkv, nkt, causal == 0, bkv, kt_i);
+    const int k0 = kt_i * 32;
+    const int key = k0 + l32;
+    const bool key_ok = key < Nk;
+    const size_t kv_head = static_cast<size_t>(bkv) * Nk * D;  // K, V, dK, dV
+    // Query blocks [qb_begin, nqt) of each query head of the group as one sequence.
+    const int qb_begin = causal ? max(0, k0 - coff) / 32 : 0;
+    const int span = nqt - qb_begin;
+    const int n_it = group * span;
+    auto load = [&](int it, int b) {
+        const int bh = bkv * group + it / span;
+        const int r0 = (qb_begin + it % span) * 32;
+        unsigned char* set = sets + b * Cfg::kSet;
+        const size_t q_head = static_cast<size_t>(bh) * Nq * D;
+        load_tile(Q + q_head, r0, Nq, set);
+        load_tile(dO + q_head, r0, Nq, set + QT);
+        lds_dma4_async(reinterpret_cast<const float*>(LD + static_cast<size_t>(bh) * Npad + r0) + lane,
+                       set + 2 * QT);
+    };
+    frag kf[KS], vf[KS];
+    row_frags(K + kv_head + static_cast<size_t>(key) * D, key_ok, kf);
+    row_frags(V + kv_head + static_cast<size_t>(key) * D, key_ok, vf);
+    f32x16 dk[NDT];
+    f32x16 dv[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) {
+        dk[dt] = f32x16{};
+        dv[dt] = f32x16{};
+    }
+    if (wave < n_it) load(wave, 0);
+    int b = 0;
+    for (int it = wave; it < n_it; it += NW, b ^= 1) {
+        wait_loads<0>();
+        wait_lds();
+        if (it + NW < n_it) load(it + NW, b ^ 1);
+        const int q0 = (qb_begin + it % span) * 32;
+        const unsigned char* qt = sets + b * Cfg::kSet;
+        const unsigned char* ot = qt + QT;
+        const float* ld = reinterpret_cast<const float*>(qt + 2 * QT);
+        f32x16 s = f32x16{};
+        f32x16 dp = f32x16{};
+        if constexpr (neg_d_rows<D>()) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const f32x4 nd = *reinterpret_cast<const f32x4*>(&ld[32 + 8 * a + 4 * g2]);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) dp[4 * a + u] = nd[u];
+            }
+        }
+        row_products(qt, ot, kf, vf, s, dp);
+        if ((causal && k0 + 31 > q0 + coff) || k0 + 31 >= Nk) {
+            const int lim = !key_ok ? 1 << 30 : (causal ? key - coff - q0 - 4 * g2 : -1);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = (8 * (r >> 2) + (r & 3) < lim) ? -INFINITY : s[r];
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            float lv[4], dd[4];
+            if constexpr (neg_d_rows<D>()) {
+                const f32x4 x = *reinterpret_cast<const f32x4*>(&ld[8 * a + 4 * g2]);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) lv[u] = x[u];
+            } else {
+                const f32x4 x = *reinterpret_cast<const f32x4*>(&ld[2 * (8 * a + 4 * g2)]);
+                const f32x4 y = *reinterpret_cast<const f32x4*>(&ld[2 * (8 * a + 4 * g2) + 4]);
+                lv[0] = x[0], lv[1] = x[2], lv[2] = y[0], lv[3] = y[2];
+                dd[0] = x[1], dd[1] = x[3], dd[2] = y[1], dd[3] = y[3];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int r = 4 * a + u;
+                const float p = fast_exp2(fmaf(s[r], cs, -lv[u]));
+                s[r] = p;
+                if constexpr (neg_d_rows<D>())
+                    dp[r] = p * dp[r];
+                else
+                    dp[r] = p * (dp[r] - dd[u]);
+            }
+        }
+        // dV^T += dO^T P and dK^T += Q^T dS (operand i: even dO^T, odd Q^T).
+        const frag bp[2] = {pack8(s, 0), pack8(s, 1)};
+        const frag bs[2] = {pack8(dp, 0), pack8(dp, 1)};
+        constexpr int kMma = 4 * NDT;
+        frag f[kMma];
+        auto operand = [&](int i) {
+            const unsigned char* a = (i & 1 ? qt : ot) + tr_off + (i / (2 * NDT)) * G::kTrRows16 +
+                                     G::dtile_off((i >> 1) % NDT);
+            return tr_frag_at<T>(a, a + G::kTrHigh);
+        };
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) f[k] = operand(k);
+#pragma unroll
+        for (int i = 0; i < kMma; ++i) {
+            if (i + kAhead < kMma) f[i + kAhead] = operand(i + kAhead);
+            const int dt = (i >> 1) % NDT;
+            if (i & 1)
+                dk[dt] = Elem<T>::mma(f[i], bs[i / (2 * NDT)], dk[dt]);
+            else
+                dv[dt] = Elem<T>::mma(f[i], bp[i / (2 * NDT)], dv[dt]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    const size_t out = kv_head + static_cast<size_t>(k0) * D;
+    sum_and_store16<T, D>(dk, scale, smem, wave, lane, dK + out, Nk - k0);
+    sum_and_store16<T, D>(dv, 1.0f, smem, wave, lane, dV + out, Nk - k0);
+}
+
 }  // namespace dev
 
 namespace detail {
@@ -1645,6 +1994,40 @@ FlashAttentionError run_backward_two_pass(const T* Q, const T* K, const T* V, co
     return from_hip(hipGetLastError());
 }
 
+// Whether bwd16_rows_kernel beats bwd_fused_kernel, from a model of both in microseconds, fitted to
+// event times of one box (4 to 32 heads, 256 to 4096 rows, causal and not). With U the 32 x 32 blocks
+// of each kind of item in the launch:
+//  * bwd16_rows_kernel: t0 per item and CU plus x per block of U, but at least its longest item,
+//    whose blocks (all query heads of a group for a key tile) are cut over the waves, at cr each;
+//  * bwd_fused_kernel: its longest item at cb per block, or about a third of that and xf per block
+//    of U once its workgroups are all busy; grouped heads add a launch that sums their shares.
+// The first spreads better, the second moves a fourth of the tile bytes per product. Measured
+// (fused -> rows, us): see the kernel; not taken: causal 16 heads, N=2048, head_dim 64 61, 69 and 128
+// 92, 140; 32 heads, N=1024, head_dim 64 38, 52; 8 heads over 1, N=2000, head_dim 128 98, 203.
+template <int D>
+bool bwd16_rows_faster(const BwdShape& sh, bool causal) {
+    constexpr double t0 = D <= 64 ? 3.3 : 3.5;
+    constexpr double x = (D == 32 ? 0.8 : D == 64 ? 1.16 : D == 96 ? 2.5 : 3.2) * 1e-3;
+    constexpr double cr = D <= 64 ? 0.8 : 1.1;
+    constexpr double cb = D == 32 ? 0.7 : D == 64 ? 0.68 : D == 96 ? 0.92 : 1.11;
+    constexpr double xf = (D == 32 ? 0.9 : D == 64 ? 1.17 : D == 96 ? 1.4 : 1.78) * 1e-3;
+    constexpr int kWaves = dev::Bwd16RowsCfg<D>::kWaves;
+    const double cus = compute_units();
+    const double nqt = (sh.Nq + 31) / 32, nkt = (sh.Nk + 31) / 32;
+    const double frac = causal ? (2.0 * sh.Nk - sh.Nq + 32.0) / (2.0 * sh.Nk) : 1.0;
+    const double blocks = sh.BH * nqt * nkt * frac;
+    const double items = sh.BH * nqt + sh.BH / sh.group * nkt;
+    // Beyond eight items per CU the fused kernel was ahead at every shape measured, by far where the
+    // items are many and short (B=4 H=8, 387 queries, 11693 keys, head_dim 96: 349 against 1057 us).
+    if (items > 8.0 * cus) return false;
+    const double rows = 3.0 + std::max(t0 + std::max(sh.group * nqt, nkt) / kWaves * cr,
+                                       items / cus * t0 + blocks * x);
+    const double longest = std::max(nqt, nkt) * cb;
+    const double fused = 6.5 + std::max(longest, 0.35 * longest + blocks * xf) +
+                         (sh.group > 1 ? 4.0 : 0.0);
+    return 1.05 * rows < fused;
+}
+
 // Path for fp16 / bf16 at head_dim 128 and 64: delta_ld_kernel, then bwd_fused_kernel (dq and
 // dkdv in one launch).
 template <typename T, int D>
@@ -1687,6 +2070,22 @@ FlashAttentionError run_backward_fused(const T* Q, const T* K, const T* V, const
                        rows_pad, queues);
     err = from_hip(hipGetLastError());
     if (err != FlashAttentionError::SUCCESS) return err;
+
+    if constexpr (D != 256) {
+        if (bwd16_rows_faster<D>(sh, causal)) {
+            const int nkt = (sh.Nk + 31) / 32;
+            const long long items = std::max(static_cast<long long>(Npad / 32) * sh.BH,
+                                             static_cast<long long>(nkt) * (sh.BH / sh.group));
+            tok = profile_kernel<T, D>("backward_dq_dkdv");
+            launch_kernel(tok, (dev::bwd16_rows_kernel<T, D>),
+                          dim3(static_cast<unsigned>((items + 7) / 8 * 16)),
+                          dim3(64 * dev::Bwd16RowsCfg<D>::kWaves), 0, stream, q, k, v, ld, go,
+                          reinterpret_cast<uint16_t*>(dQ), reinterpret_cast<uint16_t*>(dK),
+                          reinterpret_cast<uint16_t*>(dV), sh.Nq, sh.Nk, sh.Nk - sh.Nq, sh.group,
+                          Npad, nkt, sh.BH, c, scale, causal ? 1 : 0);
+            return from_hip(hipGetLastError());
+        }
+    }
 
     StreamWorkspace share_ws(stream);
     float* part = nullptr;
