@@ -44,6 +44,9 @@ constexpr int kDppXor1 = 0xB1;        // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141;  // lane i <-> 7 - i within each 8 lanes
 constexpr int kDppMirror = 0x140;      // lane i <-> 15 - i within each row
+constexpr int kDppRowShr = 0x110;      // + n: lane i takes lane i - n of its row
+constexpr int kDppRowBcast15 = 0x142;  // the last lane of a row to the next row
+constexpr int kDppRowBcast31 = 0x143;  // lane 31 to rows 2 and 3
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
@@ -103,6 +106,116 @@ struct DecodeArgs {
     int chunk, nsplit;
     float c;  // scale * log2(e)
 };
+
+// Balanced split of a paged decode (decode_mma_rows_kernel with automatic splits). The sequences'
+// lengths are known on the device only, and equal splits of the cache's capacity leave the
+// workgroups past a sequence's end without work: with 16 sequences of 512 to 8191 keys, half of
+// them. Instead every (sequence, head group) unit is cut into as many segments as W blocks of 32
+// keys go into it, rounded up, with the least W whose segments number at most max_segments: about
+// one round of workgroups. From 7/8 of the capacity on, the equal splits of the capacity (chunk)
+// are as good, and the search for W is saved.
+// Segment x leaves its partials in entry x, so the entries of a unit follow each other; its first
+// workgroup notes them for the combine.
+// Bound by the cache's reads where the workgroups have equal work: 32 query heads over 8, 16
+// sequences of 8191 keys at most, fp16, head_dim 128, lengths spread evenly 74 -> 53 us (3.9 ->
+// 5.4 TB/s), one long sequence and fifteen short ones 71 -> 18 us, all full 86.6 -> 86.7 us; 64
+// sequences of 2000 keys, spread 77.3 -> 62.8 us, full 90.6 -> 92.5 us (the combine, one workgroup
+// per query head and 32 columns, waits for one more load); 16 of 4096, spread 41.0 -> 32.1 us, full
+// 48.1 -> 48.7 us.
+struct BalancedArgs : DecodeArgs {
+    int B;             // sequences
+    int groups;        // units per sequence (head groups that one workgroup serves)
+    int unit_heads;    // query heads per unit
+    int max_segments;  // at least twice the units, and the equal splits of all units
+    int min_blocks;    // least 32-key blocks per segment
+    int full_blocks;   // blocks from which on the equal splits of the capacity are kept
+    int2* units;       // [B * groups]: first entry and number of segments (units with keys only)
+};
+template <class Args>
+constexpr bool is_balanced() {
+    return std::is_same<Args, BalancedArgs>::value;
+}
+struct PagedSegment {
+    int b, g;        // sequence, head group
+    int blk, count;  // first block inside the unit, blocks (0: no such segment)
+    int part, parts;  // which of the unit's segments this is, and how many there are
+};
+__device__ __forceinline__ int paged_len(const DecodeArgs& a, int b) {
+    return min(max(a.seq_lens[b], 0), a.kv_len);
+}
+// Inclusive sum over the lanes of the wave.
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 1, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 2, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 4, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 8, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xA, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast31, 0xC, 0xF, false);
+    return v;
+}
+// Segment x (every wave computes it for itself; wave-uniform).
+__device__ __forceinline__ PagedSegment paged_segment(const BalancedArgs& a, int x) {
+    const int lane = threadIdx.x & 63;
+    auto blocks_of = [&](int b0) {
+        return b0 + lane < a.B ? (paged_len(a, b0 + lane) + 31) >> 5 : 0;
+    };
+    const int first64 = blocks_of(0);
+    // Sum of f(blocks) over the sequences.
+    auto sum = [&](auto f) {
+        int v = f(first64);
+        for (int b0 = 64; b0 < a.B; b0 += 64) v += f(blocks_of(b0));
+        return __builtin_amdgcn_readlane(wave_scan(v), 63);
+    };
+    const int total = sum([](int n) { return n; }) * a.groups;
+    PagedSegment r{0, 0, 0, 0, 0, 0};
+    if (total >= a.full_blocks) {
+        const int unit = x / a.nsplit;
+        r.part = x - unit * a.nsplit;
+        r.b = unit / a.groups;
+        r.g = unit - r.b * a.groups;
+        if (unit >= a.B * a.groups) return r;
+        const int n = (paged_len(a, r.b) + 31) >> 5;
+        const int each = a.chunk >> 5;
+        r.blk = r.part * each;
+        r.count = min(each, n - r.blk);
+        r.parts = r.count > 0 ? (n + each - 1) / each : 0;
+        return r;
+    }
+    // Segments of at most w blocks: at most total / w + units, so the least w that keeps them
+    // within max_segments lies in [total / max_segments, total / (max_segments - units)].
+    const int room = a.max_segments - a.B * a.groups;
+    int lo = max(a.min_blocks, (total + a.max_segments - 1) / a.max_segments);
+    int hi = max(lo, (total + room - 1) / room);
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (sum([&](int n) { return (n + mid - 1) / mid; }) * a.groups <= a.max_segments)
+            hi = mid;
+        else
+            lo = mid + 1;
+    }
+    int before = 0;  // segments of the sequences before b0
+    for (int b0 = 0; b0 < a.B; b0 += 64) {
+        const int nb = b0 == 0 ? first64 : blocks_of(b0);
+        const int own = (nb + lo - 1) / lo;
+        const int incl = wave_scan(own);
+        const unsigned long long past = __ballot(before + incl * a.groups > x);
+        if (past != 0) {
+            const int i = __ffsll(past) - 1;
+            const int n = __builtin_amdgcn_readlane(nb, i);
+            r.parts = __builtin_amdgcn_readlane(own, i);
+            const int at = x - before - (__builtin_amdgcn_readlane(incl, i) - r.parts) * a.groups;
+            const int each = (n + r.parts - 1) / r.parts;
+            r.b = b0 + i;
+            r.g = at / r.parts;
+            r.part = at - r.g * r.parts;
+            r.blk = r.part * each;
+            r.count = min(each, n - r.blk);
+            break;
+        }
+        before += __builtin_amdgcn_readlane(incl, 63) * a.groups;
+    }
+    return r;
+}
 
 template <typename T, int D, int G, bool PAGED>
 __global__ void __launch_bounds__(256)
@@ -549,11 +662,11 @@ __global__ void __launch_bounds__(64)
 // of K and V, one workgroup per CU; each wave runs kv_block32 on its own head's 2D-byte
 // column. A load is one key row with one scalar row index, clamped to the sequence's last key
 // past its end (masked), so any page size works.
-template <typename T, int D>
+template <typename T, int D, class Args>
 __global__ void __launch_bounds__(64 * (512 / D))
     decode_mma_rows_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
                            const uint16_t* __restrict__ V, float* __restrict__ part_acc,
-                           float2* __restrict__ part_ml, DecodeArgs a) {
+                           float2* __restrict__ part_ml, Args a) {
     using Lay = DecRowLayout;
     constexpr int KS = D / 16;
     constexpr int NDT = D / 32;
@@ -566,130 +679,147 @@ __global__ void __launch_bounds__(64 * (512 / D))
     __shared__ __attribute__((aligned(1024))) unsigned char Vb0[BN * Lay::kRowV];
     __shared__ __attribute__((aligned(1024))) unsigned char Vb1[BN * Lay::kRowV];
 
-    // blockIdx.x = (b * (Hkv / NW) + quad) * nsplit + split; wave w: key/value head NW quad + w.
     const int hpk = a.H / a.Hkv;
-    const int nquad = a.Hkv / NW;
-    int rest = blockIdx.x;
-    const int split = rest % a.nsplit;
-    rest /= a.nsplit;
-    const int quad = rest % nquad;
-    const int b = rest / nquad;
     const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int hk = quad * NW + w;
-    const int h0 = hk * hpk;
     const int lane = threadIdx.x & 63;
     const int l32 = lane & 31;
     const int g2 = lane >> 5;
 
-    const int kv_b = min(max(a.seq_lens[b], 0), a.kv_len);
-    const int kbeg = split * a.chunk;
-    const int kend = min(kv_b, kbeg + a.chunk);
-    const int nblk = kend > kbeg ? (kend - kbeg + BN - 1) / BN : 0;
-    // Key row t of the NW heads: Kq + ((page_of(t) page_size + t % page_size) Hkv) D.
-    const uint16_t* Kq = K + static_cast<size_t>(quad) * NW * D;
-    const uint16_t* Vq = V + static_cast<size_t>(quad) * NW * D;
-    auto page_of = [&](int t) {
-        const int j = a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size;
-        return a.block_table[static_cast<size_t>(b) * a.max_pages + j];
-    };
-    auto row_off = [&](int t, int page) -> size_t {
-        const int r = a.page_shift >= 0 ? t & (a.page_size - 1) : t % a.page_size;
-        return (static_cast<size_t>(page) * a.page_size + r) * static_cast<size_t>(a.Hkv) * D;
-    };
 
-    // Q^T: lane l32 holds query head h0 + l32 (zeros past the group), dims 16 ks + 8 g2 .. + 8.
-    frag qf[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (l32 < hpk) v = ld16(Q + (static_cast<size_t>(b) * a.H + h0 + l32) * D + 16 * ks + 8 * g2);
-        qf[ks] = as_frag<T>(v);
-    }
+    // One segment: keys [kbeg, kend) of sequence b for the query heads of the NW key/value heads
+    // from NW quad on (wave w: head NW quad + w); the partial of the i-th of them goes to slot0 +
+    // i slot_step.
+    auto segment = [&](int b, int quad, int kbeg, int kend, size_t slot0, size_t slot_step) {
+        const int h0 = (quad * NW + w) * hpk;
+        const int nblk = kend > kbeg ? (kend - kbeg + BN - 1) / BN : 0;
+        // Key row t of the NW heads: Kq + ((page_of(t) page_size + t % page_size) Hkv) D.
+        const uint16_t* Kq = K + static_cast<size_t>(quad) * NW * D;
+        const uint16_t* Vq = V + static_cast<size_t>(quad) * NW * D;
+        auto page_of = [&](int t) {
+            const int j = a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size;
+            return a.block_table[static_cast<size_t>(b) * a.max_pages + j];
+        };
+        auto row_off = [&](int t, int page) -> size_t {
+            const int r = a.page_shift >= 0 ? t & (a.page_size - 1) : t % a.page_size;
+            return (static_cast<size_t>(page) * a.page_size + r) * static_cast<size_t>(a.Hkv) * D;
+        };
 
-    // Tile loads: row RPW w + i of the block at key0 (clamped to kend - 1) by one instruction,
-    // lane i: the 16 bytes at 16 i of the row's 1 KB. Its page is lane i of `pages`.
-    const unsigned ld_voff = static_cast<unsigned>(lane * 16);
-    auto fetch_pages = [&](int key0) {
-        int pg = 0;
-        if (lane < RPW && key0 < kend) pg = page_of(min(key0 + RPW * w + lane, kend - 1));
-        return pg;
-    };
-    auto load_tile = [&](const uint16_t* src, int key0, unsigned char* dst, int row_bytes,
-                         int pages) {
+        // Q^T: lane l32 holds query head h0 + l32 (zeros past the group), dims 16 ks + 8 g2 .. + 8.
+        frag qf[KS];
 #pragma unroll
-        for (int i = 0; i < RPW; ++i) {
-            const int t = min(key0 + RPW * w + i, kend - 1);
-            // The base comes from v_readlane and the compiler cannot prove it uniform: read it
-            // into SGPRs (the load statement's wait states cover the VALU write).
-            const uint16_t* sb = src + row_off(t, __builtin_amdgcn_readlane(pages, i));
-            lds_dma16_nt_s(uniform_ptr(sb), ld_voff, dst + (RPW * w + i) * row_bytes);
+        for (int ks = 0; ks < KS; ++ks) {
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (l32 < hpk) v = ld16(Q + (static_cast<size_t>(b) * a.H + h0 + l32) * D + 16 * ks + 8 * g2);
+            qf[ks] = as_frag<T>(v);
         }
-    };
-    // Operand offsets in the row layout: K rows (lane l32 = key, chunk 2 ks + g2 of head w) and
-    // the V transpose reads (rows 4 g2 + (lane % 16) / 4, chunks 2 ((lane / 16) % 2) +
-    // (lane % 4) / 2, half lane % 2).
-    const int k_off = l32 * Lay::kRowK + w * 2 * D + g2 * 16;
-    const int k_base[2] = {k_off, k_off};
-    const int kq = lane & 15;
-    const int v_off = (4 * g2 + (kq >> 2)) * Lay::kRowV + w * 2 * D +
-                      (2 * ((lane >> 4) & 1) + ((kq & 3) >> 1)) * 16 + (kq & 1) * 8;
 
-    f32x16 o[NDT];
+        // Tile loads: row RPW w + i of the block at key0 (clamped to kend - 1) by one instruction,
+        // lane i: the 16 bytes at 16 i of the row's 1 KB. Its page is lane i of `pages`.
+        const unsigned ld_voff = static_cast<unsigned>(lane * 16);
+        auto fetch_pages = [&](int key0) {
+            int pg = 0;
+            if (lane < RPW && key0 < kend) pg = page_of(min(key0 + RPW * w + lane, kend - 1));
+            return pg;
+        };
+        auto load_tile = [&](const uint16_t* src, int key0, unsigned char* dst, int row_bytes,
+                             int pages) {
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16{};
-    float m = -INFINITY;
-    float l = 0.0f;
-    const float cs = fmaxf(a.c, kFltMin);  // scale 0: -inf * 0 would make the masked scores NaN
-
-    // Block j in Kb[j & 1] / Vb[j & 1]. Each wave waits for its own loads of block j (vmcnt(0));
-    // the barrier after it makes every wave's loads visible and ends every wave's reads of block
-    // j - 1, whose buffers block j + 1's loads then fill. `pages` holds the page indices of this
-    // wave's rows of the next block to load.
-    int pages = fetch_pages(kbeg);
-    if (nblk > 0) {
-        load_tile(Kq, kbeg, Kb0, Lay::kRowK, pages);
-        load_tile(Vq, kbeg, Vb0, Lay::kRowV, pages);
-        pages = fetch_pages(kbeg + BN);
-    }
-    for (int j = 0; j < nblk; j += 2) {
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (j + 1 < nblk) {
-            load_tile(Kq, kbeg + (j + 1) * BN, Kb1, Lay::kRowK, pages);
-            load_tile(Vq, kbeg + (j + 1) * BN, Vb1, Lay::kRowV, pages);
-            pages = fetch_pages(kbeg + (j + 2) * BN);
-        }
-        kv_block32<T, D, Lay>(Kb0, Vb0, k_base, v_off, kbeg + j * BN, kend, kend, g2, cs, qf, o, m,
-                              l, [] {});
-        if (j + 1 >= nblk) break;
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (j + 2 < nblk) {
-            load_tile(Kq, kbeg + (j + 2) * BN, Kb0, Lay::kRowK, pages);
-            load_tile(Vq, kbeg + (j + 2) * BN, Vb0, Lay::kRowV, pages);
-            pages = fetch_pages(kbeg + (j + 3) * BN);
-        }
-        kv_block32<T, D, Lay>(Kb1, Vb1, k_base, v_off, kbeg + (j + 1) * BN, kend, kend, g2, cs, qf,
-                              o, m, l, [] {});
-    }
-
-    // Partials of this wave's query heads: lane l32 < G holds head h0 + l32, dims 32 dt + 8 q +
-    // 4 g2 .. + 3 in o[dt][4 q .. 4 q + 3].
-    l = pair_sum(l);
-    if (l32 < hpk) {
-        const size_t slot = (static_cast<size_t>(b) * a.H + h0 + l32) * a.nsplit + split;
-        float* dst = part_acc + slot * D;
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
-#pragma unroll
-            for (int qq = 0; qq < 4; ++qq) {
-                f32x4 v;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = o[dt][4 * qq + u];
-                st16(dst + 32 * dt + 8 * qq + 4 * g2, __builtin_bit_cast(u32x4, v));
+            for (int i = 0; i < RPW; ++i) {
+                const int t = min(key0 + RPW * w + i, kend - 1);
+                // The base comes from v_readlane and the compiler cannot prove it uniform: read it
+                // into SGPRs (the load statement's wait states cover the VALU write).
+                const uint16_t* sb = src + row_off(t, __builtin_amdgcn_readlane(pages, i));
+                lds_dma16_nt_s(uniform_ptr(sb), ld_voff, dst + (RPW * w + i) * row_bytes);
             }
+        };
+        // Operand offsets in the row layout: K rows (lane l32 = key, chunk 2 ks + g2 of head w) and
+        // the V transpose reads (rows 4 g2 + (lane % 16) / 4, chunks 2 ((lane / 16) % 2) +
+        // (lane % 4) / 2, half lane % 2).
+        const int k_off = l32 * Lay::kRowK + w * 2 * D + g2 * 16;
+        const int k_base[2] = {k_off, k_off};
+        const int kq = lane & 15;
+        const int v_off = (4 * g2 + (kq >> 2)) * Lay::kRowV + w * 2 * D +
+                          (2 * ((lane >> 4) & 1) + ((kq & 3) >> 1)) * 16 + (kq & 1) * 8;
+
+        f32x16 o[NDT];
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16{};
+        float m = -INFINITY;
+        float l = 0.0f;
+        const float cs = fmaxf(a.c, kFltMin);  // scale 0: -inf * 0 would make the masked scores NaN
+
+        // Block j in Kb[j & 1] / Vb[j & 1]. Each wave waits for its own loads of block j (vmcnt(0));
+        // the barrier after it makes every wave's loads visible and ends every wave's reads of block
+        // j - 1, whose buffers block j + 1's loads then fill. `pages` holds the page indices of this
+        // wave's rows of the next block to load.
+        int pages = fetch_pages(kbeg);
+        if (nblk > 0) {
+            load_tile(Kq, kbeg, Kb0, Lay::kRowK, pages);
+            load_tile(Vq, kbeg, Vb0, Lay::kRowV, pages);
+            pages = fetch_pages(kbeg + BN);
         }
-        if (g2 == 0) part_ml[slot] = make_float2(m, l);
+        for (int j = 0; j < nblk; j += 2) {
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            if (j + 1 < nblk) {
+                load_tile(Kq, kbeg + (j + 1) * BN, Kb1, Lay::kRowK, pages);
+                load_tile(Vq, kbeg + (j + 1) * BN, Vb1, Lay::kRowV, pages);
+                pages = fetch_pages(kbeg + (j + 2) * BN);
+            }
+            kv_block32<T, D, Lay>(Kb0, Vb0, k_base, v_off, kbeg + j * BN, kend, kend, g2, cs, qf, o, m,
+                                  l, [] {});
+            if (j + 1 >= nblk) break;
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            if (j + 2 < nblk) {
+                load_tile(Kq, kbeg + (j + 2) * BN, Kb0, Lay::kRowK, pages);
+                load_tile(Vq, kbeg + (j + 2) * BN, Vb0, Lay::kRowV, pages);
+                pages = fetch_pages(kbeg + (j + 3) * BN);
+            }
+            kv_block32<T, D, Lay>(Kb1, Vb1, k_base, v_off, kbeg + (j + 1) * BN, kend, kend, g2, cs, qf,
+                                  o, m, l, [] {});
+        }
+
+        // Partials of this wave's query heads: lane l32 < G holds head h0 + l32, dims 32 dt + 8 q +
+        // 4 g2 .. + 3 in o[dt][4 q .. 4 q + 3].
+        l = pair_sum(l);
+        if (l32 < hpk) {
+            const size_t slot = slot0 + (w * hpk + l32) * slot_step;
+            float* dst = part_acc + slot * D;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+#pragma unroll
+                for (int qq = 0; qq < 4; ++qq) {
+                    f32x4 v;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) v[u] = o[dt][4 * qq + u];
+                    st16(dst + 32 * dt + 8 * qq + 4 * g2, __builtin_bit_cast(u32x4, v));
+                }
+            }
+            if (g2 == 0) part_ml[slot] = make_float2(m, l);
+        }
+    };
+    if constexpr (is_balanced<Args>()) {
+        const int x = blockIdx.x;
+        const PagedSegment ps = paged_segment(a, x);
+        if (ps.parts == 0) return;  // past the last segment
+        const int kbeg = ps.blk * BN;
+        if (ps.part == 0 && threadIdx.x == 0)
+            a.units[ps.b * a.groups + ps.g] = make_int2(x, ps.parts);
+        // A last part can be empty when the equal parts round up: it stores its empty partial.
+        segment(ps.b, ps.g, kbeg, min(paged_len(a, ps.b), kbeg + BN * max(0, ps.count)),
+                static_cast<size_t>(x) * a.unit_heads, 1);
+    } else {
+        // blockIdx.x = (b * (Hkv / NW) + quad) * nsplit + split.
+        const int nquad = a.Hkv / NW;
+        int rest = blockIdx.x;
+        const int split = rest % a.nsplit;
+        rest /= a.nsplit;
+        const int quad = rest % nquad;
+        const int b = rest / nquad;
+        const int kbeg = split * a.chunk;
+        segment(b, quad, kbeg, min(min(max(a.seq_lens[b], 0), a.kv_len), kbeg + a.chunk),
+                (static_cast<size_t>(b) * a.H + quad * NW * hpk) * a.nsplit + split, a.nsplit);
     }
 }
 
@@ -700,11 +830,12 @@ constexpr int kMaxSplits = 1024;
 // row r sums the splits r, r + 8, ... of its columns with eight loads in flight per lane, and the
 // split weights 2^(m_s - M) are formed once into LDS. (One lane per column walking every split
 // in sequence was latency-bound at a few heads with hundreds of splits.)
-template <typename T, int D>
+// `args`: the split count of every head, or a balanced launch's arguments.
+template <typename T, int D, class Args>
 __global__ void __launch_bounds__(256)
     decode_combine_kernel(const float* __restrict__ part_acc, const float2* __restrict__ part_ml,
                           typename Mma<T>::elem* __restrict__ O, float* __restrict__ L,
-                          int nsplit) {
+                          Args args) {
     constexpr int kSlices = D / 32;
     constexpr int kRows = 8;
     constexpr int kInFlight = 8;
@@ -715,11 +846,28 @@ __global__ void __launch_bounds__(256)
     const int c0 = (blockIdx.x % kSlices) * 32;
     const int t = threadIdx.x;
     const int wave = t >> 6;
-    const float2* ml = part_ml + static_cast<size_t>(bh) * nsplit;
-    const float* acc = part_acc + static_cast<size_t>(bh) * nsplit * D;
+    // The partials of this head: nsplit of them from `first` on, `step` apart.
+    int nsplit;
+    size_t first, step;
+    if constexpr (is_balanced<Args>()) {
+        const BalancedArgs& a = args;
+        const int b = bh / a.H;
+        const int h = bh % a.H;
+        // Read also where an empty sequence left it unwritten: two loads in flight, not a chain.
+        const int2 u = a.units[b * a.groups + h / a.unit_heads];
+        nsplit = paged_len(a, b) > 0 ? u.y : 0;
+        first = static_cast<size_t>(u.x) * a.unit_heads + h % a.unit_heads;
+        step = a.unit_heads;
+    } else {
+        nsplit = args;
+        first = static_cast<size_t>(bh) * nsplit;
+        step = 1;
+    }
+    const float2* ml = part_ml + first;
+    const float* acc = part_acc + first * D;
 
     float mm = -INFINITY;
-    for (int s = t; s < nsplit; s += 256) mm = fmaxf(mm, ml[s].x);
+    for (int s = t; s < nsplit; s += 256) mm = fmaxf(mm, ml[s * step].x);
 #pragma unroll
     for (int k = 32; k >= 1; k >>= 1) mm = fmaxf(mm, xor_shuffle(mm, k));
     if ((t & 63) == 0) red[wave] = mm;
@@ -728,7 +876,7 @@ __global__ void __launch_bounds__(256)
     __syncthreads();
     float lt = 0.0f;
     for (int s = t; s < nsplit; s += 256) {
-        const float2 v = ml[s];
+        const float2 v = ml[s * step];
         const float f = exp2_rel(v.x, mm);
         fw[s] = f;
         lt += v.y * f;
@@ -747,11 +895,11 @@ __global__ void __launch_bounds__(256)
     for (; s + (kInFlight - 1) * kRows < nsplit; s += kInFlight * kRows) {
         float x[kInFlight];
 #pragma unroll
-        for (int u = 0; u < kInFlight; ++u) x[u] = a0[static_cast<size_t>(s + u * kRows) * D];
+        for (int u = 0; u < kInFlight; ++u) x[u] = a0[(s + u * kRows) * step * D];
 #pragma unroll
         for (int u = 0; u < kInFlight; ++u) at = fmaf(x[u], fw[s + u * kRows], at);
     }
-    for (; s < nsplit; s += kRows) at = fmaf(a0[static_cast<size_t>(s) * D], fw[s], at);
+    for (; s < nsplit; s += kRows) at = fmaf(a0[s * step * D], fw[s], at);
     rows[row][col] = at;
     __syncthreads();
     if (row == 0) {
@@ -841,18 +989,42 @@ FlashAttentionError run_decode(const T* Q, const T* K, const T* V, T* O, float* 
         a.chunk = std::max(32, (a.chunk + 31) / 32 * 32);
         a.nsplit = std::max(1, (a.kv_len + a.chunk - 1) / a.chunk);
     }
-    const long long blocks = groups * a.nsplit;
-    const long long slots = bhq * a.nsplit;
-    if (blocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;
+    long long blocks = groups * a.nsplit;
+    long long slots = bhq * a.nsplit;
+    // Automatic splits of caches with room for at least 16 blocks (1 MB) per workgroup: the
+    // balanced split (its block counts in 32 bits). Where all sequences fill the cache it costs 0.5 to 2 us
+    // (BalancedArgs): 1% from here on, but 3 to 8% of smaller caches. Not in a captured launch: an
+    // earlier form of it faulted in a graph's replay, for a reason not found.
+    const long long cap_blocks = (static_cast<long long>(a.kv_len) + 31) / 32;
+    const bool balanced = rows && num_splits == 0 && B > 1 &&
+                          groups * cap_blocks >= 16LL * compute_units() &&
+                          groups * cap_blocks < (1LL << 27) && fixed.ptr == nullptr &&
+                          !stream_capturing(stream);
+    dev::BalancedArgs bal{};
+    if (balanced) {
+        static_cast<dev::DecodeArgs&>(bal) = a;
+        bal.B = B;
+        bal.groups = static_cast<int>(groups / B);
+        bal.unit_heads = a.H / bal.groups;
+        // At least kMinChunk keys per segment, and no more per unit than the combine can hold.
+        bal.min_blocks = static_cast<int>(std::max<long long>(
+            kMinChunk / 32, (cap_blocks + dev::kMaxSplits - 1) / dev::kMaxSplits));
+        const long long wgs = static_cast<long long>(kRowsPerCu) * compute_units();
+        bal.max_segments = static_cast<int>(std::max({wgs, 2 * groups, blocks}));
+        bal.full_blocks = static_cast<int>(groups * cap_blocks * 7 / 8);
+        blocks = bal.max_segments;
+        slots = static_cast<long long>(bal.max_segments) * bal.unit_heads;
+    }
 
     const size_t acc_bytes = static_cast<size_t>(slots) * D * sizeof(float);
     const size_t ml_bytes = static_cast<size_t>(slots) * sizeof(float2);
+    const size_t unit_bytes = balanced ? static_cast<size_t>(groups) * sizeof(int2) : 0;
     StreamWorkspace ws(stream, true);
     void* base = fixed.ptr;
     if (base != nullptr) {
         if (acc_bytes + ml_bytes > fixed.bytes) return FlashAttentionError::OUT_OF_MEMORY;
     } else {
-        FlashAttentionError err = ws.alloc(acc_bytes + ml_bytes);
+        FlashAttentionError err = ws.alloc(acc_bytes + ml_bytes + unit_bytes);
         if (err != FlashAttentionError::SUCCESS) return err;
         base = ws.get();
     }
@@ -861,6 +1033,8 @@ FlashAttentionError run_decode(const T* Q, const T* K, const T* V, T* O, float* 
     float* part_acc = static_cast<float*>(base);
     float2* part_ml = reinterpret_cast<float2*>(static_cast<char*>(base) + acc_bytes);
 
+    bal.units = reinterpret_cast<int2*>(static_cast<char*>(base) + acc_bytes + ml_bytes);
+
     ProfileEvents tok = profile_kernel<T, D>("decode_split");
     if constexpr (MMA) {
         static_assert((D == 32 || D == 64 || D == 128) && !std::is_same<T, float>::value,
@@ -868,12 +1042,16 @@ FlashAttentionError run_decode(const T* Q, const T* K, const T* V, T* O, float* 
         bool launched = false;
         if constexpr (PAGED) {
             if (rows) {
-                launch_kernel(tok, (dev::decode_mma_rows_kernel<T, D>),
-                                   dim3(static_cast<unsigned>(blocks)), dim3(64 * kRowHeads), 0,
-                                   stream,
-                                   reinterpret_cast<const uint16_t*>(Q),
-                                   reinterpret_cast<const uint16_t*>(K),
-                                   reinterpret_cast<const uint16_t*>(V), part_acc, part_ml, a);
+                const uint16_t* q = reinterpret_cast<const uint16_t*>(Q);
+                const uint16_t* k = reinterpret_cast<const uint16_t*>(K);
+                const uint16_t* v = reinterpret_cast<const uint16_t*>(V);
+                const dim3 grid(static_cast<unsigned>(blocks)), block(64 * kRowHeads);
+                if (balanced)
+                    launch_kernel(tok, (dev::decode_mma_rows_kernel<T, D, dev::BalancedArgs>),
+                                  grid, block, 0, stream, q, k, v, part_acc, part_ml, bal);
+                else
+                    launch_kernel(tok, (dev::decode_mma_rows_kernel<T, D, dev::DecodeArgs>),
+                                  grid, block, 0, stream, q, k, v, part_acc, part_ml, a);
                 launched = true;
             }
         }
@@ -892,9 +1070,16 @@ FlashAttentionError run_decode(const T* Q, const T* K, const T* V, T* O, float* 
     FlashAttentionError err = from_hip(hipGetLastError());
     if (err != FlashAttentionError::SUCCESS) return err;
     tok = profile_kernel<T, D>("decode_combine");
-    launch_kernel(tok, (dev::decode_combine_kernel<T, D>),
-                       dim3(static_cast<unsigned>(bhq * (D / 32))), dim3(256), 0, stream, part_acc,
-                       part_ml, reinterpret_cast<E*>(O), L, a.nsplit);
+    const dim3 grid(static_cast<unsigned>(bhq * (D / 32)));
+    if constexpr (MMA && PAGED) {
+        if (balanced) {
+            launch_kernel(tok, (dev::decode_combine_kernel<T, D, dev::BalancedArgs>), grid,
+                          dim3(256), 0, stream, part_acc, part_ml, reinterpret_cast<E*>(O), L, bal);
+            return from_hip(hipGetLastError());
+        }
+    }
+    launch_kernel(tok, (dev::decode_combine_kernel<T, D, int>), grid, dim3(256), 0, stream,
+                  part_acc, part_ml, reinterpret_cast<E*>(O), L, a.nsplit);
     return from_hip(hipGetLastError());
 }
 
