@@ -1031,7 +1031,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
 // ------------------------------------------------------------------------------------------
 // fp16 / bf16 kernel for head_dim 64 and 32, four waves per SIMD
 // ------------------------------------------------------------------------------------------
-// fwd16_d64_kernel's tiles, operand layouts and arithmetic without its cross-block pipeline:
+// fwd16_d64_kernel's block sizes and arithmetic (tiles: SeqTileGroups) without its cross-block pipeline:
 // each wave forms a block's scores, applies the block's max, forms the exponentials and runs the
 // P V MFMAs in sequence, with one score set. That fits 128 registers, so 16 waves share a CU
 // (four workgroups of four waves, or two of eight, each with 36 KB of tiles) and the SIMD
@@ -1053,7 +1053,7 @@ __global__ void __launch_bounds__(64 * NW, 16 / NW)
     constexpr int BM = 32 * NW;  // query rows per workgroup
     constexpr int BN = 64;
     constexpr int kParts = 8 / NW;         // load instructions per wave per 64-row tile
-    using Lay = TileGroups<D>;
+    using Lay = SeqTileGroups<D>;
     constexpr int GRP = Lay::kBytes;       // bytes per 8-row group
     constexpr int TILE = (BN / 8) * GRP;   // bytes per 64-row tile
     using frag = typename Elem<T>::frag;
@@ -1087,7 +1087,7 @@ __global__ void __launch_bounds__(64 * NW, 16 / NW)
     const int kv_end = causal ? min(Nk, (qb + 1) * BM + coff) : Nk;
     const int nkb = (kv_end + BN - 1) / BN;
 
-    // Tile loads, operand offsets and masking exactly as in fwd16_d64_kernel.
+    // Tile loads, operand offsets and masking as in fwd16_d64_kernel, on SeqTileGroups.
     const int ld_row = Lay::ld_row(lane);
     const int ld_col = Lay::ld_col(lane);
     const unsigned ld_voff = static_cast<unsigned>(((8 * wave + ld_row) * D + ld_col) * 2);
