@@ -956,7 +956,8 @@ constexpr int kMinChunk = 128;
 // in flight (16 x 8 key/value heads x 32768 keys: 130 -> 89 us; head_dim 64: 156 -> 161 us).
 constexpr int mma_per_cu(int D) { return D == 32 ? 8 : 4; }
 constexpr int kRowsPerCu = 1;
-// Longest cache that an automatic grouped-query decode gives to the forward (run_decode_grouped).
+// Longest cache that an automatic grouped-query decode gives to the few-rows forward kernel
+// (run_decode_grouped).
 constexpr int kShortCache = 1024;
 
 // MMA: the matrix-core kernels, splits of whole 32-key blocks: decode_mma_rows_kernel (paged,
@@ -1098,16 +1099,18 @@ FlashAttentionError run_decode_grouped(const T* Q, const T* K, const T* V, T* O,
         // 64 and 32) whose per-lane byte offset within a group, (rows - 1) Hkv D 2 + 256, fits
         // 32 bits.
         constexpr int kGroupRows = dev::TileGroups<D>::kRows;
-        // Short caches: the forward of one query per head packs the query heads of a key/value
-        // head into one tile and spreads its keys over the waves of one workgroup: one launch and
-        // no partials. Per call, us, 32 heads over 8: head_dim 128, 1000 keys, B = 1
-        // 11.1 -> 8.7, B = 16 17.1 -> 13.2, B = 64 50.0 -> 41.4; 512 keys, B = 1 9.9 -> 7.2;
-        // head_dim 64, 512 keys, B = 64 17.6 -> 12.6. From 2000 keys on the split kernels are
-        // level or faster (B = 64, head_dim 128: 87.2 against 93.4).
-        if (!PAGED && num_splits == 0 && fx.ptr == nullptr && hpk >= 2 && hpk <= 32 && a.kv_len <= kShortCache &&
+        // Short caches: the few-rows forward kernel packs the query heads of a key/value head into
+        // one tile and spreads its keys over the waves of one workgroup: one launch and no
+        // partials. Per call, us, 32 heads over 8 (split kernels -> this): head_dim 128, 1000
+        // keys, B = 1 11.1 -> 8.7, B = 16 17.1 -> 13.2, B = 64 50.0 -> 41.4; 512 keys, B = 1
+        // 9.9 -> 7.2; 33 keys, B = 64 15.6 -> 9.5 (the general forward kernel, which the
+        // forward's own rule picks there: 39.9); head_dim 64, 512 keys, B = 64 17.6 -> 12.6. From
+        // 2000 keys on the split kernels are level or faster (B = 64, head_dim 128: 87.2 against
+        // 93.4).
+        if (!PAGED && num_splits == 0 && fx.ptr == nullptr && hpk >= 2 && hpk <= 32 &&
+            a.kv_len <= kShortCache &&
             static_cast<long long>(B) * a.Hkv <= 2LL * compute_units())
-            return launch_forward_ext<T>(Q, K, V, O, L, B, a.H, a.Hkv, 1, a.kv_len, D,
-                                         scale, false, stream);
+            return launch_decode_rows<T>(Q, K, V, O, L, B, a.H, a.Hkv, a.kv_len, D, scale, stream);
         if (hpk >= 2 && hpk <= 32 &&
             (!PAGED || a.Hkv % (512 / D) == 0 ||
              (a.page_size % kGroupRows == 0 && a.Hkv <= (1 << 20))))

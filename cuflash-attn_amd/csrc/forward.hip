@@ -1254,6 +1254,7 @@ struct FwdSplit {
     float2* ml;   // [nsplit, rows]: m in log2 units, l
     int chunk;    // keys per split, a multiple of the 32-key blocks
     int nsplit;
+    bool zero_rows;  // one split only: a row whose scores are all -inf is O = 0 (a decode), not NaN
 };
 
 // The workgroup's place in a split launch: key/value head, row block, split.
@@ -1568,7 +1569,9 @@ __global__ void __launch_bounds__(64 * fwd_rows_waves<D>(), D <= 64 ? 2 : 1)
             st16(sp.acc + slot * D + cc + 4, __builtin_bit_cast(u32x4, a1));
             if (cc == 0) sp.ml[slot] = make_float2(MM, lt);
         } else {
-            const float inv = 1.0f / lt;
+            const bool zero = sp.zero_rows && lt == 0.0f;
+            const float inv = zero ? 0.0f : 1.0f / lt;
+            if (zero) a0 = a1 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             u32x4 w;
             w[0] = Elem<T>::pack2(a0[0] * inv, a0[1] * inv);
             w[1] = Elem<T>::pack2(a0[2] * inv, a0[3] * inv);
@@ -2009,14 +2012,14 @@ int forward_rows_chunks(const FwdShape& sh, bool causal) {
 // One workgroup per (32 rows of a key/value head's query heads, chunk of keys), and a merge kernel
 // when there are several chunks. The partials need a workspace: a launch that cannot have one,
 // and a captured one (a graph would hold an allocation of tens of MiB where the forward had none),
-// walks all keys in one chunk.
+// walks all keys in one chunk. zero_rows: see FwdSplit (with one chunk).
 template <typename T, int D>
 FlashAttentionError run_forward16_rows(const T* Q, const T* K, const T* V, T* O, float* L,
                                        const FwdShape& sh, int chunks, float scale, bool causal,
-                                       hipStream_t stream) {
+                                       hipStream_t stream, bool zero_rows = false) {
     const long long rows = static_cast<long long>(sh.BH) * sh.Nq;
     const long long nqb = (static_cast<long long>(sh.group) * sh.Nq + 31) / 32;
-    dev::FwdSplit sp{nullptr, nullptr, sh.Nk, 1};
+    dev::FwdSplit sp{nullptr, nullptr, sh.Nk, 1, zero_rows};
     StreamWorkspace ws(stream, true);
     if (chunks > 1) {
         const int chunk = ((sh.Nk + chunks - 1) / chunks + 31) / 32 * 32;
@@ -2256,6 +2259,27 @@ FlashAttentionError launch_forward_ext(const T* Q, const T* K, const T* V, T* O,
     const FwdShape sh{static_cast<int>(bh), q_len, kv_len, num_heads / num_kv_heads};
     return run_forward<T>(Q, K, V, O, L, sh, head_dim, true, scale, causal, stream);
 }
+
+template <typename T>
+FlashAttentionError launch_decode_rows(const T* Q, const T* K, const T* V, T* O, float* L,
+                                       int batch_size, int num_heads, int num_kv_heads,
+                                       int kv_len, int head_dim, float scale,
+                                       hipStream_t stream) {
+    const FwdShape sh{batch_size * num_heads, 1, kv_len, num_heads / num_kv_heads};
+    switch (head_dim) {
+        case 32: return run_forward16_rows<T, 32>(Q, K, V, O, L, sh, 1, scale, false, stream, true);
+        case 64: return run_forward16_rows<T, 64>(Q, K, V, O, L, sh, 1, scale, false, stream, true);
+        case 128:
+            return run_forward16_rows<T, 128>(Q, K, V, O, L, sh, 1, scale, false, stream, true);
+    }
+    return FlashAttentionError::UNSUPPORTED_HEAD_DIM;
+}
+template FlashAttentionError launch_decode_rows<__half>(const __half*, const __half*,
+                                                        const __half*, __half*, float*, int, int,
+                                                        int, int, int, float, hipStream_t);
+template FlashAttentionError launch_decode_rows<__hip_bfloat16>(
+    const __hip_bfloat16*, const __hip_bfloat16*, const __hip_bfloat16*, __hip_bfloat16*, float*,
+    int, int, int, int, int, float, hipStream_t);
 
 #define CUFLASH_FORWARD_TYPE(T)                                                                 \
     template FlashAttentionError launch_forward<T>(const T*, const T*, const T*, T*, float*,    \

@@ -57,6 +57,15 @@ FlashAttentionError launch_decode_gqa(const T* Q, const T* K, const T* V, T* O, 
                                       int kv_len, int head_dim, float scale, int num_splits,
                                       hipStream_t stream);
 
+// The same for a short cache with 2 to 32 query heads per key/value head (fp16 / bf16,
+// batch_size * num_heads within 32 bits): one launch of the few-rows forward kernel, no workspace.
+// As in every decode, a query whose scores are all -inf has O = 0 and L = -inf.
+template <typename T>
+FlashAttentionError launch_decode_rows(const T* Q, const T* K, const T* V, T* O, float* L,
+                                       int batch_size, int num_heads, int num_kv_heads,
+                                       int kv_len, int head_dim, float scale,
+                                       hipStream_t stream);
+
 // Decode over a paged cache K_cache, V_cache [num_pages, page_size, num_kv_heads, D] with
 // block_table [B, max_pages_per_seq] and seq_lens [B].
 template <typename T>

@@ -269,3 +269,30 @@ def test_decode_gqa_matches_mha_on_repeated_heads(torch_gpu):
     torch.cuda.synchronize()
     assert float((o1.float() - o2.float()).abs().max()) <= 1e-3
     assert float((l1 - l2).abs().max()) <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("kv_len", [1, 500, 1500])
+def test_decode_gqa_of_scores_that_are_all_minus_infinity(torch_gpu, dtype, d, kv_len):
+    """A query whose scores are all -inf (its cache masked by infinities or by the type's lowest
+    value) has no weight: every decode returns O = 0 and L = -inf for it, on one launch (short
+    caches) as on splits and partials. The other sequence of the batch is an ordinary one."""
+    torch = torch_gpu
+    q = synth.round_to(np.abs(synth.normal(61, (2, 8, 1, d))) + 1.0, dtype)
+    k, v = (synth.round_to(synth.normal(s, (2, 2, kv_len, d)), dtype) for s in (62, 63))
+    scale = 4.0 * d ** -0.5
+    o_ref, l_ref = oracle.forward(q, _expand_heads(k, 4), _expand_heads(v, 4), scale, False)
+    tq, tk, tv = (synth.to_torch(x, dtype) for x in (q, k, v))
+    lowest = torch.finfo(tk.dtype).min if dtype == "bfloat16" else float("-inf")
+    for mask in (float("-inf"), lowest):
+        tk[0] = mask
+        for splits in (0, 3):
+            print(f"[-inf scores] {dtype} d={d} kv_len={kv_len} splits={splits}", flush=True)
+            o, lse = cuflash_attn.flash_attention_decode(tq, tk, tv, scale=scale,
+                                                         num_splits=splits)
+            torch.cuda.synchronize()
+            assert not o[0].any() and bool(torch.isneginf(lse[0]).all()), (mask, splits)
+            check(dtype, synth.to_numpy(o[1:]), o_ref[1:], "O")
+            check(dtype, synth.to_numpy(lse[1:]), l_ref[1:], "L")
