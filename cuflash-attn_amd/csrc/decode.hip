@@ -992,6 +992,7 @@ FlashAttentionError run_decode(const T* Q, const T* K, const T* V, T* O, float* 
     }
     long long blocks = groups * a.nsplit;
     long long slots = bhq * a.nsplit;
+    if (blocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;  // the grid's limit
     // Automatic splits of caches with room for at least 16 blocks (1 MB) per workgroup: the
     // balanced split (its block counts in 32 bits). Where all sequences fill the cache it costs 0.5 to 2 us
     // (BalancedArgs): 1% from here on, but 3 to 8% of smaller caches. Not in a captured launch: an

@@ -194,6 +194,22 @@ def test_decode_paged_validation(lib):
 
 
 @pytest.mark.parametrize("sfx", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("kind", ["decode", "decode_gqa", "decode_paged"])
+def test_decode_grid_beyond_32_bits_is_refused(lib, sfx, kind):
+    """Heads and splits that are valid by themselves but whose product exceeds a 32-bit grid are
+    refused before a workspace is asked for."""
+    heads, splits = 1 << 22, 1024
+    fn = lib.fn(kind, sfx)
+    if kind == "decode":
+        got = fn(*[P] * 5, heads, 1, 16 * splits, 32, 1.0, splits, None)
+    elif kind == "decode_gqa":
+        got = fn(*[P] * 5, heads, 2, 1, 32 * splits, 32, 1.0, splits, None)
+    else:
+        got = fn(*[P] * 7, heads, 32, 16, 16, 2 * splits, 32, 1.0, splits, None)
+    assert got == cuflash_attn.INVALID_DIMENSION
+
+
+@pytest.mark.parametrize("sfx", ["f32", "f16", "bf16"])
 def test_ext_validation(lib, sfx):
     """Extended forward / backward: the forward checks in order (null pointers, dimensions
     including num_kv_heads and both lengths, head_dim in {32, 64, 96, 128, 256}, scale), then
