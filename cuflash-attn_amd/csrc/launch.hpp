@@ -134,7 +134,8 @@ bool stream_cached_buffer(hipStream_t stream, size_t bytes, void** out,
 // workspace instead.
 FlashAttentionError release_stream_buffers();
 
-// Whether `stream` is being captured into a graph (false if that cannot be determined).
+// Whether `stream` is being captured into a graph. True if that cannot be determined: what must
+// stay out of a graph (the cached buffers, the balanced paged decode) then stays out of the call.
 bool stream_capturing(hipStream_t stream);
 
 // Stream-ordered device workspace, the counterpart of the reference's AsyncFloatBuffer

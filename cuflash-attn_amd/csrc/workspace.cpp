@@ -78,7 +78,7 @@ bool stream_capturing(hipStream_t stream) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        return true;  // unknown: the callers' capture paths are right for an eager call as well
     }
     return status != hipStreamCaptureStatusNone;
 }
