@@ -20,6 +20,7 @@
 #include "common.hpp"
 #include "kv_block.hpp"
 #include "launch.hpp"
+#include "paged_split.hpp"
 #include "profile.hpp"
 #include "softmax.hpp"
 #include "tile_groups.hpp"
@@ -91,131 +92,35 @@ __device__ __forceinline__ float exp2_rel(float x, float m) {
     return x == -INFINITY ? 0.0f : fast_exp2(x - m);
 }
 
-// Where the keys come from. Contiguous: K, V [B, Hkv, kv_len, D]. Paged: K, V
-// [num_pages, page_size, Hkv, D] with block_table [B, max_pages] naming the page of each
-// page_size keys of a sequence and seq_lens [B] its length (clamped to [0, kv_len], kv_len =
-// max_pages * page_size). A workgroup serves G query heads that share one key/value head:
-// query head h reads key/value head h / (H / Hkv).
-struct DecodeArgs {
-    const int* block_table;
-    const int* seq_lens;
-    int H, Hkv;
-    int kv_len;
-    int page_size, max_pages;
-    int page_shift;  // log2(page_size) when it is a power of two, else -1
-    int chunk, nsplit;
-    float c;  // scale * log2(e)
-};
-
-// Balanced split of a paged decode (decode_mma_rows_kernel with automatic splits). The sequences'
-// lengths are known on the device only, and equal splits of the cache's capacity leave the
-// workgroups past a sequence's end without work: with 16 sequences of 512 to 8191 keys, half of
-// them. Instead every (sequence, head group) unit is cut into as many segments as W blocks of 32
-// keys go into it, rounded up, with the least W whose segments number at most max_segments: about
-// one round of workgroups. From 7/8 of the capacity on, the equal splits of the capacity (chunk)
-// are as good, and the search for W is saved.
-// Segment x leaves its partials in entry x, so the entries of a unit follow each other; its first
-// workgroup notes them for the combine.
-// Bound by the cache's reads where the workgroups have equal work: 32 query heads over 8, 16
-// sequences of 8191 keys at most, fp16, head_dim 128, lengths spread evenly 74 -> 53 us (3.9 ->
-// 5.4 TB/s), one long sequence and fifteen short ones 71 -> 18 us, all full 86.6 -> 86.7 us; 64
-// sequences of 2000 keys, spread 77.3 -> 62.8 us, full 90.6 -> 92.5 us (the combine, one workgroup
-// per query head and 32 columns, waits for one more load); 16 of 4096, spread 41.0 -> 32.1 us, full
-// 48.1 -> 48.7 us.
-struct BalancedArgs : DecodeArgs {
-    int B;             // sequences
-    int groups;        // units per sequence (head groups that one workgroup serves)
-    int unit_heads;    // query heads per unit
-    int max_segments;  // at least twice the units, and the equal splits of all units
-    int min_blocks;    // least 32-key blocks per segment
-    int full_blocks;   // blocks from which on the equal splits of the capacity are kept
-    int2* units;       // [B * groups]: first entry and number of segments (units with keys only)
-};
-template <class Args>
-constexpr bool is_balanced() {
-    return std::is_same<Args, BalancedArgs>::value;
-}
-struct PagedSegment {
-    int b, g;        // sequence, head group
-    int blk, count;  // first block inside the unit, blocks (0: no such segment)
-    int part, parts;  // which of the unit's segments this is, and how many there are
-};
-__device__ __forceinline__ int paged_len(const DecodeArgs& a, int b) {
-    return min(max(a.seq_lens[b], 0), a.kv_len);
-}
-// Inclusive sum over the lanes of the wave.
-__device__ __forceinline__ int wave_scan(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 1, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 2, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 4, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 8, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xA, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast31, 0xC, 0xF, false);
-    return v;
-}
-// Segment x (every wave computes it for itself; wave-uniform).
-__device__ __forceinline__ PagedSegment paged_segment(const BalancedArgs& a, int x) {
-    const int lane = threadIdx.x & 63;
-    auto blocks_of = [&](int b0) {
-        return b0 + lane < a.B ? (paged_len(a, b0 + lane) + 31) >> 5 : 0;
-    };
-    const int first64 = blocks_of(0);
-    // Sum of f(blocks) over the sequences.
-    auto sum = [&](auto f) {
-        int v = f(first64);
-        for (int b0 = 64; b0 < a.B; b0 += 64) v += f(blocks_of(b0));
-        return __builtin_amdgcn_readlane(wave_scan(v), 63);
-    };
-    const int total = sum([](int n) { return n; }) * a.groups;
-    PagedSegment r{0, 0, 0, 0, 0, 0};
-    if (total >= a.full_blocks) {
-        const int unit = x / a.nsplit;
-        r.part = x - unit * a.nsplit;
-        r.b = unit / a.groups;
-        r.g = unit - r.b * a.groups;
-        if (unit >= a.B * a.groups) return r;
-        const int n = (paged_len(a, r.b) + 31) >> 5;
-        const int each = a.chunk >> 5;
-        r.blk = r.part * each;
-        r.count = min(each, n - r.blk);
-        r.parts = r.count > 0 ? (n + each - 1) / each : 0;
-        return r;
+// The 64 lanes of a wave for paged_segment (paged_split.hpp); results are wave-uniform.
+struct GpuWave {
+    using Int = int;
+    template <class F>
+    __device__ static Int each(F f) {
+        return f(static_cast<int>(threadIdx.x & 63));
     }
-    // Segments of at most w blocks: at most total / w + units, so the least w that keeps them
-    // within max_segments lies in [total / max_segments, total / (max_segments - units)].
-    const int room = a.max_segments - a.B * a.groups;
-    int lo = max(a.min_blocks, (total + a.max_segments - 1) / a.max_segments);
-    int hi = max(lo, (total + room - 1) / room);
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (sum([&](int n) { return (n + mid - 1) / mid; }) * a.groups <= a.max_segments)
-            hi = mid;
-        else
-            lo = mid + 1;
+    template <class F>
+    __device__ static Int map(Int v, F f) {
+        return f(v);
     }
-    int before = 0;  // segments of the sequences before b0
-    for (int b0 = 0; b0 < a.B; b0 += 64) {
-        const int nb = b0 == 0 ? first64 : blocks_of(b0);
-        const int own = (nb + lo - 1) / lo;
-        const int incl = wave_scan(own);
-        const unsigned long long past = __ballot(before + incl * a.groups > x);
-        if (past != 0) {
-            const int i = __ffsll(past) - 1;
-            const int n = __builtin_amdgcn_readlane(nb, i);
-            r.parts = __builtin_amdgcn_readlane(own, i);
-            const int at = x - before - (__builtin_amdgcn_readlane(incl, i) - r.parts) * a.groups;
-            const int each = (n + r.parts - 1) / r.parts;
-            r.b = b0 + i;
-            r.g = at / r.parts;
-            r.part = at - r.g * r.parts;
-            r.blk = r.part * each;
-            r.count = min(each, n - r.blk);
-            break;
-        }
-        before += __builtin_amdgcn_readlane(incl, 63) * a.groups;
+    __device__ static Int add(Int a, Int b) { return a + b; }
+    // Inclusive sum over the lanes.
+    __device__ static Int scan(Int v) {
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 1, 0xF, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 2, 0xF, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 4, 0xF, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr + 8, 0xF, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xA, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast31, 0xC, 0xF, false);
+        return v;
     }
-    return r;
-}
+    __device__ static int lane(Int v, int i) { return __builtin_amdgcn_readlane(v, i); }
+    // The first lane where f is not 0, or -1.
+    template <class F>
+    __device__ static int first(Int v, F f) {
+        return __ffsll(static_cast<unsigned long long>(__ballot(f(v)))) - 1;
+    }
+};
 
 template <typename T, int D, int G, bool PAGED>
 __global__ void __launch_bounds__(256)
@@ -801,14 +706,11 @@ __global__ void __launch_bounds__(64 * (512 / D))
     };
     if constexpr (is_balanced<Args>()) {
         const int x = blockIdx.x;
-        const PagedSegment ps = paged_segment(a, x);
+        const PagedSegment ps = paged_segment<GpuWave>(a, x);
         if (ps.parts == 0) return;  // past the last segment
-        const int kbeg = ps.blk * BN;
         if (ps.part == 0 && threadIdx.x == 0)
             a.units[ps.b * a.groups + ps.g] = make_int2(x, ps.parts);
-        // A last part can be empty when the equal parts round up: it stores its empty partial.
-        segment(ps.b, ps.g, kbeg, min(paged_len(a, ps.b), kbeg + BN * max(0, ps.count)),
-                static_cast<size_t>(x) * a.unit_heads, 1);
+        segment(ps.b, ps.g, ps.kbeg, ps.kend, static_cast<size_t>(x) * a.unit_heads, 1);
     } else {
         // blockIdx.x = (b * (Hkv / NW) + quad) * nsplit + split.
         const int nquad = a.Hkv / NW;
@@ -822,9 +724,6 @@ __global__ void __launch_bounds__(64 * (512 / D))
                 (static_cast<size_t>(b) * a.H + quad * NW * hpk) * a.nsplit + split, a.nsplit);
     }
 }
-
-// Upper bound of the split count (choose_splits).
-constexpr int kMaxSplits = 1024;
 
 // One workgroup per (batch*head, 32-column slice of D): its 256 lanes are 8 rows of 32 columns,
 // row r sums the splits r, r + 8, ... of its columns with eight loads in flight per lane, and the
@@ -854,9 +753,10 @@ __global__ void __launch_bounds__(256)
         const int b = bh / a.H;
         const int h = bh % a.H;
         // Read also where an empty sequence left it unwritten: two loads in flight, not a chain.
-        const int2 u = a.units[b * a.groups + h / a.unit_heads];
-        nsplit = paged_len(a, b) > 0 ? u.y : 0;
-        first = static_cast<size_t>(u.x) * a.unit_heads + h % a.unit_heads;
+        const HeadPartials hp =
+            head_partials(a, a.units[b * a.groups + h / a.unit_heads], paged_len(a, b), h);
+        nsplit = hp.count;
+        first = hp.first;
         step = a.unit_heads;
     } else {
         nsplit = args;
@@ -924,18 +824,6 @@ namespace detail {
 
 namespace {
 
-// Split count: enough (batch*head, split) workgroups to give every CU per_cu, with chunks of at
-// least min_chunk keys; an explicit request is clamped to [1, min(1024, ceil(kv_len / 16))]
-// (1024 = dev::kMaxSplits, the combine kernel's bound).
-int choose_splits(int requested, int BH, int kv_len, int min_chunk, int per_cu) {
-    const int max_useful = std::max(1, std::min(dev::kMaxSplits, (kv_len + 15) / 16));
-    if (requested > 0) return std::min(requested, max_useful);
-    const int target_blocks = per_cu * compute_units();
-    int s = (target_blocks + BH - 1) / BH;
-    s = std::min(s, std::max(1, kv_len / min_chunk));
-    return std::max(1, std::min(s, max_useful));
-}
-
 // One decode: the layout and head grouping come in `a` (chunk and nsplit are set here).
 // Workgroups: one per (batch, key/value head, group of G query heads, split); partials and the
 // combine: one slot per (batch, query head).
@@ -946,11 +834,6 @@ struct FixedScratch {
     size_t bytes;
 };
 
-// Minimum keys per split of the automatic split count (4 blocks of the matrix-core kernels):
-// short sequences still spread over the chip (512-key chunks -> 128: plain decode, B = 1, 32
-// heads, 1024 keys 13.6 -> 9.0 us; grouped-query, B = 1, 2 key/value heads, 32768 keys 26 ->
-// 19 us; config 4's automatic 4 splits are unaffected).
-constexpr int kMinChunk = 128;
 // Workgroups per CU that the one-head matrix-core kernel's split count aims at: 4 (its LDS
 // occupancy at head_dim 128); 8 at head_dim 32, whose 512-byte group loads need more workgroups
 // in flight (16 x 8 key/value heads x 32768 keys: 130 -> 89 us; head_dim 64: 156 -> 161 us).
@@ -982,38 +865,20 @@ FlashAttentionError run_decode(const T* Q, const T* K, const T* V, T* O, float* 
     // The one-head matrix-core kernel's workgroup is one wave: mma_per_cu(D) workgroups per CU
     // (grouped-query decode, head_dim 128, 16 x 8 key/value heads x 32768 keys: 8 -> 4 per CU,
     // 327 -> 314 us). The four-head kernel: one workgroup per CU (its LDS occupancy).
-    a.nsplit = choose_splits(num_splits, static_cast<int>(groups), a.kv_len,
-                             kMinChunk,
-                             rows ? kRowsPerCu : (MMA ? mma_per_cu(D) : 8));
-    a.chunk = (a.kv_len + a.nsplit - 1) / a.nsplit;
-    if constexpr (MMA) {
-        a.chunk = std::max(32, (a.chunk + 31) / 32 * 32);
-        a.nsplit = std::max(1, (a.kv_len + a.chunk - 1) / a.chunk);
-    }
+    dev::equal_splits(a, num_splits, static_cast<int>(groups),
+                      (rows ? kRowsPerCu : (MMA ? mma_per_cu(D) : 8)) * compute_units(), MMA);
     long long blocks = groups * a.nsplit;
     long long slots = bhq * a.nsplit;
     if (blocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;  // the grid's limit
     // Automatic splits of caches with room for at least 16 blocks (1 MB) per workgroup: the
-    // balanced split (its block counts in 32 bits). Where all sequences fill the cache it costs 0.5 to 2 us
-    // (BalancedArgs): 1% from here on, but 3 to 8% of smaller caches. Not in a captured launch: an
-    // earlier form of it faulted in a graph's replay, for a reason not found.
-    const long long cap_blocks = (static_cast<long long>(a.kv_len) + 31) / 32;
-    const bool balanced = rows && num_splits == 0 && B > 1 &&
-                          groups * cap_blocks >= 16LL * compute_units() &&
-                          groups * cap_blocks < (1LL << 27) && fixed.ptr == nullptr &&
-                          !stream_capturing(stream);
+    // balanced split. Where all sequences fill the cache it costs 0.5 to 2 us (BalancedArgs): 1%
+    // from here on, but 3 to 8% of smaller caches. Not in a captured launch: an earlier form of it
+    // faulted in a graph's replay, for a reason not found.
     dev::BalancedArgs bal{};
+    const bool balanced = rows && num_splits == 0 && B > 1 && fixed.ptr == nullptr &&
+                          dev::balanced_plan(bal, a, B, groups, kRowsPerCu * compute_units()) &&
+                          !stream_capturing(stream);
     if (balanced) {
-        static_cast<dev::DecodeArgs&>(bal) = a;
-        bal.B = B;
-        bal.groups = static_cast<int>(groups / B);
-        bal.unit_heads = a.H / bal.groups;
-        // At least kMinChunk keys per segment, and no more per unit than the combine can hold.
-        bal.min_blocks = static_cast<int>(std::max<long long>(
-            kMinChunk / 32, (cap_blocks + dev::kMaxSplits - 1) / dev::kMaxSplits));
-        const long long wgs = static_cast<long long>(kRowsPerCu) * compute_units();
-        bal.max_segments = static_cast<int>(std::max({wgs, 2 * groups, blocks}));
-        bal.full_blocks = static_cast<int>(groups * cap_blocks * 7 / 8);
         blocks = bal.max_segments;
         slots = static_cast<long long>(bal.max_segments) * bal.unit_heads;
     }

@@ -25,3 +25,8 @@ def _run(name, tmp_path, *args):
 
 def test_unknown_capture_status_counts_as_captured(tmp_path):
     _run("test_capture_status", tmp_path)
+
+
+def test_balanced_paged_split_stays_in_bounds(tmp_path):
+    """Over launches that keep the equal splits, that balance, and that are nearly full."""
+    _run("test_paged_split", tmp_path, 3000, 1)

@@ -1,8 +1,8 @@
 """The balanced split of a paged grouped-query decode (BalancedArgs in decode.hip).
 
 A paged decode with automatic splits cuts each sequence into as many segments as its length asks
-for, so a sequence can have none, one or many, a last segment can be short or empty, and where the
-cache is almost full the equal splits of its capacity are kept. Lengths that do each of these are
+for, so a sequence can have none, one or many, a last segment can be short, and where the cache is
+almost full the equal splits of its capacity are kept. Lengths that do each of these are
 checked row by row against the fp64 oracle; the bounds are those of an MFMA decode with V in
 [-1, 1): the unit roundoff of P and of O, and 2e-5 for L (fp32 sums of exact products).
 """
