@@ -584,144 +584,150 @@ __global__ void __launch_bounds__(64 * (512 / D))
     __shared__ __attribute__((aligned(1024))) unsigned char Vb0[BN * Lay::kRowV];
     __shared__ __attribute__((aligned(1024))) unsigned char Vb1[BN * Lay::kRowV];
 
+    // The workgroup's keys [kbeg, kend) of sequence b, for the query heads of the NW key/value heads
+    // from NW quad on (wave w: head NW quad + w).
     const int hpk = a.H / a.Hkv;
-    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int lane = threadIdx.x & 63;
-    const int l32 = lane & 31;
-    const int g2 = lane >> 5;
-
-
-    // One segment: keys [kbeg, kend) of sequence b for the query heads of the NW key/value heads
-    // from NW quad on (wave w: head NW quad + w); the partial of the i-th of them goes to slot0 +
-    // i slot_step.
-    auto segment = [&](int b, int quad, int kbeg, int kend, size_t slot0, size_t slot_step) {
-        const int h0 = (quad * NW + w) * hpk;
-        const int nblk = kend > kbeg ? (kend - kbeg + BN - 1) / BN : 0;
-        // Key row t of the NW heads: Kq + ((page_of(t) page_size + t % page_size) Hkv) D.
-        const uint16_t* Kq = K + static_cast<size_t>(quad) * NW * D;
-        const uint16_t* Vq = V + static_cast<size_t>(quad) * NW * D;
-        auto page_of = [&](int t) {
-            const int j = a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size;
-            return a.block_table[static_cast<size_t>(b) * a.max_pages + j];
-        };
-        auto row_off = [&](int t, int page) -> size_t {
-            const int r = a.page_shift >= 0 ? t & (a.page_size - 1) : t % a.page_size;
-            return (static_cast<size_t>(page) * a.page_size + r) * static_cast<size_t>(a.Hkv) * D;
-        };
-
-        // Q^T: lane l32 holds query head h0 + l32 (zeros past the group), dims 16 ks + 8 g2 .. + 8.
-        frag qf[KS];
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if (l32 < hpk) v = ld16(Q + (static_cast<size_t>(b) * a.H + h0 + l32) * D + 16 * ks + 8 * g2);
-            qf[ks] = as_frag<T>(v);
-        }
-
-        // Tile loads: row RPW w + i of the block at key0 (clamped to kend - 1) by one instruction,
-        // lane i: the 16 bytes at 16 i of the row's 1 KB. Its page is lane i of `pages`.
-        const unsigned ld_voff = static_cast<unsigned>(lane * 16);
-        auto fetch_pages = [&](int key0) {
-            int pg = 0;
-            if (lane < RPW && key0 < kend) pg = page_of(min(key0 + RPW * w + lane, kend - 1));
-            return pg;
-        };
-        auto load_tile = [&](const uint16_t* src, int key0, unsigned char* dst, int row_bytes,
-                             int pages) {
-#pragma unroll
-            for (int i = 0; i < RPW; ++i) {
-                const int t = min(key0 + RPW * w + i, kend - 1);
-                // The base comes from v_readlane and the compiler cannot prove it uniform: read it
-                // into SGPRs (the load statement's wait states cover the VALU write).
-                const uint16_t* sb = src + row_off(t, __builtin_amdgcn_readlane(pages, i));
-                lds_dma16_nt_s(uniform_ptr(sb), ld_voff, dst + (RPW * w + i) * row_bytes);
-            }
-        };
-        // Operand offsets in the row layout: K rows (lane l32 = key, chunk 2 ks + g2 of head w) and
-        // the V transpose reads (rows 4 g2 + (lane % 16) / 4, chunks 2 ((lane / 16) % 2) +
-        // (lane % 4) / 2, half lane % 2).
-        const int k_off = l32 * Lay::kRowK + w * 2 * D + g2 * 16;
-        const int k_base[2] = {k_off, k_off};
-        const int kq = lane & 15;
-        const int v_off = (4 * g2 + (kq >> 2)) * Lay::kRowV + w * 2 * D +
-                          (2 * ((lane >> 4) & 1) + ((kq & 3) >> 1)) * 16 + (kq & 1) * 8;
-
-        f32x16 o[NDT];
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16{};
-        float m = -INFINITY;
-        float l = 0.0f;
-        const float cs = fmaxf(a.c, kFltMin);  // scale 0: -inf * 0 would make the masked scores NaN
-
-        // Block j in Kb[j & 1] / Vb[j & 1]. Each wave waits for its own loads of block j (vmcnt(0));
-        // the barrier after it makes every wave's loads visible and ends every wave's reads of block
-        // j - 1, whose buffers block j + 1's loads then fill. `pages` holds the page indices of this
-        // wave's rows of the next block to load.
-        int pages = fetch_pages(kbeg);
-        if (nblk > 0) {
-            load_tile(Kq, kbeg, Kb0, Lay::kRowK, pages);
-            load_tile(Vq, kbeg, Vb0, Lay::kRowV, pages);
-            pages = fetch_pages(kbeg + BN);
-        }
-        for (int j = 0; j < nblk; j += 2) {
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            if (j + 1 < nblk) {
-                load_tile(Kq, kbeg + (j + 1) * BN, Kb1, Lay::kRowK, pages);
-                load_tile(Vq, kbeg + (j + 1) * BN, Vb1, Lay::kRowV, pages);
-                pages = fetch_pages(kbeg + (j + 2) * BN);
-            }
-            kv_block32<T, D, Lay>(Kb0, Vb0, k_base, v_off, kbeg + j * BN, kend, kend, g2, cs, qf, o, m,
-                                  l, [] {});
-            if (j + 1 >= nblk) break;
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            if (j + 2 < nblk) {
-                load_tile(Kq, kbeg + (j + 2) * BN, Kb0, Lay::kRowK, pages);
-                load_tile(Vq, kbeg + (j + 2) * BN, Vb0, Lay::kRowV, pages);
-                pages = fetch_pages(kbeg + (j + 3) * BN);
-            }
-            kv_block32<T, D, Lay>(Kb1, Vb1, k_base, v_off, kbeg + (j + 1) * BN, kend, kend, g2, cs, qf,
-                                  o, m, l, [] {});
-        }
-
-        // Partials of this wave's query heads: lane l32 < G holds head h0 + l32, dims 32 dt + 8 q +
-        // 4 g2 .. + 3 in o[dt][4 q .. 4 q + 3].
-        l = pair_sum(l);
-        if (l32 < hpk) {
-            const size_t slot = slot0 + (w * hpk + l32) * slot_step;
-            float* dst = part_acc + slot * D;
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) {
-#pragma unroll
-                for (int qq = 0; qq < 4; ++qq) {
-                    f32x4 v;
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) v[u] = o[dt][4 * qq + u];
-                    st16(dst + 32 * dt + 8 * qq + 4 * g2, __builtin_bit_cast(u32x4, v));
-                }
-            }
-            if (g2 == 0) part_ml[slot] = make_float2(m, l);
-        }
-    };
+    int b, quad, split, kbeg, kend;
     if constexpr (is_balanced<Args>()) {
-        const int x = blockIdx.x;
-        const PagedSegment ps = paged_segment<GpuWave>(a, x);
+        const PagedSegment ps = paged_segment<GpuWave>(a, blockIdx.x);
         if (ps.parts == 0) return;  // past the last segment
         if (ps.part == 0 && threadIdx.x == 0)
-            a.units[ps.b * a.groups + ps.g] = make_int2(x, ps.parts);
-        segment(ps.b, ps.g, ps.kbeg, ps.kend, static_cast<size_t>(x) * a.unit_heads, 1);
+            a.units[ps.b * a.groups + ps.g] = make_int2(blockIdx.x, ps.parts);
+        b = ps.b;
+        quad = ps.g;
+        kbeg = ps.kbeg;
+        kend = ps.kend;
     } else {
         // blockIdx.x = (b * (Hkv / NW) + quad) * nsplit + split.
         const int nquad = a.Hkv / NW;
         int rest = blockIdx.x;
-        const int split = rest % a.nsplit;
+        split = rest % a.nsplit;
         rest /= a.nsplit;
-        const int quad = rest % nquad;
-        const int b = rest / nquad;
-        const int kbeg = split * a.chunk;
-        segment(b, quad, kbeg, min(min(max(a.seq_lens[b], 0), a.kv_len), kbeg + a.chunk),
-                (static_cast<size_t>(b) * a.H + quad * NW * hpk) * a.nsplit + split, a.nsplit);
+        quad = rest % nquad;
+        b = rest / nquad;
+    }
+    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int hk = quad * NW + w;
+    const int h0 = hk * hpk;
+    const int lane = threadIdx.x & 63;
+    const int l32 = lane & 31;
+    const int g2 = lane >> 5;
+
+    if constexpr (!is_balanced<Args>()) {
+        const int kv_b = paged_len(a, b);
+        kbeg = split * a.chunk;
+        kend = min(kv_b, kbeg + a.chunk);
+    }
+    const int nblk = kend > kbeg ? (kend - kbeg + BN - 1) / BN : 0;
+    // Key row t of the NW heads: Kq + ((page_of(t) page_size + t % page_size) Hkv) D.
+    const uint16_t* Kq = K + static_cast<size_t>(quad) * NW * D;
+    const uint16_t* Vq = V + static_cast<size_t>(quad) * NW * D;
+    auto page_of = [&](int t) {
+        const int j = a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size;
+        return a.block_table[static_cast<size_t>(b) * a.max_pages + j];
+    };
+    auto row_off = [&](int t, int page) -> size_t {
+        const int r = a.page_shift >= 0 ? t & (a.page_size - 1) : t % a.page_size;
+        return (static_cast<size_t>(page) * a.page_size + r) * static_cast<size_t>(a.Hkv) * D;
+    };
+
+    // Q^T: lane l32 holds query head h0 + l32 (zeros past the group), dims 16 ks + 8 g2 .. + 8.
+    frag qf[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (l32 < hpk) v = ld16(Q + (static_cast<size_t>(b) * a.H + h0 + l32) * D + 16 * ks + 8 * g2);
+        qf[ks] = as_frag<T>(v);
+    }
+
+    // Tile loads: row RPW w + i of the block at key0 (clamped to kend - 1) by one instruction,
+    // lane i: the 16 bytes at 16 i of the row's 1 KB. Its page is lane i of `pages`.
+    const unsigned ld_voff = static_cast<unsigned>(lane * 16);
+    auto fetch_pages = [&](int key0) {
+        int pg = 0;
+        if (lane < RPW && key0 < kend) pg = page_of(min(key0 + RPW * w + lane, kend - 1));
+        return pg;
+    };
+    auto load_tile = [&](const uint16_t* src, int key0, unsigned char* dst, int row_bytes,
+                         int pages) {
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) {
+            const int t = min(key0 + RPW * w + i, kend - 1);
+            // The base comes from v_readlane and the compiler cannot prove it uniform: read it
+            // into SGPRs (the load statement's wait states cover the VALU write).
+            const uint16_t* sb = src + row_off(t, __builtin_amdgcn_readlane(pages, i));
+            lds_dma16_nt_s(uniform_ptr(sb), ld_voff, dst + (RPW * w + i) * row_bytes);
+        }
+    };
+    // Operand offsets in the row layout: K rows (lane l32 = key, chunk 2 ks + g2 of head w) and
+    // the V transpose reads (rows 4 g2 + (lane % 16) / 4, chunks 2 ((lane / 16) % 2) +
+    // (lane % 4) / 2, half lane % 2).
+    const int k_off = l32 * Lay::kRowK + w * 2 * D + g2 * 16;
+    const int k_base[2] = {k_off, k_off};
+    const int kq = lane & 15;
+    const int v_off = (4 * g2 + (kq >> 2)) * Lay::kRowV + w * 2 * D +
+                      (2 * ((lane >> 4) & 1) + ((kq & 3) >> 1)) * 16 + (kq & 1) * 8;
+
+    f32x16 o[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16{};
+    float m = -INFINITY;
+    float l = 0.0f;
+    const float cs = fmaxf(a.c, kFltMin);  // scale 0: -inf * 0 would make the masked scores NaN
+
+    // Block j in Kb[j & 1] / Vb[j & 1]. Each wave waits for its own loads of block j (vmcnt(0));
+    // the barrier after it makes every wave's loads visible and ends every wave's reads of block
+    // j - 1, whose buffers block j + 1's loads then fill. `pages` holds the page indices of this
+    // wave's rows of the next block to load.
+    int pages = fetch_pages(kbeg);
+    if (nblk > 0) {
+        load_tile(Kq, kbeg, Kb0, Lay::kRowK, pages);
+        load_tile(Vq, kbeg, Vb0, Lay::kRowV, pages);
+        pages = fetch_pages(kbeg + BN);
+    }
+    for (int j = 0; j < nblk; j += 2) {
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (j + 1 < nblk) {
+            load_tile(Kq, kbeg + (j + 1) * BN, Kb1, Lay::kRowK, pages);
+            load_tile(Vq, kbeg + (j + 1) * BN, Vb1, Lay::kRowV, pages);
+            pages = fetch_pages(kbeg + (j + 2) * BN);
+        }
+        kv_block32<T, D, Lay>(Kb0, Vb0, k_base, v_off, kbeg + j * BN, kend, kend, g2, cs, qf, o, m,
+                              l, [] {});
+        if (j + 1 >= nblk) break;
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (j + 2 < nblk) {
+            load_tile(Kq, kbeg + (j + 2) * BN, Kb0, Lay::kRowK, pages);
+            load_tile(Vq, kbeg + (j + 2) * BN, Vb0, Lay::kRowV, pages);
+            pages = fetch_pages(kbeg + (j + 3) * BN);
+        }
+        kv_block32<T, D, Lay>(Kb1, Vb1, k_base, v_off, kbeg + (j + 1) * BN, kend, kend, g2, cs, qf,
+                              o, m, l, [] {});
+    }
+
+    // Partials of this wave's query heads: lane l32 < G holds head h0 + l32, dims 32 dt + 8 q +
+    // 4 g2 .. + 3 in o[dt][4 q .. 4 q + 3].
+    l = pair_sum(l);
+    if (l32 < hpk) {
+        size_t slot;
+        if constexpr (is_balanced<Args>())
+            slot = static_cast<size_t>(blockIdx.x) * a.unit_heads + w * hpk + l32;
+        else
+            slot = (static_cast<size_t>(b) * a.H + h0 + l32) * a.nsplit + split;
+        float* dst = part_acc + slot * D;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) {
+#pragma unroll
+            for (int qq = 0; qq < 4; ++qq) {
+                f32x4 v;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = o[dt][4 * qq + u];
+                st16(dst + 32 * dt + 8 * qq + 4 * g2, __builtin_bit_cast(u32x4, v));
+            }
+        }
+        if (g2 == 0) part_ml[slot] = make_float2(m, l);
     }
 }
 
