@@ -877,16 +877,16 @@ FlashAttentionError run_decode(const T* Q, const T* K, const T* V, T* O, float* 
     long long slots = bhq * a.nsplit;
     if (blocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;  // the grid's limit
     // Automatic splits of caches with room for at least 16 blocks (1 MB) per workgroup: the
-    // balanced split. Where all sequences fill the cache it costs 0.5 to 2 us (BalancedArgs): 1%
-    // from here on, but 3 to 8% of smaller caches. Not in a captured launch: an earlier form of it
+    // balanced split. Where all sequences fill the cache it costs 0.5 to 2.7 us (BalancedArgs): up to
+    // 1.5% from here on, but 3 to 8% of smaller caches. Not in a captured launch: an earlier form of it
     // faulted in a graph's replay, for a reason not found.
     dev::BalancedArgs bal{};
     const bool balanced = rows && num_splits == 0 && B > 1 && fixed.ptr == nullptr &&
                           dev::balanced_plan(bal, a, B, groups, kRowsPerCu * compute_units()) &&
                           !stream_capturing(stream);
     if (balanced) {
-        blocks = bal.max_segments;
-        slots = static_cast<long long>(bal.max_segments) * bal.unit_heads;
+        blocks = bal.entries;
+        slots = static_cast<long long>(bal.entries) * bal.unit_heads;
     }
 
     const size_t acc_bytes = static_cast<size_t>(slots) * D * sizeof(float);

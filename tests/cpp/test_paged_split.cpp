@@ -3,7 +3,8 @@
 // address checked against the array it goes to. No GPU call is made.
 //
 // Checked for each launch: every segment lies inside its sequence and has keys; every key of every
-// unit belongs to exactly one segment; every partial is written to one entry below max_segments;
+// unit belongs to exactly one segment; every partial is written to one of the `entries`;
+// the segments of caches that are not nearly full fit whole rounds of workgroups;
 // the entries of a unit follow each other from the one its first segment notes; the combine of
 // every query head reads just these, at most kMaxSplits; pages stay below max_pages.
 //
@@ -108,17 +109,18 @@ int launch(std::mt19937& rng) {
     if (!balanced_plan(bal, a, B, units, wgs)) return 0;
     CHECK(bal.groups * static_cast<long long>(B) == units);
     CHECK(bal.unit_heads * bal.groups == a.H);
-    CHECK(bal.max_segments >= 2 * units && bal.max_segments >= units * a.nsplit);
+    CHECK(bal.max_segments >= 2 * units && bal.max_segments % wgs == 0);
+    CHECK(bal.entries >= bal.max_segments && bal.entries >= units * a.nsplit);
 
     // The split kernel: one workgroup per entry.
     const int2 unwritten = make_int2(0x7ffffff0, 0x7ffffff0);
     std::vector<int2> table(units, unwritten);
-    std::vector<int> owner(bal.max_segments, -1);  // the unit that wrote entry x
+    std::vector<int> owner(bal.entries, -1);  // the unit that wrote entry x
     std::vector<std::vector<std::array<int, 2>>> keys(units);
     long long total = 0;
     for (int b = 0; b < B; ++b) total += (paged_len(a, b) + 31) / 32;
     const bool full = total * bal.groups >= bal.full_blocks;
-    for (int x = 0; x < bal.max_segments; ++x) {
+    for (int x = 0; x < bal.entries; ++x) {
         const PagedSegment s = paged_segment<HostWave>(bal, x);
         if (s.parts == 0) continue;
         CHECK(s.b >= 0 && s.b < B && s.g >= 0 && s.g < bal.groups);
@@ -135,6 +137,12 @@ int launch(std::mt19937& rng) {
         CHECK(x == table[unit].x + s.part && s.parts == table[unit].y);
         keys[unit].push_back({s.kbeg, s.kend});
     }
+    // Below 7/8 of the capacity: at most max_segments, whole rounds of workgroups.
+    if (!full) {
+        size_t segments = 0;
+        for (const auto& k : keys) segments += k.size();
+        CHECK(segments <= static_cast<size_t>(bal.max_segments));
+    }
     // Every key of a unit once, in order.
     for (int unit = 0; unit < units; ++unit) {
         int at = 0;
@@ -145,7 +153,7 @@ int launch(std::mt19937& rng) {
         CHECK(at == paged_len(a, unit / bal.groups));
     }
     // The combine: head bh reads `count` entries from `first` on, unit_heads apart.
-    const size_t slots = static_cast<size_t>(bal.max_segments) * bal.unit_heads;
+    const size_t slots = static_cast<size_t>(bal.entries) * bal.unit_heads;
     for (int b = 0; b < B; ++b) {
         for (int h = 0; h < a.H; ++h) {
             const int unit = b * bal.groups + h / bal.unit_heads;
