@@ -715,8 +715,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
     constexpr int BM = 32 * NW;  // query rows per workgroup (NW waves of 32 rows)
     constexpr int BN = 64;
     constexpr int kParts = 8 / NW;  // load instructions per wave per 64-row tile
-    using Lay = TileGroups<D>;
-    constexpr int GRP = Lay::kBytes;       // bytes per 8-row group
+    constexpr int GRP = 1152;              // bytes per 8-row group
     constexpr int TILE = (BN / 8) * GRP;   // bytes per 64-row tile
     static_assert(kParts >= 1, "at most eight waves");
     using frag = typename Elem<T>::frag;
@@ -753,14 +752,14 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
     const int nkb = (kv_end + BN - 1) / BN;
 
     // Loads of one 64-row tile: wave w fills groups w, w + NW, ... (kParts of them), one
-    // 8-row group (1 KB, TileGroups) per load instruction. Rows past Nk are clamped to row Nk - 1
-    // (finite values; their scores are masked). Issued from inline assembly as in
-    // fwd16_d128_kernel.
+    // 8-row group (1 KB) per load instruction: lane i writes slot i, i.e. chunk i / 8 of row
+    // (i % 8) ^ (4 ((i >> 4) & 1)) of the group. Rows past Nk are clamped to row Nk - 1 (finite
+    // values; their scores are masked). Issued from inline assembly as in fwd16_d128_kernel.
     // A tile that lies inside [0, Nk) is addressed as a scalar base plus a fixed per-lane offset.
-    const int ld_row = Lay::ld_row(lane);
+    const int ld_row = (lane & 7) ^ (4 * ((lane >> 4) & 1));
     // At head_dim 32 a row fills chunks 0-3 of its 128-byte slot; lanes 32-63 load the same
     // chunks again into the unused slots 4-7.
-    const int ld_col = Lay::ld_col(lane);
+    const int ld_col = ((lane >> 3) % (D / 8)) * 8;
     const unsigned ld_voff = static_cast<unsigned>(((8 * wave + ld_row) * D + ld_col) * 2);
     // Part i (0..kParts-1) of a tile load: this wave's group wave + NW i.
     auto load_part = [&](const uint16_t* src, int key0, unsigned char* dst, int i) {
@@ -777,15 +776,20 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
 #pragma unroll
         for (int i = 0; i < kParts; ++i) load_part(src, key0, dst, i);
     };
-    // Per-lane byte offsets of the operand reads (TileGroups): 16 rows of one chunk (K row
-    // reads) fall on 16 distinct 16-byte bank slots and the 32 lanes of a V transpose read
-    // (4 rows x 8 chunk halves) on 32 distinct 8-byte slots. K row reads: chunk 2 ks + g2, so
-    // the swizzle depends on ks & 1.
-    const int k_off_even = Lay::row_base(lane, 0);
-    const int k_off_odd = Lay::row_base(lane, 1);
-    const int v_off = Lay::tr_off(lane);
+    // Per-lane byte offsets of the operand reads. Chunk c of row r of a group sits at
+    // 16 (8 c + (r ^ 4 ((c >> 1) & 1))): 16 rows of one chunk (K row reads) fall on 16 distinct
+    // 16-byte bank slots (the 128 bytes of padding per group shift the next 8 rows by 8 slots),
+    // and the 32 lanes of a V transpose read (4 rows x 8 chunk halves) on 32 distinct 8-byte
+    // slots (the row swizzle moves the chunks 2-3 of a 64-byte span to the other rows).
+    // K row reads: chunk 2 ks + g2, so the swizzle bit is ks & 1.
+    const int k_off_even = (l32 >> 3) * GRP + g2 * 128 + (l32 & 7) * 16;
+    const int k_off_odd = (l32 >> 3) * GRP + g2 * 128 + ((l32 & 7) ^ 4) * 16;
+    const int kq = lane & 15;
+    const int gl = (lane >> 4) & 1;
+    const int v_off = (2 * gl + ((kq & 3) >> 1)) * 128 + (g2 ^ gl) * 64 + (kq >> 2) * 16 +
+                      (kq & 1) * 8;
     auto k_addr = [&](const unsigned char* kt, int t, int ks) {
-        return kt + ((ks & 1) ? k_off_odd : k_off_even) + 4 * t * GRP + Lay::k_off(ks);
+        return kt + ((ks & 1) ? k_off_odd : k_off_even) + 4 * t * GRP + ks * 256;
     };
 
     auto scores = [&](const unsigned char* kt, f32x16 (&s)[2]) {
@@ -841,7 +845,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
         return as_frag<T>(ld16(k_addr(kt, i / KS, i % KS)));
     };
     auto v_frag = [&](const unsigned char* vt, int i) {
-        const unsigned char* a0 = vt + v_off + 2 * (i / NDT) * GRP + Lay::dtile_off(i % NDT);
+        const unsigned char* a0 = vt + v_off + 2 * (i / NDT) * GRP + (i % NDT) * 512;
         return tr_frag_at<T>(a0, a0 + GRP);
     };
 
