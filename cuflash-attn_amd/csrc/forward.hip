@@ -1108,9 +1108,9 @@ __global__ void __launch_bounds__(64 * NW, 16 / NW)
             }
         }
     };
-    const int k_off_even = Lay::row_base(lane, 0);
-    const int k_off_odd = Lay::row_base(lane, 1);
-    const int v_off = Lay::tr_off(lane);
+    const int k_off_even = Lay::row_base(lane, l32, g2, 0);
+    const int k_off_odd = Lay::row_base(lane, l32, g2, 1);
+    const int v_off = Lay::tr_off(lane, g2);
     auto k_frag = [&](const unsigned char* kt, int i) {  // K rows of tile i / KS, k-step i % KS
         const int t = i / KS, ks = i % KS;
         return as_frag<T>(ld16(kt + ((ks & 1) ? k_off_odd : k_off_even) + 4 * t * GRP + Lay::k_off(ks)));

@@ -110,27 +110,34 @@ struct TileGroups<96> : TileGroups<128> {
 };
 // The tiles of fwd16_d64_seq_kernel. Its loads hide behind the vector work of four waves per SIMD,
 // so at head_dim 64 the rows of a group stay interleaved by 16 bytes, chunk c of row r at
-// 16 (8 c + (r ^ 4 ((c / 2) % 2))), on the same 16 and 32 bank slots. Measured, no mask, this
-// order -> TileGroups<64> on one box: B=4, 16 heads, N=3000 162.5 -> 164.7 us; B=12, 16 heads over
-// 4, 183 queries of 2264 keys 45.0 -> 45.7. At head_dim 32 TileGroups is the faster one (causal,
-// B=2, 32 heads, N=2500 49.5 -> 49.0).
+// 16 (8 c + (r ^ 4 ((c / 2) % 2))), on the same 16 and 32 bank slots (fwd16_d64_kernel has the same
+// order). Measured, no mask, this order -> TileGroups<64> on one box: B=4, 16 heads, N=3000
+// 162.5 -> 164.7 us; B=12, 16 heads over 4, 183 queries of 2264 keys 45.0 -> 45.7. At head_dim 32
+// TileGroups is the faster one (causal, B=2, 32 heads, N=2500 49.5 -> 49.0).
+// The row and transpose offsets take the kernel's l32 = lane % 32 and g2 = lane / 32 too: formed
+// from the lane, the compiler's address code made the four-wave kernel 1.5% slower (no mask, 32
+// heads, N=1024 17.1 -> 17.4 us; from l32 and g2 16.6).
 template <int D>
-struct SeqTileGroups : TileGroups<D> {};
+struct SeqTileGroups : TileGroups<D> {
+    __device__ static int row_base(int lane, int, int, int odd) {
+        return TileGroups<D>::row_base(lane, odd);
+    }
+    __device__ static int tr_off(int lane, int) { return TileGroups<D>::tr_off(lane); }
+};
 template <>
 struct SeqTileGroups<64> {
     static constexpr int kBytes = 1152;
     static constexpr int k_off(int ks) { return ks * 256; }
     static constexpr int dtile_off(int dt) { return dt * 512; }
     __device__ static int ld_row(int lane) { return (lane & 7) ^ (4 * ((lane >> 4) & 1)); }
-    __device__ static int ld_col(int lane) { return (lane >> 3) * 8; }
-    __device__ static int row_base(int lane, int odd) {
-        return ((lane & 31) >> 3) * kBytes + (lane >> 5) * 128 + ((lane & 7) ^ (4 * odd)) * 16;
+    __device__ static int ld_col(int lane) { return ((lane >> 3) % 8) * 8; }
+    __device__ static int row_base(int, int l32, int g2, int odd) {
+        return (l32 >> 3) * kBytes + g2 * 128 + ((l32 & 7) ^ (4 * odd)) * 16;
     }
-    __device__ static int tr_off(int lane) {
+    __device__ static int tr_off(int lane, int g2) {
         const int kq = lane & 15;
         const int gl = (lane >> 4) & 1;
-        return (2 * gl + ((kq & 3) >> 1)) * 128 + ((lane >> 5) ^ gl) * 64 + (kq >> 2) * 16 +
-               (kq & 1) * 8;
+        return (2 * gl + ((kq & 3) >> 1)) * 128 + (g2 ^ gl) * 64 + (kq >> 2) * 16 + (kq & 1) * 8;
     }
 };
 
