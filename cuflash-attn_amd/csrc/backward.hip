@@ -30,6 +30,7 @@
 // key/value head over all `group` query heads that read it, in registers, before one store.
 
 #include "common.hpp"
+#include "kernel_rules.hpp"
 #include "launch.hpp"
 #include "profile.hpp"
 #include "tile_groups.hpp"
@@ -1534,7 +1535,7 @@ __global__ void __launch_bounds__(256)
 // every wave loads its own tiles, four times the bytes per product of the fused items.
 template <int D>
 struct Bwd16RowsCfg {
-    static constexpr int kWaves = D <= 64 ? 8 : 4;  // two waves per SIMD, or one (registers)
+    static constexpr int kWaves = detail::bwd16_rows_waves<D>();
     static constexpr int kTile = (32 / TileGroups<D>::kRows) * TileGroups<D>::kBytes;
     static constexpr int kSet = 2 * kTile + 256;  // Q and dO (or K and V) block, 32 (L, D)
     static constexpr int P = D + 4;               // pitch of the merge rows (floats)
@@ -1872,14 +1873,6 @@ namespace detail {
 
 namespace {
 
-// Query/key extents of one launch (see the shape note at the top of this file).
-struct BwdShape {
-    int BH;     // query heads over the batch
-    int Nq;     // query rows per head
-    int Nk;     // key rows per key/value head
-    int group;  // query heads per key/value head
-};
-
 // Whether bwd32_kernel (32-row items whose blocks are spread over the waves) beats the kernels of
 // 128-row items for an fp32 backward, from a model of both in units of one matrix-core product over
 // a 128-row item (dq 3, dkdv 4 per query head): the 128-row kernels run in whole rounds of
@@ -1994,40 +1987,6 @@ FlashAttentionError run_backward_two_pass(const T* Q, const T* K, const T* V, co
     return from_hip(hipGetLastError());
 }
 
-// Whether bwd16_rows_kernel beats bwd_fused_kernel, from a model of both in microseconds, fitted to
-// event times of one box (4 to 32 heads, 256 to 4096 rows, causal and not). With U the 32 x 32 blocks
-// of each kind of item in the launch:
-//  * bwd16_rows_kernel: t0 per item and CU plus x per block of U, but at least its longest item,
-//    whose blocks (all query heads of a group for a key tile) are cut over the waves, at cr each;
-//  * bwd_fused_kernel: its longest item at cb per block, or about a third of that and xf per block
-//    of U once its workgroups are all busy; grouped heads add a launch that sums their shares.
-// The first spreads better, the second moves a fourth of the tile bytes per product. Measured
-// (fused -> rows, us): see the kernel; not taken: causal 16 heads, N=2048, head_dim 64 61, 69 and 128
-// 92, 140; 32 heads, N=1024, head_dim 64 38, 52; 8 heads over 1, N=2000, head_dim 128 98, 203.
-template <int D>
-bool bwd16_rows_faster(const BwdShape& sh, bool causal) {
-    constexpr double t0 = D <= 64 ? 3.3 : 3.5;
-    constexpr double x = (D == 32 ? 0.8 : D == 64 ? 1.16 : D == 96 ? 2.5 : 3.2) * 1e-3;
-    constexpr double cr = D <= 64 ? 0.8 : 1.1;
-    constexpr double cb = D == 32 ? 0.7 : D == 64 ? 0.68 : D == 96 ? 0.92 : 1.11;
-    constexpr double xf = (D == 32 ? 0.9 : D == 64 ? 1.17 : D == 96 ? 1.4 : 1.78) * 1e-3;
-    constexpr int kWaves = dev::Bwd16RowsCfg<D>::kWaves;
-    const double cus = compute_units();
-    const double nqt = (sh.Nq + 31) / 32, nkt = (sh.Nk + 31) / 32;
-    const double frac = causal ? (2.0 * sh.Nk - sh.Nq + 32.0) / (2.0 * sh.Nk) : 1.0;
-    const double blocks = sh.BH * nqt * nkt * frac;
-    const double items = sh.BH * nqt + sh.BH / sh.group * nkt;
-    // Beyond eight items per CU the fused kernel was ahead at every shape measured, by far where the
-    // items are many and short (B=4 H=8, 387 queries, 11693 keys, head_dim 96: 349 against 1057 us).
-    if (items > 8.0 * cus) return false;
-    const double rows = 3.0 + std::max(t0 + std::max(sh.group * nqt, nkt) / kWaves * cr,
-                                       items / cus * t0 + blocks * x);
-    const double longest = std::max(nqt, nkt) * cb;
-    const double fused = 6.5 + std::max(longest, 0.35 * longest + blocks * xf) +
-                         (sh.group > 1 ? 4.0 : 0.0);
-    return 1.05 * rows < fused;
-}
-
 // Path for fp16 / bf16 at head_dim 128 and 64: delta_ld_kernel, then bwd_fused_kernel (dq and
 // dkdv in one launch).
 template <typename T, int D>
@@ -2051,7 +2010,6 @@ FlashAttentionError run_backward_fused(const T* Q, const T* K, const T* V, const
     // Grouped heads: one dkdv item per (query head, key block) with fp32 shares of dK, dV that a
     // second kernel sums, when the shares fit in kMaxShareBytes; an item per (key/value head,
     // key block) would run `group` times longer and leave the launch's tail to a few of them.
-    constexpr long long kMaxShareBytes = 2LL << 30;
     const long long share_bytes = 2LL * sh.BH * sh.Nk * D * static_cast<long long>(sizeof(float));
     const bool shares = sh.group > 1 && share_bytes <= kMaxShareBytes;
     const long long qblocks = static_cast<long long>(nqb) * sh.BH;
@@ -2072,13 +2030,14 @@ FlashAttentionError run_backward_fused(const T* Q, const T* K, const T* V, const
     if (err != FlashAttentionError::SUCCESS) return err;
 
     if constexpr (D != 256) {
-        if (bwd16_rows_faster<D>(sh, causal)) {
-            const int nkt = (sh.Nk + 31) / 32;
-            const long long items = std::max(static_cast<long long>(Npad / 32) * sh.BH,
-                                             static_cast<long long>(nkt) * (sh.BH / sh.group));
+        const int nkt = (sh.Nk + 31) / 32;
+        const long long items = std::max(static_cast<long long>(Npad / 32) * sh.BH,
+                                         static_cast<long long>(nkt) * (sh.BH / sh.group));
+        const long long blocks = (items + 7) / 8 * 16;
+        if (blocks <= 0x7fffffffLL && bwd16_rows_faster<D>(sh, causal, compute_units())) {
             tok = profile_kernel<T, D>("backward_dq_dkdv");
             launch_kernel(tok, (dev::bwd16_rows_kernel<T, D>),
-                          dim3(static_cast<unsigned>((items + 7) / 8 * 16)),
+                          dim3(static_cast<unsigned>(blocks)),
                           dim3(64 * dev::Bwd16RowsCfg<D>::kWaves), 0, stream, q, k, v, ld, go,
                           reinterpret_cast<uint16_t*>(dQ), reinterpret_cast<uint16_t*>(dK),
                           reinterpret_cast<uint16_t*>(dV), sh.Nq, sh.Nk, sh.Nk - sh.Nq, sh.group,

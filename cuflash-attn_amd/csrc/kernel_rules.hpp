@@ -1,0 +1,123 @@
+#pragma once
+
+// Which of two kernels a launch takes: models of both kernels' times, in microseconds, from the
+// shape and the number of CUs. Host code without HIP calls; tests/cpp/test_kernel_rules.cpp holds the
+// rules to times measured on both sides of their lines.
+
+#include <algorithm>
+#include <cmath>
+
+namespace cuflash {
+namespace detail {
+
+// Query/key extents of one launch.
+struct BwdShape {
+    int BH;     // query heads over the batch
+    int Nq;     // query rows per head
+    int Nk;     // key rows per key/value head
+    int group;  // query heads per key/value head
+};
+
+// Waves per workgroup of bwd16_rows_kernel, and the device memory that the fused backward's dK / dV
+// shares of grouped heads may take.
+template <int D>
+constexpr int bwd16_rows_waves() {
+    return D <= 64 ? 8 : 4;  // two waves per SIMD, or one (registers)
+}
+constexpr long long kMaxShareBytes = 2LL << 30;
+
+// A backward's items: dq and dkdv items, the average and the longest item of each kind. For the
+// kernels of 32-row items in rounds of one 32 x 32 block per wave, for those of 128-row items in
+// 32-row blocks of the other side.
+struct BwdItems {
+    double nq, nk;  // items
+    double aq, ak;  // average
+    double lq, lk;  // longest
+};
+inline BwdItems row_items(const BwdShape& sh, bool causal, int waves) {
+    const double nqt = (sh.Nq + 31LL) / 32, nkt = (sh.Nk + 31LL) / 32;
+    BwdItems it;
+    it.nq = sh.BH * nqt;
+    it.nk = sh.BH / sh.group * nkt;
+    it.lq = std::ceil(nkt / waves);
+    it.lk = std::ceil(sh.group * nqt / waves);
+    it.aq = it.lq;
+    it.ak = it.lk;
+    if (causal && nqt > 1) {
+        const double half = (waves - 1) / (2.0 * waves);  // what rounding up adds on average
+        const double q = nkt - (nqt - 1) / 2.0, k = nqt * (1.0 - (nqt - 1) / (2.0 * nkt));
+        it.aq = std::min(std::max(1.0, q / waves + half), it.lq);
+        it.ak = std::min(std::max(1.0, sh.group * k / waves + half), it.lk);
+    }
+    return it;
+}
+// heads: the query heads that one dkdv item takes (the group, or 1 where they leave shares).
+inline BwdItems block_items(const BwdShape& sh, bool causal, int heads) {
+    const double nqt = (sh.Nq + 31LL) / 32, nkt = (sh.Nk + 31LL) / 32;
+    BwdItems it;
+    it.nq = static_cast<double>(sh.BH) * ((sh.Nq + 127LL) / 128);
+    it.nk = static_cast<double>(sh.BH / heads) * ((sh.Nk + 127LL) / 128);
+    it.lq = nkt;
+    it.lk = heads * nqt;
+    it.aq = it.lq;
+    it.ak = it.lk;
+    if (causal) {
+        if (nqt > 4) it.aq = nkt - (nqt - 4) / 2.0;
+        const double k = nqt * (1.0 - (nqt - 1) / (2.0 * nkt));
+        it.ak = heads * std::min(nqt, std::max(k, 1.0) + (nqt > 1 ? 1.5 : 0.0));
+    }
+    return it;
+}
+
+// A kernel's costs: what an item of each kind pays besides its blocks (start, merge, store) and per
+// round or block, the share by which blocks cost more once the CUs are full, and the part of the
+// longest item by which a launch of many items ends late.
+struct BwdCost {
+    double iq, ik;
+    double cq, ck;
+    double full, tail;
+};
+// Time of `it` where `per_cu` workgroups share a CU: the longest item, or all of them spread over
+// the CUs and the tail.
+inline double item_time(const BwdItems& it, const BwdCost& c, double cus, double per_cu) {
+    const double n = it.nq + it.nk;
+    const double per = std::min(per_cu, std::max(1.0, n / cus));
+    const double more = 1.0 + c.full * (per_cu > 1 ? per - 1.0 : std::min(1.0, n / cus));
+    const double work = (it.nq * (c.iq + it.aq * c.cq * more) + it.nk * (c.ik + it.ak * c.ck * more)) /
+                        (cus * per);
+    const double longest = std::max(c.iq + it.lq * c.cq, c.ik + it.lk * c.ck);
+    return std::max(longest, work + c.tail * longest);
+}
+
+// Whether bwd16_rows_kernel beats bwd_fused_kernel. The first spreads better, the second moves a
+// fourth of the tile bytes per product; grouped heads leave it shares that another launch sums. The
+// costs are fitted to 2200 random launches (32 to 8192 keys), in which the choice is on average
+// 1.6% slower than the better kernel (bwd_fused_kernel alone: 37%) and 20 take a kernel that is
+// more than 2% slower. Measured (bwd_fused_kernel, bwd16_rows_kernel, us; more at the kernel): taken:
+// 8 heads, N=1024, head_dim 64 28.5, 14.4. Not taken: causal 16 heads, N=2048, head_dim 64 61, 69
+// and 128 92, 140; 32 heads, N=1024, head_dim 64 38, 52; 8 heads over 1, N=2000, head_dim 128 98,
+// 203; no mask, 22 heads, 278 of 943 keys, head_dim 96 29, 53 (and causal 36 heads, 43 of 349
+// keys, head_dim 128 19, 26): the short side has too few blocks for the waves.
+template <int D>
+bool bwd16_rows_faster(const BwdShape& sh, bool causal, int compute_units) {
+    constexpr BwdCost kRows = D == 32   ? BwdCost{3.25, 3.74, 0.80, 1.03, 0.14, 0.47}
+                              : D == 64 ? BwdCost{4.97, 6.71, 0.93, 1.19, 0.19, 0.36}
+                              : D == 96 ? BwdCost{4.77, 6.48, 1.13, 1.46, 0.31, 0.24}
+                                        : BwdCost{5.26, 7.65, 1.35, 1.63, 0.36, 0.19};
+    constexpr BwdCost kFused = D == 32   ? BwdCost{10.6, 10.6, 0.44, 0.56, 0.03, 0.62}
+                               : D == 64 ? BwdCost{10.7, 10.7, 0.48, 0.68, 0.73, 0.41}
+                               : D == 96 ? BwdCost{10.8, 10.8, 0.61, 0.93, 0.81, 0.38}
+                                         : BwdCost{12.8, 12.8, 0.65, 1.05, 0.93, 0.54};
+    // The sum of the shares: its launch, and the shares at so many bytes per microsecond.
+    constexpr double kSum = D == 32 ? 0.2 : D == 64 ? 6.2 : D == 96 ? 8.2 : 5.4;
+    constexpr double kRate = (D == 32 ? 0.76 : D == 64 ? 1.90 : D == 96 ? 2.28 : 2.49) * 1e6;
+    const double cus = compute_units;
+    const double share_bytes = 2.0 * sh.BH * sh.Nk * D * sizeof(float);
+    const bool shares = sh.group > 1 && share_bytes <= kMaxShareBytes;
+    double fused = item_time(block_items(sh, causal, shares ? 1 : sh.group), kFused, cus, 2.0);
+    if (shares) fused += kSum + share_bytes / kRate;
+    return 1.2 * item_time(row_items(sh, causal, bwd16_rows_waves<D>()), kRows, cus, 1.0) < fused;
+}
+
+}  // namespace detail
+}  // namespace cuflash

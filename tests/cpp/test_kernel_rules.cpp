@@ -1,0 +1,81 @@
+// The rules that choose between two kernels (cuflash-attn_amd/csrc/kernel_rules.hpp), held to measured
+// times: where one kernel was more than 15% faster, the rule takes that one. No GPU call is made.
+//
+// Times of one box in microseconds of a whole call, fp16 / bf16 or fp32, on 256 CUs.
+
+#include <cstdio>
+
+#include "kernel_rules.hpp"
+
+namespace {
+
+using namespace cuflash::detail;
+constexpr int kCus = 256;
+
+struct Row {
+    int D, B, H, Hkv, Nq, Nk;
+    bool causal;
+    double before, rows;  // the kernels of 128-row blocks, the kernel of 32-row items
+};
+
+// bwd_fused_kernel and bwd16_rows_kernel.
+constexpr Row kBackward16[] = {
+    {128, 1, 8, 8, 1147, 5009, false, 139.2, 249.3},
+    {64, 3, 16, 16, 54, 371, true, 15.2, 26.9},
+    {64, 10, 4, 4, 71, 579, true, 19.9, 32.5},
+    {128, 14, 1, 1, 393, 2682, false, 82.6, 133.2},
+    {96, 5, 8, 8, 74, 575, true, 22.5, 35.6},
+    {128, 11, 1, 1, 794, 1944, true, 57.3, 90.3},
+    {128, 5, 4, 4, 293, 1527, true, 53.2, 80.0},
+    {64, 1, 32, 32, 97, 948, true, 28.3, 42.4},
+    {96, 11, 1, 1, 166, 1019, true, 29.6, 22.2},
+    {128, 3, 2, 2, 223, 411, true, 20.3, 13.2},
+    {32, 1, 8, 8, 513, 5734, true, 97.0, 69.0},
+    {64, 6, 1, 1, 47, 4603, true, 81.8, 37.2},
+    {96, 4, 12, 2, 295, 295, true, 39.1, 28.1},
+    {128, 3, 4, 4, 364, 364, true, 25.8, 15.1},
+    {32, 1, 8, 1, 45, 868, true, 40.3, 14.3},
+    {64, 3, 1, 1, 1787, 1787, false, 53.9, 28.5},
+    {128, 1, 32, 4, 36, 536, false, 37.5, 14.3},
+    {128, 1, 32, 8, 87, 89, false, 40.1, 14.4},
+    {32, 6, 16, 16, 137, 567, true, 37.0, 49.0},
+    {64, 5, 8, 8, 1689, 1689, true, 99.0, 149.7},
+    {128, 10, 32, 32, 57, 443, true, 110.0, 219.0},
+    {96, 1, 8, 1, 1376, 1376, true, 65.6, 125.4},
+    {96, 10, 8, 1, 1083, 1083, true, 137.1, 299.8},
+    {64, 15, 4, 4, 61, 428, false, 20.8, 36.4},
+};
+
+template <class Rule>
+int wrong(const char* name, const Row* rows, int n, Rule rule) {
+    int bad = 0;
+    for (int i = 0; i < n; ++i) {
+        const Row& r = rows[i];
+        const bool takes_rows = rule(r);
+        if (takes_rows == (r.rows < r.before)) continue;
+        std::printf("%s: head_dim %d, B=%d, %d heads over %d, %d queries, %d keys, causal %d: %g, "
+                    "%g us, takes the %s\n", name, r.D, r.B, r.H, r.Hkv, r.Nq, r.Nk, r.causal,
+                    r.before, r.rows, takes_rows ? "second" : "first");
+        ++bad;
+    }
+    return bad;
+}
+#define COUNT(t) static_cast<int>(sizeof(t) / sizeof(t[0]))
+
+bool backward16(const Row& r) {
+    const BwdShape s{r.B * r.H, r.Nq, r.Nk, r.H / r.Hkv};
+    switch (r.D) {
+        case 32: return bwd16_rows_faster<32>(s, r.causal, kCus);
+        case 64: return bwd16_rows_faster<64>(s, r.causal, kCus);
+        case 96: return bwd16_rows_faster<96>(s, r.causal, kCus);
+        case 128: return bwd16_rows_faster<128>(s, r.causal, kCus);
+    }
+    return false;
+}
+
+}  // namespace
+
+int main() {
+    int bad = wrong("16-bit backward", kBackward16, COUNT(kBackward16), backward16);
+    return bad;
+}

@@ -30,3 +30,7 @@ def test_unknown_capture_status_counts_as_captured(tmp_path):
 def test_balanced_paged_split_stays_in_bounds(tmp_path):
     """Over launches that keep the equal splits, that balance, and that are nearly full."""
     _run("test_paged_split", tmp_path, 3000, 1)
+
+
+def test_kernel_rules_take_the_measured_faster_kernel(tmp_path):
+    _run("test_kernel_rules", tmp_path)
