@@ -36,7 +36,6 @@
 #include "tile_groups.hpp"
 
 #include <algorithm>
-#include <cmath>
 #include <type_traits>
 
 namespace cuflash {
@@ -1873,34 +1872,6 @@ namespace detail {
 
 namespace {
 
-// Whether bwd32_kernel (32-row items whose blocks are spread over the waves) beats the kernels of
-// 128-row items for an fp32 backward, from a model of both in units of one matrix-core product over
-// a 128-row item (dq 3, dkdv 4 per query head): the 128-row kernels run in whole rounds of
-// workgroups, each as long as its longest item, or, under a causal mask, in their total plus a
-// tail; bwd32_kernel in its total, at a lower rate, since each wave stages blocks of its own.
-// Measured (128-row kernels -> bwd32_kernel, us, whole backward). Taken: causal B=2 H=8 N=1024
-// head_dim 64 169 -> 101, head_dim 32 104 -> 52; B=2 H=16 N=4096 head_dim 64 2930 -> 2330; B=1 H=8
-// N=4096 head_dim 128 2037 -> 1343; 32 heads over 8, N=512, head_dim 128 575 -> 173; non-causal
-// B=2 H=8 N=1024 head_dim 64 170 -> 156. Not taken: causal B=2 H=16 N=4096 head_dim 128 4726, 5314;
-// non-causal B=2 H=16 N=4096 head_dim 64 3853, 4455; B=1 H=8 N=2048 head_dim 128 586, 661;
-// 32 heads over 8, N=2000, head_dim 128 3240, 4030.
-template <int D>
-bool bwd32_faster(const BwdShape& sh, bool causal, double qblocks, double kblocks) {
-    constexpr double kPer = D <= 64 ? 2.0 : 1.0;  // workgroups of the 128-row kernels per CU
-    const double rate = D <= 64 ? 1.13 : sh.group > 1 && !causal ? 1.6 : 1.25;
-    const double cus = compute_units();
-    const double frac = causal ? (2.0 * sh.Nk - sh.Nq + 128.0) / (2.0 * sh.Nk) : 1.0;
-    const double dq = 3.0, dkdv = 4.0 * sh.group;
-    auto rounds = [&](double blocks) {
-        return causal ? std::max(1.0, kPer * (blocks * frac / (cus * kPer) + 0.4))
-                      : std::max(1.0, kPer * std::ceil(blocks / (cus * kPer)));
-    };
-    const double old_time = qblocks + kblocks <= cus
-                                ? std::max(dq, dkdv)
-                                : rounds(qblocks) * dq + rounds(kblocks) * dkdv;
-    return (qblocks * dq + kblocks * dkdv) * frac / cus * rate < old_time;
-}
-
 // Generic path (fp32): delta_kernel, then bwd32_kernel or dq_kernel and dkdv_kernel.
 template <typename T, int D>
 FlashAttentionError run_backward_two_pass(const T* Q, const T* K, const T* V, const T* O,
@@ -1941,13 +1912,12 @@ FlashAttentionError run_backward_two_pass(const T* Q, const T* K, const T* V, co
     const long long kblocks = static_cast<long long>(nkb) * BHkv;
     if (qblocks + kblocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;
     if constexpr (D <= 128) {
-        if (bwd32_faster<D>(sh, causal, static_cast<double>(qblocks), static_cast<double>(kblocks))) {
-            const int nqt = (sh.Nq + 31) / 32;
-            const int nkt = (sh.Nk + 31) / 32;
-            const long long items =
-                std::max(static_cast<long long>(nqt) * sh.BH, static_cast<long long>(nkt) * BHkv);
-            const long long blocks = (items + 7) / 8 * 16;
-            if (blocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;
+        const int nqt = (sh.Nq + 31) / 32;
+        const int nkt = (sh.Nk + 31) / 32;
+        const long long items =
+            std::max(static_cast<long long>(nqt) * sh.BH, static_cast<long long>(nkt) * BHkv);
+        const long long blocks = (items + 7) / 8 * 16;
+        if (blocks <= 0x7fffffffLL && bwd32_faster<D>(sh, causal, compute_units())) {
             // Longest items first, unless all are of one length or there are many per slot.
             const bool head_major =
                 !causal || items >= 8LL * dev::Bwd32Cfg<D>::kPerCu * compute_units();

@@ -89,6 +89,45 @@ inline double item_time(const BwdItems& it, const BwdCost& c, double cus, double
     return std::max(longest, work + c.tail * longest);
 }
 
+// Whether bwd32_kernel (32-row items whose blocks are spread over four waves) beats the kernels of
+// 128-row items for an fp32 backward. Those run dq and dkdv one after the other, each in its longest
+// item or its total and a tail under a causal mask, in whole rounds of workgroups without; or
+// both at once where they fit the CUs. The costs are fitted to 1500 random launches (32 to 8192
+// keys), in which the choice is on average 1.2% slower than the better kernel (bwd32_kernel alone
+// wins by 2x on average) and 8 take a kernel that is more than 2% slower.
+// Measured (128-row kernels, bwd32_kernel, us, whole backward). Taken: causal B=2 H=8 N=1024
+// head_dim 64 169, 101, head_dim 32 104, 52; B=2 H=16 N=4096 head_dim 64 2930, 2330; B=1 H=8
+// N=4096 head_dim 128 2037, 1343; 32 heads over 8, N=512, head_dim 128 575, 173. Not taken: causal
+// B=2 H=16 N=4096 head_dim 128 4726, 5314; 32 heads over 8, N=2000, head_dim 128 3240, 4030; and
+// where the short side has few blocks for the waves: 448 heads, 98 of 459 keys, head_dim 64 292, 458.
+template <int D>
+bool bwd32_faster(const BwdShape& sh, bool causal, int compute_units) {
+    constexpr double kPer = D <= 64 ? 2.0 : 1.0;  // workgroups per CU, of either kind
+    constexpr BwdCost kRows = D == 32   ? BwdCost{1.61, 1.37, 2.05, 2.94, 0.95, 0.35}
+                              : D == 64 ? BwdCost{2.15, 2.67, 3.98, 5.12, 1.34, 0.30}
+                              : D == 96 ? BwdCost{3.03, 3.81, 5.87, 7.55, 0.58, 0.09}
+                                        : BwdCost{6.70, 4.23, 7.38, 9.85, 0.54, 0.19};
+    constexpr BwdCost kBlocks = D == 32   ? BwdCost{2.49, 2.49, 2.29, 3.09, 0.72, 0.18}
+                                : D == 64 ? BwdCost{4.45, 4.45, 3.89, 5.16, 0.80, 0.35}
+                                : D == 96 ? BwdCost{8.45, 8.45, 5.36, 7.02, 0.80, 0.42}
+                                          : BwdCost{10.8, 10.8, 6.86, 9.21, 0.80, 0.48};
+    const double cus = compute_units;
+    const BwdItems it = block_items(sh, causal, sh.group);
+    auto grid = [&](double n, double average, double longest, double c) {
+        const double per = std::min(kPer, std::max(1.0, n / cus));
+        c *= 1.0 + (kPer > 1 ? kBlocks.full * (per - 1.0) : 0.0);
+        if (!causal) return std::ceil(n / (cus * per)) * (kBlocks.iq + average * c);
+        longest = kBlocks.iq + longest * c;
+        return std::max(longest, n * (kBlocks.iq + average * c) / (cus * per) +
+                                     kBlocks.tail * longest);
+    };
+    const double blocks = it.nq + it.nk <= cus
+                              ? kBlocks.iq + std::max(it.lq * kBlocks.cq, it.lk * kBlocks.ck)
+                              : grid(it.nq, it.aq, it.lq, kBlocks.cq) +
+                                    grid(it.nk, it.ak, it.lk, kBlocks.ck);
+    return 1.15 * item_time(row_items(sh, causal, 4), kRows, cus, kPer) < blocks;
+}
+
 // Whether bwd16_rows_kernel beats bwd_fused_kernel. The first spreads better, the second moves a
 // fourth of the tile bytes per product; grouped heads leave it shares that another launch sums. The
 // costs are fitted to 2200 random launches (32 to 8192 keys), in which the choice is on average

@@ -46,6 +46,34 @@ constexpr Row kBackward16[] = {
     {64, 15, 4, 4, 61, 428, false, 20.8, 36.4},
 };
 
+// dq_kernel and dkdv_kernel, bwd32_kernel.
+constexpr Row kBackward32[] = {
+    {64, 8, 32, 32, 57, 562, false, 171.7, 281.5},
+    {64, 14, 32, 32, 98, 459, false, 291.9, 457.5},
+    {96, 7, 32, 32, 68, 206, true, 126.2, 183.9},
+    {96, 12, 16, 16, 40, 231, true, 111.6, 159.7},
+    {128, 7, 32, 32, 97, 244, true, 190.5, 265.4},
+    {64, 8, 32, 32, 77, 214, true, 81.8, 110.2},
+    {32, 6, 32, 32, 173, 1775, false, 403.2, 543.2},
+    {64, 9, 16, 16, 54, 1242, true, 259.5, 335.1},
+    {96, 2, 8, 8, 685, 685, true, 169.0, 96.2},
+    {64, 1, 16, 4, 73, 81, false, 68.8, 21.8},
+    {64, 1, 16, 4, 464, 464, true, 309.4, 84.1},
+    {128, 10, 2, 2, 112, 3011, true, 783.3, 249.4},
+    {96, 5, 32, 32, 152, 152, true, 163.2, 101.1},
+    {32, 1, 16, 16, 1946, 1946, true, 333.4, 160.7},
+    {128, 1, 12, 2, 57, 281, true, 128.0, 38.7},
+    {96, 8, 12, 2, 171, 854, true, 415.7, 305.8},
+    {64, 1, 1, 1, 283, 415, false, 60.8, 22.1},
+    {32, 8, 32, 4, 109, 119, true, 117.0, 30.2},
+    {96, 14, 32, 32, 51, 138, true, 183.4, 246.5},
+    {96, 3, 32, 32, 164, 1000, true, 367.3, 589.2},
+    {128, 15, 16, 16, 50, 608, false, 348.7, 636.9},
+    {64, 15, 32, 32, 244, 539, false, 655.0, 893.9},
+    {96, 6, 16, 16, 171, 1036, false, 421.9, 639.2},
+    {96, 3, 32, 32, 132, 1124, true, 408.5, 615.7},
+};
+
 template <class Rule>
 int wrong(const char* name, const Row* rows, int n, Rule rule) {
     int bad = 0;
@@ -72,10 +100,21 @@ bool backward16(const Row& r) {
     }
     return false;
 }
+bool backward32(const Row& r) {
+    const BwdShape s{r.B * r.H, r.Nq, r.Nk, r.H / r.Hkv};
+    switch (r.D) {
+        case 32: return bwd32_faster<32>(s, r.causal, kCus);
+        case 64: return bwd32_faster<64>(s, r.causal, kCus);
+        case 96: return bwd32_faster<96>(s, r.causal, kCus);
+        case 128: return bwd32_faster<128>(s, r.causal, kCus);
+    }
+    return false;
+}
 
 }  // namespace
 
 int main() {
     int bad = wrong("16-bit backward", kBackward16, COUNT(kBackward16), backward16);
+    bad += wrong("fp32 backward", kBackward32, COUNT(kBackward32), backward32);
     return bad;
 }
