@@ -28,10 +28,8 @@
 // j <= i + coff, coff = Nk - Nq >= 0 (the queries are the last Nq positions of the key
 // sequence; Nq == Nk gives the usual j <= i).
 
-#include <algorithm>
-#include <cmath>
-
 #include "common.hpp"
+#include "kernel_rules.hpp"
 #include "kv_block.hpp"
 #include "launch.hpp"
 #include "profile.hpp"
@@ -1378,18 +1376,14 @@ __global__ void __launch_bounds__(256)
 // Eight waves with one buffer each for K and V (two waves per SIMD, one computing while the
 // other loads) take 11.7 us where four waves with double buffers in the same LDS take 14.6 (head_dim
 // 128, 4 heads, N = 1024), 20.6 against 35 at head_dim 256 with four waves against two.
-template <int D>
-constexpr int fwd_rows_waves() {
-    return D == 256 ? 4 : 8;  // LDS: 135 KB at head_dim 256, 139 KB at 128 and 96, 74 KB below
-}
 template <typename T, int D, bool kSplit>
-__global__ void __launch_bounds__(64 * fwd_rows_waves<D>(), D <= 64 ? 2 : 1)
+__global__ void __launch_bounds__(64 * detail::fwd_rows_waves<D>(), D <= 64 ? 2 : 1)
     fwd16_rows_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
                       const uint16_t* __restrict__ V, uint16_t* __restrict__ O,
                       float* __restrict__ L, int Nq, int Nk, int coff, int group, int nqb,
                       float c, int causal, FwdSplit sp) {
     using Lay = TileGroups<D>;
-    constexpr int NW = fwd_rows_waves<D>();
+    constexpr int NW = detail::fwd_rows_waves<D>();
     constexpr int KS = D / 16;
     constexpr int NDT = D / 32;
     constexpr int BN = 32;            // keys per block
@@ -1953,66 +1947,6 @@ namespace detail {
 
 namespace {
 
-// Query/key extents of one launch (see the shape note at the top of this file).
-struct FwdShape {
-    int BH;     // query heads over the batch
-    int Nq;     // query rows per head
-    int Nk;     // key rows per key/value head
-    int group;  // query heads per key/value head
-};
-
-// Chunks over which fwd16_rows_kernel cuts the keys of this launch, or 0 where the general kernels
-// are faster. The times are modelled in microseconds from measurements (causal and not, 4 to 32
-// heads, 64 to 16384 keys; event times of one box):
-//  * fwd16_rows_kernel: a workgroup walks its longest tile in rounds of one block per wave, tb
-//    each, and t0 for its start, merge and store; as many workgroups as the slots run at once.
-//    Several chunks add the merge kernel and the partials, written and read at about 4 TB/s.
-//  * the general kernels: g per 64-key block of the longest row while their 128-row workgroups all
-//    run at once (more with two workgroups per CU), else 1.5 g per round of them and block of the
-//    average row. They do not pack heads: a few tokens of many heads fill their rows badly.
-// bf16/fp16, causal, B = 1, before -> after: 8 heads, head_dim 128, N = 129 8.4 -> 6.3, 1024 23.9 ->
-// 11.9, 4096 82 -> 64; head_dim 64, N = 256 6.3 -> 5.0, 1024 16.9 -> 8.5, 4096 55.6 -> 34.5;
-// head_dim 256, N = 1024 40.1 -> 22.0; 32 heads over 8 against 8253 keys, head_dim 128: 61 queries
-// 160 -> 22 (4 chunks), one query 156 -> 11.6 (16 chunks); one query of 64 x 32 heads over 8,
-// 1000 keys 206 -> 41. The other side of the line: 32 heads,
-// head_dim 128, N = 1024 25.7 general, 32.7 here; head_dim 64, N = 1536 25.8 and 26.9.
-template <int D>
-int forward_rows_chunks(const FwdShape& sh, bool causal) {
-    constexpr double tb = D == 32 ? 1.2 : D == 64 ? 1.6 : D == 96 ? 1.1 : D == 128 ? 1.36 : 1.95;
-    constexpr double t0 = D <= 64 ? 3.0 : 4.2;
-    constexpr double g = D == 32 ? 0.75 : D == 64 ? 0.85 : D == 96 ? 1.15 : D == 128 ? 1.27 : 2.25;
-    constexpr int kWaves = dev::fwd_rows_waves<D>();
-    const double cus = compute_units();
-    const double slots = D <= 64 ? 2 * cus : cus;
-    const double rows = static_cast<double>(sh.BH) * sh.Nq;
-    const double units = static_cast<double>(sh.BH) * ((sh.Nq + 127) / 128);
-    const double tiles = static_cast<double>(sh.BH / sh.group) *
-                         ((static_cast<long long>(sh.group) * sh.Nq + 31) / 32);
-    const double longest = (sh.Nk + 31) / 32 / static_cast<double>(kWaves);
-    const double average = causal ? longest * (2.0 * sh.Nk - sh.Nq) / (2.0 * sh.Nk) : longest;
-    double best = 0.0;
-    int chunks = 0;
-    for (int n = 1; n == 1 || (n <= 32 && 2 * n <= longest); ++n) {
-        const double rounds = std::ceil(tiles * n / slots);
-        const double walk = rounds > 1 ? average / n : std::ceil(longest / n);
-        double t = rounds * (walk * tb + t0) - 2.0;
-        if (n > 1) t += 4.0 + 2.0 * n * rows * D * sizeof(float) / 4e6;
-        if (chunks == 0 || t < best) {
-            best = t;
-            chunks = n;
-        }
-    }
-    const double blocks = (sh.Nk + 63) / 64;
-    double general;
-    if (units > 2 * cus)
-        general = 1.5 * g * blocks * (average / longest) * units / (2 * cus);
-    else if (D <= 64)
-        general = g * blocks * (1.0 + 0.3 * std::min(1.0, std::max(0.0, units / cus - 1.0)));
-    else
-        general = g * blocks + 4.0 * units / cus;
-    return 1.1 * best < general ? chunks : 0;
-}
-
 // One workgroup per (32 rows of a key/value head's query heads, chunk of keys), and a merge kernel
 // when there are several chunks. The partials need a workspace: a launch that cannot have one,
 // and a captured one (a graph would hold an allocation of tens of MiB where the forward had none),
@@ -2044,7 +1978,7 @@ FlashAttentionError run_forward16_rows(const T* Q, const T* K, const T* V, T* O,
     launch_kernel(tok,
                   sp.nsplit > 1 ? dev::fwd16_rows_kernel<T, D, true>
                                 : dev::fwd16_rows_kernel<T, D, false>,
-                  dim3(static_cast<unsigned>(blocks)), dim3(64 * dev::fwd_rows_waves<D>()), 0,
+                  dim3(static_cast<unsigned>(blocks)), dim3(64 * fwd_rows_waves<D>()), 0,
                   stream, reinterpret_cast<const uint16_t*>(Q),
                   reinterpret_cast<const uint16_t*>(K), reinterpret_cast<const uint16_t*>(V),
                   reinterpret_cast<uint16_t*>(O), L, sh.Nq, sh.Nk, coff, sh.group,
@@ -2081,7 +2015,7 @@ FlashAttentionError run_forward16(const T* Q, const T* K, const T* V, T* O, floa
     long long blocks = static_cast<long long>(nqb) * sh.BH;
     if (blocks > 0x7fffffffLL) return FlashAttentionError::INVALID_DIMENSION;
     const int coff = sh.Nk - sh.Nq;
-    const int chunks = forward_rows_chunks<D>(sh, causal);
+    const int chunks = forward_rows_chunks<D>(sh, causal, compute_units());
     if (chunks > 0)
         return run_forward16_rows<T, D>(Q, K, V, O, L, sh, chunks, scale, causal, stream);
     const ProfileEvents tok = profile_kernel<T, D>("forward");

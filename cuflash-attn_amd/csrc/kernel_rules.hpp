@@ -11,6 +11,14 @@ namespace cuflash {
 namespace detail {
 
 // Query/key extents of one launch.
+struct FwdShape {
+    int BH;     // query heads over the batch
+    int Nq;     // query rows per head
+    int Nk;     // key rows per key/value head
+    int group;  // query heads per key/value head
+};
+
+// Query/key extents of one launch.
 struct BwdShape {
     int BH;     // query heads over the batch
     int Nq;     // query rows per head
@@ -18,13 +26,81 @@ struct BwdShape {
     int group;  // query heads per key/value head
 };
 
-// Waves per workgroup of bwd16_rows_kernel, and the device memory that the fused backward's dK / dV
-// shares of grouped heads may take.
+// Waves per workgroup of fwd16_rows_kernel and bwd16_rows_kernel, and the device memory that the
+// fused backward's dK / dV shares of grouped heads may take.
+template <int D>
+constexpr int fwd_rows_waves() {
+    return D == 256 ? 4 : 8;  // LDS: 134 KB at head_dim 256, 140 KB at 128 and 96, 75 KB below
+}
 template <int D>
 constexpr int bwd16_rows_waves() {
     return D <= 64 ? 8 : 4;  // two waves per SIMD, or one (registers)
 }
 constexpr long long kMaxShareBytes = 2LL << 30;
+
+// Chunks over which fwd16_rows_kernel cuts the keys of this launch, or 0 where the general kernels
+// are faster. The times are modelled from measurements (causal and not, 4 to 32 heads, 64 to 16384
+// keys; event times of one box):
+//  * fwd16_rows_kernel: a workgroup walks its longest tile in rounds of one block per wave, tb
+//    each, and t0 for its start, merge and store; as many workgroups as the slots run at once.
+//    Several chunks add the merge kernel and the partials, written and read at about 4 TB/s. In one
+//    chunk every tile reads its head's keys by itself: where they do not stay in the L2s, at about
+//    6 TB/s.
+//  * the general kernels: g per 64-key block of the longest row while their 128-row workgroups all
+//    run at once (more with two workgroups per CU), else 1.5 g per round of them and block of the
+//    average row. They do not pack heads: a few tokens of many heads fill their rows badly.
+// bf16/fp16, causal, B = 1, before -> after: 8 heads, head_dim 128, N = 129 8.4 -> 6.3, 1024 23.9 ->
+// 11.9, 4096 82 -> 64; head_dim 64, N = 256 6.3 -> 5.0, 1024 16.9 -> 8.5, 4096 55.6 -> 34.5;
+// head_dim 256, N = 1024 40.1 -> 22.0; 32 heads over 8 against 8253 keys, head_dim 128: 61 queries
+// 160 -> 22 (4 chunks), one query 156 -> 11.6 (11 chunks); one query of 64 x 32 heads over 8,
+// 1000 keys 206 -> 41. The other side of the line: 32 heads, head_dim 128, N = 1024 25.7 general,
+// 32.7 here; head_dim 64, N = 1536 25.8 and 26.9; 224 heads, 62 of 458 keys, head_dim 128 16.4, 22.4.
+// Over 2500 random launches of 1 to 8192 keys the choice is on average 0.9% slower than the better
+// kernel, and no launch is both 3% and 0.8 us slower than the general kernel.
+template <int D>
+int forward_rows_chunks(const FwdShape& sh, bool causal, int compute_units) {
+    constexpr double tb = D == 32 ? 1.2 : D == 64 ? 1.6 : D == 96 ? 1.1 : D == 128 ? 1.36 : 1.95;
+    constexpr double t0 = D <= 64 ? 3.0 : 4.2;
+    constexpr double g = D == 32 ? 0.75 : D == 64 ? 0.85 : D == 96 ? 1.15 : D == 128 ? 1.27 : 2.25;
+    constexpr int kWaves = fwd_rows_waves<D>();
+    constexpr double kL2Bytes = 32e6;
+    const double cus = compute_units;
+    const double slots = D <= 64 ? 2 * cus : cus;
+    const double rows = static_cast<double>(sh.BH) * sh.Nq;
+    const double units = static_cast<double>(sh.BH) * ((sh.Nq + 127LL) / 128);
+    const double tiles = static_cast<double>(sh.BH / sh.group) *
+                         ((static_cast<long long>(sh.group) * sh.Nq + 31) / 32);
+    const double longest = (sh.Nk + 31LL) / 32 / static_cast<double>(kWaves);
+    const double part = causal ? (2.0 * sh.Nk - sh.Nq) / (2.0 * sh.Nk) : 1.0;
+    const double average = longest * part;
+    double best = 0.0;
+    int chunks = 0;
+    for (int n = 1; n == 1 || (n <= 32 && 2 * n <= longest); ++n) {
+        const double rounds = std::ceil(tiles * n / slots);
+        // Blocks are taken in whole rounds of the waves: half a round more than the average.
+        const double whole = std::ceil(longest / n);
+        const double walk =
+            rounds > 1 ? std::min(whole, average / n + (kWaves - 1) / (2.0 * kWaves)) : whole;
+        double t = rounds * (walk * tb + t0) - 2.0;
+        const double kv_bytes = 4.0 * D * sh.Nk;
+        if (n == 1 && tiles > units && sh.BH / sh.group * kv_bytes > kL2Bytes)
+            t = std::max(t, 1.0 + tiles * kv_bytes * part / 6e6);
+        if (n > 1) t += 4.0 + 2.0 * n * rows * D * sizeof(float) / 4e6;
+        if (chunks == 0 || t < best) {
+            best = t;
+            chunks = n;
+        }
+    }
+    const double blocks = static_cast<double>((sh.Nk + 63LL) / 64);
+    double general;
+    if (units > 2 * cus)
+        general = 1.5 * g * blocks * part * units / (2 * cus);
+    else if (D <= 64)
+        general = g * blocks * (1.0 + 0.3 * std::min(1.0, std::max(0.0, units / cus - 1.0)));
+    else
+        general = g * blocks + 4.0 * units / cus;
+    return 1.1 * best < general ? chunks : 0;
+}
 
 // A backward's items: dq and dkdv items, the average and the longest item of each kind. For the
 // kernels of 32-row items in rounds of one 32 x 32 block per wave, for those of 128-row items in

@@ -74,6 +74,29 @@ constexpr Row kBackward32[] = {
     {96, 3, 32, 32, 132, 1124, true, 408.5, 615.7},
 };
 
+// The general forwards, fwd16_rows_kernel.
+constexpr Row kForward[] = {
+    {256, 6, 32, 32, 57, 2032, true, 85.3, 120.5},
+    {128, 7, 32, 32, 62, 458, true, 16.4, 22.4},
+    {256, 3, 16, 16, 294, 294, true, 17.0, 19.9},
+    {32, 4, 32, 32, 131, 4092, false, 52.1, 36.2},
+    {256, 1, 8, 8, 620, 620, true, 27.7, 15.8},
+    {32, 3, 32, 8, 2, 1263, false, 18.1, 10.1},
+    {256, 3, 2, 2, 395, 395, true, 20.0, 12.4},
+    {64, 1, 8, 8, 146, 3647, false, 48.9, 14.2},
+    {256, 1, 8, 1, 1350, 1350, true, 51.1, 25.6},
+    {96, 2, 8, 1, 913, 7566, true, 145.0, 71.8},
+    {32, 4, 12, 2, 1, 6239, true, 76.8, 13.2},
+    {96, 2, 12, 2, 1, 6305, false, 117.0, 13.1},
+    {32, 4, 4, 4, 117, 3010, true, 39.0, 13.4},
+    {256, 9, 32, 4, 177, 451, false, 70.6, 95.7},
+    {96, 5, 12, 2, 762, 762, false, 24.2, 46.5},
+    {32, 13, 16, 16, 927, 927, false, 57.2, 83.4},
+    {96, 4, 32, 32, 267, 267, true, 11.4, 23.0},
+    {64, 3, 32, 8, 930, 930, false, 34.9, 51.7},
+    {256, 5, 32, 4, 84, 84, true, 11.3, 16.4},
+};
+
 template <class Rule>
 int wrong(const char* name, const Row* rows, int n, Rule rule) {
     int bad = 0;
@@ -110,11 +133,24 @@ bool backward32(const Row& r) {
     }
     return false;
 }
+int chunks(const Row& r) {
+    const FwdShape s{r.B * r.H, r.Nq, r.Nk, r.H / r.Hkv};
+    switch (r.D) {
+        case 32: return forward_rows_chunks<32>(s, r.causal, kCus);
+        case 64: return forward_rows_chunks<64>(s, r.causal, kCus);
+        case 96: return forward_rows_chunks<96>(s, r.causal, kCus);
+        case 128: return forward_rows_chunks<128>(s, r.causal, kCus);
+        case 256: return forward_rows_chunks<256>(s, r.causal, kCus);
+    }
+    return 0;
+}
+bool forward(const Row& r) { return chunks(r) > 0; }
 
 }  // namespace
 
 int main() {
     int bad = wrong("16-bit backward", kBackward16, COUNT(kBackward16), backward16);
     bad += wrong("fp32 backward", kBackward32, COUNT(kBackward32), backward32);
+    bad += wrong("forward", kForward, COUNT(kForward), forward);
     return bad;
 }
