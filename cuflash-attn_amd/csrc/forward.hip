@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW)
     constexpr int BM = 32 * NW;  // query rows per workgroup (NW waves of 32 rows)
     constexpr int BN = 64;
     constexpr int kParts = 16 / NW;  // load instructions per wave per 64-row tile
-    using Lay = TileGroups<D>;
+    using Lay = FwdTileGroups<D, NW>;
     constexpr int GRP = Lay::kBytes;       // bytes per 4-row group
     constexpr int TILE = (BN / 4) * GRP;   // bytes per 64-row tile
     using frag = typename Elem<T>::frag;
