@@ -905,6 +905,13 @@ template <int D>
 constexpr bool bwd_early_loads() {
     return D == 256;
 }
+// The dq items of head_dim 96 issue them early as well. Late -> early, no mask, B=4: 12 heads over 2,
+// N=648 79 -> 74 us; 16 heads, N=1100 151 -> 143 (but N=1300 183 -> 198: late was faster than before
+// at some lengths and slower at others, early at none slower).
+template <int D>
+constexpr bool dq_early_loads() {
+    return bwd_early_loads<D>() || D == 96;
+}
 // Whether the items store their output rows through LDS (store_rows_staged: whole contiguous
 // rows per store instruction). Not at head_dim 128, where the staging code makes the kernel
 // spill at its 256-register budget and measured no faster.
@@ -1312,7 +1319,7 @@ __device__ __forceinline__ void dq_lds_tiles(const uint16_t* __restrict__ Q,
         const int key0 = kb * BN;
         __builtin_amdgcn_s_waitcnt(0);  // block kb is in LDS
         __syncthreads();                // ... for every wave; block kb - 1 is no longer read
-        if (bwd_early_loads<D>() && kb + 1 < nkb) load_block(kb + 1, b ^ 1);
+        if (dq_early_loads<D>() && kb + 1 < nkb) load_block(kb + 1, b ^ 1);
         const unsigned char* kt = smem + b * SET;
         const unsigned char* vt = kt + KT;
 
@@ -1347,7 +1354,7 @@ __device__ __forceinline__ void dq_lds_tiles(const uint16_t* __restrict__ Q,
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (!bwd_early_loads<D>() && kb + 1 < nkb) load_block(kb + 1, b ^ 1);
+        if (!dq_early_loads<D>() && kb + 1 < nkb) load_block(kb + 1, b ^ 1);
         if (key0 + BN > Nk || (causal && key0 + BN - 1 > q0 + coff)) {
             const int lim = min(Nk, causal ? q + 1 + coff : Nk) - key0 - 4 * g2;
 #pragma unroll
