@@ -1960,16 +1960,15 @@ FlashAttentionError run_forward16_rows(const T* Q, const T* K, const T* V, T* O,
     dev::FwdSplit sp{nullptr, nullptr, sh.Nk, 1, zero_rows};
     StreamWorkspace ws(stream, true);
     if (chunks > 1) {
-        const int chunk = ((sh.Nk + chunks - 1) / chunks + 31) / 32 * 32;
-        const int nsplit = (sh.Nk + chunk - 1) / chunk;
-        const size_t slots = static_cast<size_t>(rows) * nsplit;
+        const KeyChunks kc = key_chunks(sh.Nk, chunks);
+        const size_t slots = static_cast<size_t>(rows) * kc.nsplit;
         const size_t bytes = slots * (D * sizeof(float) + sizeof(float2));
-        if (nsplit > 1 && bytes <= kStreamCacheBytes && !stream_capturing(stream) &&
+        if (kc.nsplit > 1 && bytes <= kStreamCacheBytes && !stream_capturing(stream) &&
             ws.alloc(bytes) == FlashAttentionError::SUCCESS) {
             sp.acc = static_cast<float*>(ws.get());
             sp.ml = reinterpret_cast<float2*>(sp.acc + slots * D);
-            sp.chunk = chunk;
-            sp.nsplit = nsplit;
+            sp.chunk = kc.chunk;
+            sp.nsplit = kc.nsplit;
         }
     }
     const long long blocks = nqb * (sh.BH / sh.group) * sp.nsplit;

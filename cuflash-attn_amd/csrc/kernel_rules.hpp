@@ -102,6 +102,15 @@ int forward_rows_chunks(const FwdShape& sh, bool causal, int compute_units) {
     return 1.1 * best < general ? chunks : 0;
 }
 
+// The keys of each chunk (whole 32-key blocks) and the number of chunks that have any.
+struct KeyChunks {
+    int chunk, nsplit;
+};
+inline KeyChunks key_chunks(int Nk, int chunks) {
+    const int chunk = ((Nk + chunks - 1) / chunks + 31) / 32 * 32;
+    return {chunk, (Nk + chunk - 1) / chunk};
+}
+
 // A backward's items: dq and dkdv items, the average and the longest item of each kind. For the
 // kernels of 32-row items in rounds of one 32 x 32 block per wave, for those of 128-row items in
 // 32-row blocks of the other side.

@@ -2,8 +2,12 @@
 // times: where one kernel was more than 15% faster, the rule takes that one. No GPU call is made.
 //
 // Times of one box in microseconds of a whole call, fp16 / bf16 or fp32, on 256 CUs.
+//
+// With arguments (B, heads, key/value heads, queries, keys, head_dim, causal of each launch): prints
+// the chunks of a 16-bit forward, 0 for the general kernels, and the keys of a chunk.
 
 #include <cstdio>
+#include <cstdlib>
 
 #include "kernel_rules.hpp"
 
@@ -148,7 +152,17 @@ bool forward(const Row& r) { return chunks(r) > 0; }
 
 }  // namespace
 
-int main() {
+int main(int argc, char** argv) {
+    if (argc > 1) {
+        for (int i = 1; i + 6 < argc; i += 7) {
+            int v[7];
+            for (int j = 0; j < 7; ++j) v[j] = std::atoi(argv[i + j]);
+            const int n = chunks(Row{v[5], v[0], v[1], v[2], v[3], v[4], v[6] != 0, 0.0, 0.0});
+            const KeyChunks kc = n > 1 ? key_chunks(v[4], n) : KeyChunks{v[4], n};
+            std::printf("%d %d\n", kc.nsplit, kc.chunk);
+        }
+        return 0;
+    }
     int bad = wrong("16-bit backward", kBackward16, COUNT(kBackward16), backward16);
     bad += wrong("fp32 backward", kBackward32, COUNT(kBackward32), backward32);
     bad += wrong("forward", kForward, COUNT(kForward), forward);

@@ -5,14 +5,17 @@ every eighth (head_dim 256: fourth) 32-key block, and with very few rows also cu
 chunks that a second kernel merges. Checked against the fp64 oracle on every row where that can go
 wrong: one row, rows that end inside a tile, heads packed into one tile, fewer blocks than waves,
 a last block and a last chunk of one key, causal rows that end before, inside and after a chunk,
-every head_dim.
+merges with several rows' parts in one workgroup, every head_dim. Each shape names the chunks that
+it must run in; the host rule is held to that on the CPU, the launches on the GPU.
 
 Bounds: V lies in [-1, 1), so rounding P to the input type moves a row of O by at most the unit
 roundoff u, and rounding O by as much again; fp32 sums add less than u / 4. L is a sum of at most
-8193 fp32 terms of exact products: its error is well under 2e-5.
+12289 fp32 terms of exact products: its error is well under 2e-5.
 """
 
 from __future__ import annotations
+
+import contextlib
 
 import numpy as np
 import pytest
@@ -21,25 +24,64 @@ import cuflash_attn
 import oracle
 from conftest import max_abs
 from cuflash_attn import synth
+from test_host_rules import run_program
 
 UNIT = {"bfloat16": 2.0 ** -9, "float16": 2.0 ** -11}
 
-# B, H, Hkv, Nq, Nk, D, causal
+# B, H, Hkv, Nq, Nk, D, causal, chunks
 SHAPES = [
-    (1, 8, 2, 61, 1025, 128, True),
-    (1, 4, 1, 1, 4097, 128, True),
-    (2, 2, 2, 1, 8193, 64, False),
-    (1, 2, 2, 129, 577, 64, False),
-    (1, 8, 8, 700, 700, 64, True),
-    (1, 3, 3, 1057, 1057, 128, True),
-    (1, 4, 2, 300, 515, 32, True),
-    (2, 6, 2, 33, 3000, 96, True),
-    (1, 3, 1, 40, 1300, 256, True),
-    (1, 2, 2, 300, 300, 256, False),
-    (1, 8, 1, 17, 2048, 128, False),
-    (20, 32, 8, 1, 70, 64, False),
-    (20, 32, 8, 2, 130, 128, True),
+    (1, 8, 2, 61, 1025, 128, True, 1),
+    (1, 4, 1, 1, 4097, 128, True, 6),
+    (2, 2, 2, 1, 8193, 64, False, 11),
+    (1, 2, 2, 129, 577, 64, False, 1),
+    (1, 8, 8, 700, 700, 64, True, 1),
+    (1, 3, 3, 1057, 1057, 128, True, 1),
+    (1, 4, 2, 300, 515, 32, True, 1),
+    (2, 6, 2, 33, 3000, 96, True, 4),
+    (1, 3, 1, 40, 1300, 256, True, 4),
+    (1, 2, 2, 300, 300, 256, False, 1),
+    (1, 8, 1, 17, 2048, 128, False, 4),
+    (20, 32, 8, 1, 70, 64, False, 1),
+    (20, 32, 8, 2, 130, 128, True, 1),
+    # Causal rows that end before a chunk: whole tiles that skip it, and rows inside a tile.
+    (1, 1, 1, 1000, 2100, 128, True, 3),
+    (1, 1, 1, 600, 4097, 64, True, 6),
+    (1, 2, 2, 700, 1100, 256, True, 3),
+    (1, 1, 1, 2001, 2001, 64, True, 3),
+    (1, 4, 1, 400, 1500, 256, True, 4),
+    # A last chunk of one key that one row sees; merges that share a row over two and four groups.
+    (1, 1, 1, 64, 12289, 256, True, 25),
+    (1, 2, 1, 40, 12289, 96, True, 17),
+    (1, 4, 4, 3, 8193, 128, True, 11),
 ]
+
+
+@contextlib.contextmanager
+def kernels_of(torch, lib):
+    """The labels of the kernels that the library launches inside the block (filled at its end)."""
+    launched = set()
+    torch.cuda.synchronize()
+    lib.profile_report()
+    lib.profile_enable(True)
+    try:
+        yield launched
+        torch.cuda.synchronize()
+    finally:
+        lib.profile_enable(False)
+        launched.update(lib.profile_report())
+
+
+def test_shapes_run_in_the_chunks_that_they_name(tmp_path):
+    args = [int(x) for shape in SHAPES for x in shape[:7]]
+    got = [tuple(map(int, line.split()))
+           for line in run_program("test_kernel_rules", tmp_path, *args).splitlines()]
+    assert [n for n, _ in got] == [shape[7] for shape in SHAPES]
+    # What the comments of SHAPES say of the last chunks.
+    last = [shape[4] - (n - 1) * chunk for shape, (n, chunk) in zip(SHAPES, got)]
+    assert 1 in last
+    assert sum(shape[6] and n > 1 and shape[4] - shape[3] < (n - 1) * chunk
+               for shape, (n, chunk) in zip(SHAPES, got)) >= 6
+
 
 # B, H, Hkv, keys, D: grouped-query decodes of short caches, which run the same kernel.
 DECODES = [(1, 32, 8, 1000, 128), (3, 12, 2, 1, 128), (2, 32, 1, 33, 64), (5, 8, 4, 1024, 32)]
@@ -48,15 +90,16 @@ DECODES = [(1, 32, 8, 1000, 128), (3, 12, 2, 1, 128), (2, 32, 1, 33, 64), (5, 8,
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(map(str, s)))
-def test_forward_of_few_rows_matches_the_oracle(torch_gpu, dtype, shape):
-    B, H, Hkv, Nq, Nk, D, causal = shape
+def test_forward_of_few_rows_matches_the_oracle(torch_gpu, lib, dtype, shape):
+    B, H, Hkv, Nq, Nk, D, causal, chunks = shape
     q = synth.round_to(synth.uniform(1, (B, H, Nq, D)), dtype)
     k, v = (synth.round_to(synth.uniform(s, (B, Hkv, Nk, D)), dtype) for s in (2, 3))
     scale = 2.0 * D ** -0.5
     print(f"[forward rows] {dtype} {shape}", flush=True)
-    o, lse = cuflash_attn.flash_attention_forward_ext(
-        *(synth.to_torch(x, dtype) for x in (q, k, v)), scale=scale, causal=causal)
-    torch_gpu.cuda.synchronize()
+    tensors = [synth.to_torch(x, dtype) for x in (q, k, v)]
+    with kernels_of(torch_gpu, lib) as launched:
+        o, lse = cuflash_attn.flash_attention_forward_ext(*tensors, scale=scale, causal=causal)
+    assert any(label.startswith("forward_combine") for label in launched) == (chunks > 1), launched
     o_ref, l_ref = oracle.forward(q, *(np.repeat(x, H // Hkv, axis=1) for x in (k, v)), scale,
                                   causal)
     assert max_abs(synth.to_numpy(o), o_ref) <= 2.25 * UNIT[dtype]

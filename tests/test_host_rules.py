@@ -9,7 +9,7 @@ import subprocess
 import build as cuflash_build  # cuflash-attn_amd/build.py
 
 
-def _run(name, tmp_path, *args):
+def run_program(name, tmp_path, *args):
     exe = tmp_path / name
     env = {k: v for k, v in os.environ.items() if k != "LD_PRELOAD"}
     subprocess.run(
@@ -24,13 +24,13 @@ def _run(name, tmp_path, *args):
 
 
 def test_unknown_capture_status_counts_as_captured(tmp_path):
-    _run("test_capture_status", tmp_path)
+    run_program("test_capture_status", tmp_path)
 
 
 def test_balanced_paged_split_stays_in_bounds(tmp_path):
     """Over launches that keep the equal splits, that balance, and that are nearly full."""
-    _run("test_paged_split", tmp_path, 3000, 1)
+    run_program("test_paged_split", tmp_path, 3000, 1)
 
 
 def test_kernel_rules_take_the_measured_faster_kernel(tmp_path):
-    _run("test_kernel_rules", tmp_path)
+    run_program("test_kernel_rules", tmp_path)
