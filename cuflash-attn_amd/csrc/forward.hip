@@ -1954,7 +1954,8 @@ namespace {
 template <typename T, int D>
 FlashAttentionError run_forward16_rows(const T* Q, const T* K, const T* V, T* O, float* L,
                                        const FwdShape& sh, int chunks, float scale, bool causal,
-                                       hipStream_t stream, bool zero_rows = false) {
+                                       hipStream_t stream, const char* label = "forward",
+                                       bool zero_rows = false) {
     const long long rows = static_cast<long long>(sh.BH) * sh.Nq;
     const long long nqb = (static_cast<long long>(sh.group) * sh.Nq + 31) / 32;
     dev::FwdSplit sp{nullptr, nullptr, sh.Nk, 1, zero_rows};
@@ -1973,7 +1974,7 @@ FlashAttentionError run_forward16_rows(const T* Q, const T* K, const T* V, T* O,
     }
     const long long blocks = nqb * (sh.BH / sh.group) * sp.nsplit;
     const int coff = sh.Nk - sh.Nq;
-    ProfileEvents tok = profile_kernel<T, D>("forward");
+    ProfileEvents tok = profile_kernel<T, D>(label);
     launch_kernel(tok,
                   sp.nsplit > 1 ? dev::fwd16_rows_kernel<T, D, true>
                                 : dev::fwd16_rows_kernel<T, D, false>,
@@ -2203,11 +2204,14 @@ FlashAttentionError launch_decode_rows(const T* Q, const T* K, const T* V, T* O,
                                        int kv_len, int head_dim, float scale,
                                        hipStream_t stream) {
     const FwdShape sh{batch_size * num_heads, 1, kv_len, num_heads / num_kv_heads};
+    auto run = [&](auto d) {
+        return run_forward16_rows<T, decltype(d)::value>(Q, K, V, O, L, sh, 1, scale, false, stream,
+                                                         "decode_rows", true);
+    };
     switch (head_dim) {
-        case 32: return run_forward16_rows<T, 32>(Q, K, V, O, L, sh, 1, scale, false, stream, true);
-        case 64: return run_forward16_rows<T, 64>(Q, K, V, O, L, sh, 1, scale, false, stream, true);
-        case 128:
-            return run_forward16_rows<T, 128>(Q, K, V, O, L, sh, 1, scale, false, stream, true);
+        case 32: return run(std::integral_constant<int, 32>());
+        case 64: return run(std::integral_constant<int, 64>());
+        case 128: return run(std::integral_constant<int, 128>());
     }
     return FlashAttentionError::UNSUPPORTED_HEAD_DIM;
 }

@@ -109,15 +109,17 @@ def test_forward_of_few_rows_matches_the_oracle(torch_gpu, lib, dtype, shape):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 @pytest.mark.parametrize("shape", DECODES, ids=lambda s: "-".join(map(str, s)))
-def test_short_grouped_decode_matches_the_oracle(torch_gpu, dtype, shape):
+def test_short_grouped_decode_matches_the_oracle(torch_gpu, lib, dtype, shape):
     B, H, Hkv, Nk, D = shape
     q = synth.round_to(synth.uniform(1, (B, H, 1, D)), dtype)
     k, v = (synth.round_to(synth.uniform(s, (B, Hkv, Nk, D)), dtype) for s in (2, 3))
     print(f"[short decode] {dtype} {shape}", flush=True)
     for scale in (2.0 * D ** -0.5, 0.0):
-        o, lse = cuflash_attn.flash_attention_decode(
-            *(synth.to_torch(x, dtype) for x in (q, k, v)), scale=scale)
-        torch_gpu.cuda.synchronize()
+        tensors = [synth.to_torch(x, dtype) for x in (q, k, v)]
+        with kernels_of(torch_gpu, lib) as launched:
+            o, lse = cuflash_attn.flash_attention_decode(*tensors, scale=scale)
+        suffix = {"bfloat16": "bf16", "float16": "f16"}[dtype]
+        assert launched == {f"decode_rows_{suffix}_d{D}"}
         o_ref, l_ref = oracle.forward(q, *(np.repeat(x, H // Hkv, axis=1) for x in (k, v)), scale,
                                       False)
         assert max_abs(synth.to_numpy(o), o_ref) <= 2.25 * UNIT[dtype]
