@@ -75,3 +75,28 @@ def test_small_backward_matches_float64(torch_gpu, dtype, shape):
             close(got[0][-1, h], ds @ kd, "dQ")
         close(got[1][-1, hk], dk, "dK")
         close(got[2][-1, hk], dv, "dV")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("head_dim", [32, 64, 96, 128])
+def test_nan_reaches_what_sees_it_and_no_other_tile(torch_gpu, dtype, head_dim):
+    """A NaN in one row of dO: that row of dQ and every key it sees are NaN; the other rows of dQ,
+    and the keys of later 32-key tiles, are as without it, bit for bit."""
+    torch = torch_gpu
+    dt = getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(head_dim)
+    q, k, v, do = ((torch.rand((1, 4, 200, head_dim), device="cuda", generator=gen) * 2 - 1).to(dt)
+                   for _ in range(4))
+    o, lse = cuflash_attn.flash_attention_forward_ext(q, k, v, causal=True)
+    clean = cuflash_attn.flash_attention_backward_ext(q, k, v, o, lse, do, causal=True)
+    row = 100
+    do[:, :, row, 3] = float("nan")
+    dq, dk, dv = cuflash_attn.flash_attention_backward_ext(q, k, v, o, lse, do, causal=True)
+    torch.cuda.synchronize()
+    others = torch.arange(200, device="cuda") != row
+    assert torch.equal(dq[:, :, others], clean[0][:, :, others])
+    assert bool(dq[:, :, row].isnan().all())
+    assert torch.equal(dk[:, :, 128:], clean[1][:, :, 128:])
+    assert torch.equal(dv[:, :, 128:], clean[2][:, :, 128:])
+    assert bool(dk[:, :, :row + 1].isnan().all()) and bool(dv[:, :, :row + 1, 3].isnan().all())

@@ -124,3 +124,57 @@ def test_short_grouped_decode_matches_the_oracle(torch_gpu, lib, dtype, shape):
                                       False)
         assert max_abs(synth.to_numpy(o), o_ref) <= 2.25 * UNIT[dtype]
         assert max_abs(synth.to_numpy(lse), l_ref) <= 2e-5
+
+
+# B, H, Hkv, Nq, Nk, D: one chunk and several, with a merge over one and over several groups.
+SPECIAL = [(1, 4, 4, 300, 300, 64), (1, 2, 2, 700, 1100, 256), (1, 8, 2, 61, 4097, 128),
+           (1, 2, 1, 40, 12289, 96)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("shape", SPECIAL, ids=lambda s: "-".join(map(str, s)))
+def test_infinities_and_nan_reach_the_rows_that_see_them_and_no_other(torch_gpu, dtype, shape):
+    """A NaN or infinite key makes the rows that see it NaN and leaves the others as they were, bit
+    for bit; an infinite value reaches its own column only; a key whose scores are -inf has no
+    weight (the oracle without that key); rows whose scores are all -inf are NaN with L = -inf."""
+    torch = torch_gpu
+    B, H, Hkv, Nq, Nk, D = shape
+    scale = D ** -0.5
+    q = synth.round_to(np.abs(synth.uniform(1, (B, H, Nq, D))) + 0.25, dtype)
+    k, v = (synth.round_to(synth.uniform(s, (B, Hkv, Nk, D)), dtype) for s in (2, 3))
+    tq, tk, tv = (synth.to_torch(x, dtype) for x in (q, k, v))
+    at = Nk - Nq + Nq // 2  # the key that row Nq // 2 is the first to see
+
+    def run(k, v, causal=True):
+        out = cuflash_attn.flash_attention_forward_ext(tq, k, v, scale=scale, causal=causal)
+        torch.cuda.synchronize()
+        return out
+
+    print(f"[special values] {dtype} {shape}", flush=True)
+    clean_o, clean_l = run(tk, tv)
+    for value in (float("nan"), float("inf")):
+        bad = tk.clone()
+        bad[:, :, at] = value
+        o, lse = run(bad, tv)
+        before, seen = slice(None, Nq // 2), slice(Nq // 2, None)
+        assert torch.equal(o[:, :, before], clean_o[:, :, before])
+        assert torch.equal(lse[:, :, before], clean_l[:, :, before])
+        assert bool(o[:, :, seen].isnan().all())
+    bad = tv.clone()
+    bad[:, :, at, 5] = float("inf")
+    o, lse = run(tk, bad)
+    assert torch.equal(lse, clean_l)
+    rest = torch.arange(D, device="cuda") != 5
+    assert torch.equal(o[..., rest], clean_o[..., rest])
+    assert not bool(o[:, :, Nq // 2:, 5].isfinite().any())
+
+    bad = tk.clone()
+    bad[:, :, at] = float("-inf")
+    o, lse = run(bad, tv, causal=False)
+    o_ref, l_ref = oracle.forward(
+        q, *(np.repeat(np.delete(x, at, axis=2), H // Hkv, axis=1) for x in (k, v)), scale, False)
+    assert max_abs(synth.to_numpy(o), o_ref) <= 2.25 * UNIT[dtype]
+    assert max_abs(synth.to_numpy(lse), l_ref) <= 2e-5
+    o, lse = run(torch.full_like(tk, float("-inf")), tv)
+    assert bool(o.isnan().all()) and bool(torch.isneginf(lse).all())
