@@ -3,7 +3,10 @@ grouped-query and paged decodes.
 
 Each captured sequence is replayed three times with new inputs written between the replays (the
 program's own eager work and a synchronization between them), and every replay is compared
-bitwise with the same calls run eagerly on the same inputs (the kernels are deterministic).
+bitwise with the same calls run eagerly on the same inputs (the kernels are deterministic), except
+for the calls that take another order of sums in a captured launch: a forward of few query rows
+that runs in chunks eagerly (compared within rounding), and a large paged grouped-query decode
+(not captured here).
 Inside a capture the library takes per-call workspaces, a stream-ordered allocation and free that
 the graph records, instead of the capturing stream's cached buffer, which later calls could
 replace while the graph still refers to it. The kernels record no memset.
@@ -108,4 +111,49 @@ def test_decodes_in_a_captured_graph(torch_gpu):
         torch.cuda.synchronize()
         for i, (a, b) in enumerate(zip(got, ref)):
             assert torch.equal(a, b), f"replay {rep}: output {i}"
+    del graph
+
+
+@pytest.mark.gpu
+def test_chunked_forward_in_a_captured_graph(torch_gpu, lib):
+    """A forward of few query rows that runs in chunks eagerly runs in one chunk when captured (its
+    graph holds no allocation): its sums stand in another order, so the replays equal the eager
+    call within rounding. Values lie in [-1, 1), so each O is within 2.25 unit roundoffs of the
+    exact one (P, O and the fp32 sums) and each L within 2e-5."""
+    import cuflash_attn
+    from test_forward_rows_gpu import kernels_of
+
+    torch = torch_gpu
+    B, H, HKV, NQ, NK, D = 1, 8, 2, 7, 4097, 128
+    q = torch.empty((B, H, NQ, D), device="cuda", dtype=torch.bfloat16)
+    k, v = (torch.empty((B, HKV, NK, D), device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    static = {}
+
+    def fill(seed):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        for t in (q, k, v):
+            t.copy_(torch.rand(t.shape, generator=g, device="cuda") * 2 - 1)
+
+    def step():
+        static["out"] = cuflash_attn.flash_attention_forward_ext(q, k, v, causal=True)
+
+    fill(1)
+    with kernels_of(torch, lib) as launched:
+        step()
+    assert launched == {"forward_bf16_d128", "forward_combine_bf16_d128"}
+    graph = _capture(torch, step)
+    for rep in range(3):
+        print(f"[graph chunked forward] replay {rep}", flush=True)
+        fill(30 + rep)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        o, lse = (t.clone() for t in static["out"])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, static["out"][0]) and torch.equal(lse, static["out"][1])
+        o_ref, l_ref = cuflash_attn.flash_attention_forward_ext(q, k, v, causal=True)
+        torch.cuda.synchronize()
+        assert float((o.float() - o_ref.float()).abs().max()) <= 4.5 * 2.0 ** -9
+        assert float((lse - l_ref).abs().max()) <= 4e-5
     del graph
