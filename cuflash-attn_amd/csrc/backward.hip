@@ -1533,6 +1533,9 @@ __global__ void __launch_bounds__(256)
 // bwd32_kernel) the waves of a workgroup share one 32-row tile and take every NW-th block through
 // LDS-DMA double buffers of their own (no barrier in the loop), and their sums are added through
 // LDS in wave order at the end: chains a fourth or an eighth as long over four times the workgroups.
+// The second buffer hides little as built: the compiler does not see the tile loads, and its own
+// waits for the row fragments stand in the block loops, where they wait for the next block's loads
+// too (all loops but that of the dq items at head_dim 64).
 // A key tile runs over all query heads of its group, so grouped heads need no shares. Products,
 // roundings and the order inside a block are those of dq_lds_tiles and dkdv_lds_tiles.
 // Backward kernel, causal, us (bwd_fused_kernel -> this): head_dim 64, 8 heads, N=300 13.1 -> 6.8,

@@ -1373,8 +1373,8 @@ __global__ void __launch_bounds__(256)
 // also cut into chunks over workgroups.
 // What bounds it: every wave loads its own tiles, 128 KB for a round of eight blocks at head_dim
 // 128, 1.0 us at the CU's 64 bytes per clock, beside 0.5 us of MFMAs; measured 1.36 us a round.
-// Eight waves with one buffer each for K and V (two waves per SIMD, one computing while the
-// other loads) take 11.7 us where four waves with double buffers in the same LDS take 14.6 (head_dim
+// Eight waves with one buffer each for K and V (two waves per SIMD, one computing while the other
+// loads: that is what overlaps, a wave's own loads hardly do) take 11.7 us where four waves with double buffers in the same LDS take 14.6 (head_dim
 // 128, 4 heads, N = 1024), 20.6 against 35 at head_dim 256 with four waves against two.
 template <typename T, int D, bool kSplit>
 __global__ void __launch_bounds__(64 * detail::fwd_rows_waves<D>(), D <= 64 ? 2 : 1)
@@ -1467,7 +1467,7 @@ __global__ void __launch_bounds__(64 * detail::fwd_rows_waves<D>(), D <= 64 ? 2 
             qf[ks] = as_frag<T>(v);
         }
     }
-    // After the Q loads, so that waiting for those leaves the tile loads in flight.
+    // After the Q loads (see the waits of the loop below).
     asm volatile("" ::: "memory");
     if (wave < nblk) {
         load_tile(Kh, wave * BN, kt);
@@ -1485,9 +1485,11 @@ __global__ void __launch_bounds__(64 * detail::fwd_rows_waves<D>(), D <= 64 ? 2 
     // This lane's key limit, and the first key that some row of the tile does not see.
     const int kend = causal ? min(Nk, q + 1 + coff) : Nk;
     const int mask_from = causal ? min(Nk, r0 / group + 1 + coff) : Nk;
-    // K and V are waited for separately (vmcnt counts a wave's loads in order, kLoads per tile):
-    // the scores start when K has landed, with V still in flight; the next K is issued once the
-    // scores have read this one, the next V once P V has.
+    // K and V are waited for separately (vmcnt counts a wave's loads in order, kLoads per tile): K
+    // before the scores, V before P V; the next K is issued once the scores have read this one, the
+    // next V once P V has. The compiler does not see the tile loads, and its own wait for the Q
+    // fragments, vmcnt(0), stands before the first product of every block: as built, the scores wait
+    // for V as well, and only the next K overlaps products (those of P V).
     constexpr int kLoads = NG * Lay::kHalves;
     for (int b = wave; b < nblk; b += NW) {
         const bool next = b + NW < nblk;
