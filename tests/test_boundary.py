@@ -259,6 +259,18 @@ def test_candidate_paths_follow_reference_order(monkeypatch):
     assert paths[2].endswith(os.path.join("build", "default", "libcuflash_attn.so"))
 
 
+def test_current_stream_handle_with_and_without_torchs_internal_function(monkeypatch):
+    from types import SimpleNamespace as NS
+
+    cuda = NS(current_device=lambda: 3, current_stream=lambda: NS(cuda_stream=0x70))
+    internal = NS(_cuda_getCurrentRawStream=lambda device: 0x60 + device)
+    monkeypatch.setattr(cuflash_attn, "_TORCH", NS(cuda=cuda, _C=internal))
+    assert cuflash_attn._stream_ptr() == 0x63
+    monkeypatch.setattr(cuflash_attn, "_TORCH", NS(cuda=cuda, _C=NS()))
+    assert cuflash_attn._stream_ptr() == 0x70
+    assert cuflash_attn._stream_ptr(NS(cuda_stream=0x50)) == 0x50
+
+
 def test_missing_library_fails_loudly():
     with pytest.raises(OSError):
         cuflash_attn.load_library("/nonexistent/libcuflash_attn.so")
