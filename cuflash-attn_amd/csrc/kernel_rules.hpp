@@ -216,12 +216,14 @@ bool bwd32_faster(const BwdShape& sh, bool causal, int compute_units) {
 // Whether bwd16_rows_kernel beats bwd_fused_kernel. The first spreads better, the second moves a
 // fourth of the tile bytes per product; grouped heads leave it shares that another launch sums. The
 // costs are fitted to 2200 random launches (32 to 8192 keys), in which the choice is on average
-// 1.6% slower than the better kernel (bwd_fused_kernel alone: 37%) and 20 take a kernel that is
+// 3% slower than the better kernel (bwd_fused_kernel alone: 37%) and 20 take a kernel that is
 // more than 2% slower. Measured (bwd_fused_kernel, bwd16_rows_kernel, us; more at the kernel): taken:
 // 8 heads, N=1024, head_dim 64 28.5, 14.4. Not taken: causal 16 heads, N=2048, head_dim 64 61, 69
 // and 128 92, 140; 32 heads, N=1024, head_dim 64 38, 52; 8 heads over 1, N=2000, head_dim 128 98,
 // 203; no mask, 22 heads, 278 of 943 keys, head_dim 96 29, 53 (and causal 36 heads, 43 of 349
 // keys, head_dim 128 19, 26): the short side has too few blocks for the waves.
+// Beyond eight items per CU the fused kernel is kept, although with grouped heads and few query rows
+// this one measures faster there as well (B=10, 32 heads over 4, 65 of 2197 keys, head_dim 32 524, 144).
 template <int D>
 bool bwd16_rows_faster(const BwdShape& sh, bool causal, int compute_units) {
     constexpr BwdCost kRows = D == 32   ? BwdCost{3.25, 3.74, 0.80, 1.03, 0.14, 0.47}
@@ -240,7 +242,8 @@ bool bwd16_rows_faster(const BwdShape& sh, bool causal, int compute_units) {
     const bool shares = sh.group > 1 && share_bytes <= kMaxShareBytes;
     double fused = item_time(block_items(sh, causal, shares ? 1 : sh.group), kFused, cus, 2.0);
     if (shares) fused += kSum + share_bytes / kRate;
-    return 1.2 * item_time(row_items(sh, causal, bwd16_rows_waves<D>()), kRows, cus, 1.0) < fused;
+    const BwdItems rows = row_items(sh, causal, bwd16_rows_waves<D>());
+    return rows.nq + rows.nk <= 8.0 * cus && 1.2 * item_time(rows, kRows, cus, 1.0) < fused;
 }
 
 }  // namespace detail

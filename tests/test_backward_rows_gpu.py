@@ -29,8 +29,8 @@ SHAPES = [
     (1, 4, 4, 700, 700, 128, True),
     (1, 2, 2, 300, 77, 64, False),
     # Several items per CU: grouped heads with few query rows.
-    (8, 32, 8, 46, 1092, 32, True),
-    (8, 24, 8, 40, 900, 128, False),
+    (8, 32, 8, 46, 700, 32, True),
+    (7, 24, 8, 40, 900, 128, False),
 ]
 
 
