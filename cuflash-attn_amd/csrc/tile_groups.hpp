@@ -15,7 +15,10 @@ namespace dev {
 // GB/s per CU, as for wholly linear lanes, against 37 with the rows of a group interleaved by 16
 // bytes (consecutive lanes in four rows). The kernels, whose loads hide in part behind their
 // MFMAs, gained 0.5 to 4% (bf16 training step, 16 heads over 4, N = 2001: 231.8 -> 222.3 us;
-// head_dim 256, N = 2049: 246.1 -> 238.6 us; head_dim 128, N = 16384: 8454 -> 8381 us).
+// head_dim 256, N = 2049: 246.1 -> 238.6 us; head_dim 128, N = 16384: 8454 -> 8381 us). The one-head
+// decode kernel (decode_mma_kernel) gained 1 to 9% up to some 5000 keys and 1 to 14% on paged caches
+// (32 heads over 8, B = 4, 3000 keys, head_dim 128: 15.2 -> 14.1 us); where it runs at the HBM rate it
+// is level, or 1% slower (head_dim 128, B = 16, 12000 keys: 119.7 -> 120.9 us).
 //   D = 128: 4-row groups, chunk c of row r at 16 (16 (c / 4) + 4 r + c % 4): the rows of a group
 //            interleaved by 64 bytes. The padding of kBytes shifts successive groups by an odd
 //            number of 16-byte slots modulo 64 bytes, so that 16 rows read at one chunk cover all
