@@ -569,7 +569,7 @@ def host_cpus():
 
 
 def host_threads():
-    """Threads of the CPU-side work: the host CPUs, at most 16 (the GPU box's CPU share)."""
+    """Threads of the CPU-side work: the host CPUs, at most 16."""
     return max(1, min(16, host_cpus()))
 
 

@@ -40,7 +40,7 @@ constexpr long long kMaxShareBytes = 2LL << 30;
 
 // Chunks over which fwd16_rows_kernel cuts the keys of this launch, or 0 where the general kernels
 // are faster. The times are modelled from measurements (causal and not, 4 to 32 heads, 64 to 16384
-// keys; event times of one box):
+// keys; event times of one MI355X):
 //  * fwd16_rows_kernel: a workgroup walks its longest tile in rounds of one block per wave, tb
 //    each, and t0 for its start, merge and store; as many workgroups as the slots run at once.
 //    Several chunks add the merge kernel and the partials, written and read at about 4 TB/s. In one

@@ -136,7 +136,7 @@ struct FwdTileGroups<96, 4> {
 // The tiles of fwd16_d64_seq_kernel. Its loads hide behind the vector work of four waves per SIMD,
 // so at head_dim 64 the rows of a group stay interleaved by 16 bytes, chunk c of row r at
 // 16 (8 c + (r ^ 4 ((c / 2) % 2))), on the same 16 and 32 bank slots (fwd16_d64_kernel has the same
-// order). Measured, no mask, this order -> TileGroups<64> on one box: B=4, 16 heads, N=3000
+// order). Measured, no mask, this order -> TileGroups<64> on one MI355X: B=4, 16 heads, N=3000
 // 162.5 -> 164.7 us; B=12, 16 heads over 4, 183 queries of 2264 keys 45.0 -> 45.7. At head_dim 32
 // TileGroups is the faster one (causal, B=2, 32 heads, N=2500 49.5 -> 49.0).
 // The row and transpose offsets take the kernel's l32 = lane % 32 and g2 = lane / 32 too: formed

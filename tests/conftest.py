@@ -1,6 +1,6 @@
 """Shared pytest setup.
 
-Markers: `gpu` = needs an MI355X (run with -m gpu on the GPU box); everything else runs on the
+Markers: `gpu` = needs an MI355X (run with -m gpu); everything else runs on the
 CPU. The CPU suite checks the oracle, the host logic and the C-ABI boundary without any GPU
 call; the GPU suite compares the HIP kernels (through the C ABI) with the oracle.
 """

@@ -1,7 +1,7 @@
 // The rules that choose between two kernels (cuflash-attn_amd/csrc/kernel_rules.hpp), held to measured
 // times: where one kernel was more than 15% faster, the rule takes that one. No GPU call is made.
 //
-// Times of one box in microseconds of a whole call, fp16 / bf16 or fp32, on 256 CUs.
+// Times of one MI355X in microseconds of a whole call, fp16 / bf16 or fp32, on 256 CUs.
 //
 // With arguments (B, heads, key/value heads, queries, keys, head_dim, causal of each launch): prints
 // the chunks of a 16-bit forward, 0 for the general kernels, and the keys of a chunk.
